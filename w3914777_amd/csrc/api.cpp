@@ -1005,13 +1005,11 @@ extern "C" int amps_adjoint(amps_ctx* c, const double* dJ_du, const int32_t* par
     const int k_every = c->tape_every;
     AdjMem mem;
     double* lam[2];
-    double* w[6];
     double* gacc;
     long long* dstep;
     std::vector<double*> seg(k_every + 1);
     RCCHK(mem.get((void**)&lam[0], state * 8));
     RCCHK(mem.get((void**)&lam[1], state * 8));
-    for (int i = 0; i < 6; ++i) RCCHK(mem.get((void**)&w[i], TC * 8));
     RCCHK(mem.get((void**)&gacc, (size_t)NG * c->total_tiles * 8));
     RCCHK(mem.get((void**)&dstep, 8));
     for (int j = 1; j <= k_every; ++j) RCCHK(mem.get((void**)&seg[j], state * 8));
@@ -1052,10 +1050,10 @@ extern "C" int amps_adjoint(amps_ctx* c, const double* dJ_du, const int32_t* par
             a.un = seg[j + 1];
             a.lam_n = lam[cur];
             a.lam = lam[cur ^ 1];
-            a.w0 = w[0]; a.w1 = w[1]; a.w2 = w[2]; a.w3 = w[3]; a.w4 = w[4]; a.w5 = w[5];
             a.gacc = gacc;
             a.step_ctr = dstep;
             a.step_add = j;
+            a.t_halo = step_args(c, 0).t_halo;
             RCCHK(launch_adjoint_step(a, c->model, c->tile, c->stream));
             cur ^= 1;
         }

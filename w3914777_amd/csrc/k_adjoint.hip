@@ -10,10 +10,12 @@
 // the adjoint, a gather over the pre-images {j : bmap(j + d) = i}, so zero-flux
 // mirrors and periodic wrap transpose without special cases.
 //
-// Each kernel is one workgroup per tile, one thread per cell of the tile
-// (TS*TS/256 cells per thread), and writes full-grid work arrays read by the
-// next kernel.  Parameter partial sums are reduced per workgroup and added to
-// a per-tile accumulator slot, so the sums are deterministic.
+// A step is one kernel with one workgroup per tile: the intermediate
+// cotangents live in LDS, evaluated on the tile and the ring of cells around
+// it that the next stage reads (the rings overlap between tiles; their cells
+// are evaluated again by each).  Parameter partial sums are reduced per
+// workgroup and added to a per-tile accumulator slot, so the sums are
+// deterministic.
 //
 // Snowflake (forward: snowflake/function.h:5-60 restated in k_snowflake.hip):
 //   mu      = dt/tau (lam_phi' + K lam_T')                   cotangent of the bracket
@@ -54,389 +56,573 @@ __device__ inline void for_preimages(int i, int d, int n, int bc, F&& f) {
     }
 }
 
-// Sum over pre-images along x (row y fixed) of a[row][j].
-__device__ inline double gather_x(const double* a, int x, int y, int d, const InstDesc& D) {
-    double s = 0.0;
-    const double* row = a + (size_t)y * D.nx;
-    for_preimages(x, d, D.nx, D.bc, [&](int j) { s += row[j]; });
-    return s;
+// Box of a TS x TS tile with an H-cell halo in LDS, addressed by tile
+// coordinates (y, x) in [-H, TS + H); frame(r): halo cell r of the NF.
+template <int TS, int H>
+struct AdjBox {
+    static constexpr int LW = TS + 2 * H, SZ = LW * LW, NF = SZ - TS * TS;
+    __device__ static inline int at(int y, int x) { return (y + H) * LW + x + H; }
+    __device__ static inline void frame(int r, int& y, int& x) {
+        if (r < 2 * H * LW) {
+            const int row = r / LW;
+            x = r - row * LW - H;
+            y = (row < H ? row : TS + row) - H;
+        } else {
+            const int q = r - 2 * H * LW, j = q % (2 * H);
+            y = q / (2 * H);
+            x = j < H ? j - H : TS + j - H;
+        }
+    }
+};
+
+// Cell (gy, gx) of instance D, boundary-mapped (bmap by selects: a branch
+// around a load's address would split the loads of a tile into rounds).
+__device__ inline int adj_map(int i, int n, bool per) {
+    const int lo = per ? i + n : -i, hi = per ? i - n : 2 * (n - 1) - i;
+    return i < 0 ? lo : (i >= n ? hi : i);
 }
-__device__ inline double gather_y(const double* a, int x, int y, int d, const InstDesc& D) {
-    double s = 0.0;
-    for_preimages(y, d, D.ny, D.bc, [&](int j) { s += a[(size_t)j * D.nx + x]; });
-    return s;
+__device__ inline int adj_cell(const InstDesc& D, int gy, int gx) {
+    const bool per = D.bc == AMPS_BC_PERIODIC;
+    return adj_map(gy, D.ny, per) * D.nx + adj_map(gx, D.nx, per);
 }
 
-// Transposed Laplacian of the field a (instance view) at (x, y), without the
-// 1/(dx dy) factor: sum over the stencil's neighbour offsets of the
-// pre-image values minus centre weight times a(x, y).
-__device__ inline double lapT(const double* a, int x, int y, bool ref, const InstDesc& D) {
-    double s = gather_x(a, x, y, -1, D) + gather_x(a, x, y, 1, D) + gather_y(a, x, y, -1, D) +
-               gather_y(a, x, y, 1, D);
+// Tile origin of the transposed reads.  MIRROR: the tile meets a zero-flux
+// edge and its reads walk the pre-images; elsewhere the pre-image of a read
+// at distance d is the cell at distance -d of the box (the halo of a
+// periodic grid holds the wrapped values).
+struct AdjEdge {
+    int oy, ox, ny, nx;
+};
+__device__ inline bool adj_mirror(const InstDesc& D, int oy, int ox, int ts) {
+    return D.bc != AMPS_BC_PERIODIC && (oy == 0 || ox == 0 || oy + ts == D.ny || ox + ts == D.nx);
+}
+
+// Sum over the pre-images along x (row y fixed) and along y of a read at
+// distance d, and the transposed Laplacian without its 1/(dx dy) factor: the
+// pre-image values of the stencil's offsets minus centre weight times b(y, x).
+// A ring cell outside a zero-flux domain has no meaning and no reader: its
+// gather only has to stay inside the box.
+template <int TS, int H, bool MIRROR>
+__device__ inline double adj_gather_x(const double* b, int y, int x, int d, const AdjEdge& ed) {
+    if constexpr (!MIRROR) return b[AdjBox<TS, H>::at(y, x - d)];
+    double s = 0.0;
+    for_preimages(ed.ox + x, d, ed.nx, AMPS_BC_NEUMANN, [&](int j) {
+        const int r = j - ed.ox;
+        if (r >= -H && r < TS + H) s += b[AdjBox<TS, H>::at(y, r)];
+    });
+    return s;
+}
+template <int TS, int H, bool MIRROR>
+__device__ inline double adj_gather_y(const double* b, int y, int x, int d, const AdjEdge& ed) {
+    if constexpr (!MIRROR) return b[AdjBox<TS, H>::at(y - d, x)];
+    double s = 0.0;
+    for_preimages(ed.oy + y, d, ed.ny, AMPS_BC_NEUMANN, [&](int j) {
+        const int r = j - ed.oy;
+        if (r >= -H && r < TS + H) s += b[AdjBox<TS, H>::at(r, x)];
+    });
+    return s;
+}
+template <int TS, int H, bool MIRROR>
+__device__ inline double adj_lapT(const double* b, int y, int x, bool ref, const AdjEdge& ed) {
+    double s = adj_gather_x<TS, H, MIRROR>(b, y, x, -1, ed) + adj_gather_x<TS, H, MIRROR>(b, y, x, 1, ed) +
+               adj_gather_y<TS, H, MIRROR>(b, y, x, -1, ed) + adj_gather_y<TS, H, MIRROR>(b, y, x, 1, ed);
     double w0 = 4.0;
-    if (ref) {
-        s += gather_x(a, x, y, -2, D) + gather_x(a, x, y, 2, D) + gather_y(a, x, y, -2, D) + gather_y(a, x, y, 2, D);
-        w0 = 8.0;
+    if constexpr (H >= 2) {
+        if (ref) {
+            s += adj_gather_x<TS, H, MIRROR>(b, y, x, -2, ed) + adj_gather_x<TS, H, MIRROR>(b, y, x, 2, ed) +
+                 adj_gather_y<TS, H, MIRROR>(b, y, x, -2, ed) + adj_gather_y<TS, H, MIRROR>(b, y, x, 2, ed);
+            w0 = 8.0;
+        }
     }
-    return s - w0 * a[(size_t)y * D.nx + x];
+    return s - w0 * b[AdjBox<TS, H>::at(y, x)];
 }
 
-// Forward Laplacian (same operand order as the sweeps) of field f at (x, y).
-__device__ inline double lap_fwd(const double* f, int x, int y, bool ref, double inv, const InstDesc& D) {
-    const int nx = D.nx, ny = D.ny, bc = D.bc;
-    const int xs1 = bmap(x - 1, nx, bc), xa1 = bmap(x + 1, nx, bc);
-    const int ys1 = bmap(y - 1, ny, bc), ya1 = bmap(y + 1, ny, bc);
-    const double* r = f + (size_t)y * nx;
-    const double c = r[x];
-    if (ref) {
-        const int xs2 = bmap(x - 2, nx, bc), xa2 = bmap(x + 2, nx, bc);
-        const int ys2 = bmap(y - 2, ny, bc), ya2 = bmap(y + 2, ny, bc);
-        return (r[xs1] + r[xs2] + r[xa1] + r[xa2] + f[(size_t)ys1 * nx + x] + f[(size_t)ys2 * nx + x] +
-                f[(size_t)ya1 * nx + x] + f[(size_t)ya2 * nx + x] - 8.0 * c) * inv;
-    }
-    return (r[xs1] + r[xa1] + f[(size_t)ys1 * nx + x] + f[(size_t)ya1 * nx + x] - 4.0 * c) * inv;
-}
-
-// Workgroup sum of NG partials; thread 0 adds them to acc[g][tile].
-template <int NG>
+// Workgroup sum of NG partials over NW waves; thread 0 adds them to
+// acc[g][tile].
+template <int NG, int NW = WG / 64>
 __device__ inline void block_accumulate(double (&v)[NG], double* acc, int total_tiles, int tile, double* red) {
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
         double x = v[g];
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-        if ((threadIdx.x & 63) == 0) red[g * 4 + (threadIdx.x >> 6)] = x;
+        if ((threadIdx.x & 63) == 0) red[g * NW + (threadIdx.x >> 6)] = x;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < NG) {
+        const int g = threadIdx.x;
+        double s = red[g * NW];
 #pragma unroll
-        for (int g = 0; g < NG; ++g)
-            acc[(size_t)g * total_tiles + tile] += (red[g * 4] + red[g * 4 + 1]) + (red[g * 4 + 2] + red[g * 4 + 3]);
+        for (int i = 1; i < NW; ++i) s += red[g * NW + i];
+        acc[(size_t)g * total_tiles + tile] += s;
     }
-}
-
-// Cell (x, y) of instance D handled by this thread for item i of the tile.
-template <int TS>
-__device__ inline void tile_cell(const InstDesc& D, int w, int i, int& x, int& y) {
-    const int lt = w - D.tile_base;
-    const int ty = lt / D.tx, tx = lt - ty * D.tx;
-    const int e = threadIdx.x + i * WG;
-    y = ty * TS + e / TS;
-    x = tx * TS + e % TS;
 }
 
 // ============================================================== snowflake
 // gradient slots: 0 delta, 1 K, 2 epsb, 3 tau
 constexpr int SF_NG = 4;
 
-// Kernel 1: mu = dt/tau (lam_phi' + K lam_T'); partials of K and tau.
-template <int TS>
-__global__ __launch_bounds__(256) void sf_adj1_kernel(AdjArgs a) {
-    constexpr int PER = TS * TS / WG;
-    __shared__ double red[4 * SF_NG];
-    const int w = blockIdx.x;
-    const InstDesc& D = a.inst[a.tile_inst[w]];
-    const size_t TC = a.total_cells;
-    const double dtt = D.k[SFK_DT_OVER_TAU], K = D.k[SFK_KAPPA], tau = D.p[AMPS_SF_TAU];
-    double g[SF_NG] = {0.0, 0.0, 0.0, 0.0};
-    for (int i = 0; i < PER; ++i) {
-        int x, y;
-        tile_cell<TS>(D, w, i, x, y);
-        const size_t c = D.cell_base + (size_t)y * D.nx + x;
-        const double lp = a.lam_n[c], lt = a.lam_n[TC + c];
-        const double big = lp + K * lt;
-        a.w0[c] = dtt * big;
-        const double dphi = a.un[c] - a.u[c];
-        g[1] += lt * dphi;
-        g[3] -= big * dphi / tau;
-    }
-    block_accumulate<SF_NG>(g, a.gacc, a.total_tiles, w, red);
-}
+// Boxes of the fused reverse step in LDS for a Laplacian of reach S: phi
+// halo 2S, mu and lam_T' S + 1, the cotangents of the gradient (w1, w2) and
+// E2 mu (w3) S.  Tile 32: 67 KB at S = 2, 58.8 KB at S = 1 (two 512-thread
+// workgroups per CU); tile 16: 22 KB at S = 2.
+template <int TS, int NT, int S>
+struct SfAdjLds {
+    double phi[AdjBox<TS, 2 * S>::SZ];
+    double mu[AdjBox<TS, S + 1>::SZ], lt[AdjBox<TS, S + 1>::SZ];
+    double w1[AdjBox<TS, S>::SZ], w2[AdjBox<TS, S>::SZ], w3[AdjBox<TS, S>::SZ];
+    double red[NT / 64 * SF_NG];
+};
 
-// Kernel 2: lam(gx), lam(gy) and E2*mu at every cell; partials of delta, epsb.
-template <int TS>
-__global__ __launch_bounds__(256) void sf_adj2_kernel(AdjArgs a) {
-    constexpr int PER = TS * TS / WG;
-    __shared__ double red[4 * SF_NG];
-    const int w = blockIdx.x;
-    const InstDesc& D = a.inst[a.tile_inst[w]];
-    const double* phi = a.u + D.cell_base;
-    const double* mu = a.w0 + D.cell_base;
-    const bool ref = D.stencil == AMPS_STENCIL_REF;
+// w1 = lam(gx), w2 = lam(gy) and w3 = E2 mu at box cell (y, x) (halo S);
+// OWN: the tile's partials of delta and epsb.
+template <int TS, int NT, int S, bool MIRROR, bool OWN>
+__device__ inline void sf_adj_grad(SfAdjLds<TS, NT, S>& L, const InstDesc& D, const AdjEdge& ed, int y, int x,
+                                   bool ref, double (&g)[SF_NG]) {
+    using P = AdjBox<TS, 2 * S>;
     const int n = (int)D.k[SFK_ANISO_N];
-    const double inv2dx = D.k[SFK_INV_2DX], inv2dy = D.k[SFK_INV_2DY], inv = D.k[SFK_INV_DXDY];
+    const double inv2dx = D.k[SFK_INV_2DX], inv2dy = D.k[SFK_INV_2DY];
     const double cth0 = D.k[SFK_COS_N_THETA0], sth0 = D.k[SFK_SIN_N_THETA0];
     const double epsb = D.k[SFK_EPSB], epsbd = D.k[SFK_EPSB_DELTA], mend = D.k[SFK_MEPSB_ANISO_DELTA];
-    const double delta = D.p[AMPS_SF_DELTA];
-    double g[SF_NG] = {0.0, 0.0, 0.0, 0.0};
-    for (int i = 0; i < PER; ++i) {
-        int x, y;
-        tile_cell<TS>(D, w, i, x, y);
-        const size_t cl = (size_t)y * D.nx + x;
-        const int xs1 = bmap(x - 1, D.nx, D.bc), xa1 = bmap(x + 1, D.nx, D.bc);
-        const int ys1 = bmap(y - 1, D.ny, D.bc), ya1 = bmap(y + 1, D.ny, D.bc);
-        const double gx = (phi[(size_t)y * D.nx + xa1] - phi[(size_t)y * D.nx + xs1]) * inv2dx;
-        const double gy = (phi[(size_t)ya1 * D.nx + x] - phi[(size_t)ys1 * D.nx + x]) * inv2dy;
-        double c, s;
-        sf_unit_power<double>(gx, gy, n, c, s);
-        const double ca = c * cth0 + s * sth0, sa = s * cth0 - c * sth0;
-        const double eps = epsb + epsbd * ca, epsd = mend * sa;
-        const double A = eps * epsd;
-        const double lamP = inv2dy * (gather_y(mu, x, y, 1, D) - gather_y(mu, x, y, -1, D));
-        const double lamQ = -inv2dx * (gather_x(mu, x, y, 1, D) - gather_x(mu, x, y, -1, D));
-        const double mue = mu[cl];
-        const double lamE2 = mue * lap_fwd(phi, x, y, ref, inv, D);
-        const double lamA = lamP * gx + lamQ * gy;
-        const double lame = 2.0 * eps * lamE2 + epsd * lamA;
-        const double lamd = eps * lamA;
-        const double lamth = lame * epsd + lamd * ((double)n * mend * ca);
-        // d theta / d(gx, gy) = (-gy, gx) / |g|^2, evaluated on the rescaled
-        // gradient; the cotangent is multiplied in before the power-of-two
-        // scale 2^-e, which overflows on its own for subnormal gradients (a
-        // zero cotangent then gives 0, not 0 * inf)
-        double thx = 0.0, thy = 0.0;
-        const double mx = fmax(fabs(gx), fabs(gy));
-        if (mx != 0.0) {
-            int e;
-            frexp(mx, &e);
-            const double u = ldexp(gx, -e), v = ldexp(gy, -e);
-            const double ir2 = 1.0 / (u * u + v * v);
-            thx = ldexp(lamth * (-v * ir2), -e);
-            thy = ldexp(lamth * (u * ir2), -e);
-        }
-        a.w1[D.cell_base + cl] = A * lamP + thx;
-        a.w2[D.cell_base + cl] = A * lamQ + thy;
-        a.w3[D.cell_base + cl] = eps * eps * mue;
+    const double* f = L.phi + P::at(y, x);
+    constexpr int LW = P::LW;
+    const double gx = (f[1] - f[-1]) * inv2dx;
+    const double gy = (f[LW] - f[-LW]) * inv2dy;
+    double c, s;
+    sf_unit_power<double>(gx, gy, n, c, s);
+    const double ca = c * cth0 + s * sth0, sa = s * cth0 - c * sth0;
+    const double eps = epsb + epsbd * ca, epsd = mend * sa;
+    const double A = eps * epsd;
+    const double lamP = inv2dy * (adj_gather_y<TS, S + 1, MIRROR>(L.mu, y, x, 1, ed) -
+                                  adj_gather_y<TS, S + 1, MIRROR>(L.mu, y, x, -1, ed));
+    const double lamQ = -inv2dx * (adj_gather_x<TS, S + 1, MIRROR>(L.mu, y, x, 1, ed) -
+                                   adj_gather_x<TS, S + 1, MIRROR>(L.mu, y, x, -1, ed));
+    const double mue = L.mu[AdjBox<TS, S + 1>::at(y, x)];
+    double lap;
+    if (S == 2 && ref)
+        lap = (f[-1] + f[-2] + f[1] + f[2] + f[-LW] + f[-2 * LW] + f[LW] + f[2 * LW] - 8.0 * f[0]) *
+              D.k[SFK_INV_DXDY];
+    else
+        lap = (f[-1] + f[1] + f[-LW] + f[LW] - 4.0 * f[0]) * D.k[SFK_INV_DXDY];
+    const double lamE2 = mue * lap;
+    const double lamA = lamP * gx + lamQ * gy;
+    const double lame = 2.0 * eps * lamE2 + epsd * lamA;
+    const double lamd = eps * lamA;
+    const double lamth = lame * epsd + lamd * ((double)n * mend * ca);
+    // d theta / d(gx, gy) = (-gy, gx) / |g|^2, evaluated on the rescaled
+    // gradient; the cotangent is multiplied in before the power-of-two
+    // scale 2^-e, which overflows on its own for subnormal gradients (a
+    // zero cotangent then gives 0, not 0 * inf)
+    double thx = 0.0, thy = 0.0;
+    const double mx = fmax(fabs(gx), fabs(gy));
+    if (mx != 0.0) {
+        int e;
+        frexp(mx, &e);
+        const double u = ldexp(gx, -e), v = ldexp(gy, -e);
+        const double ir2 = 1.0 / (u * u + v * v);
+        thx = ldexp(lamth * (-v * ir2), -e);
+        thy = ldexp(lamth * (u * ir2), -e);
+    }
+    const int o = AdjBox<TS, S>::at(y, x);
+    L.w1[o] = A * lamP + thx;
+    L.w2[o] = A * lamQ + thy;
+    L.w3[o] = eps * eps * mue;
+    if (OWN) {
+        const double delta = D.p[AMPS_SF_DELTA];
         g[0] += lame * (epsb * ca) + lamd * (-epsb * (double)n * sa);
         g[2] += lame * (1.0 + delta * ca) + lamd * (-(double)n * delta * sa);
     }
-    block_accumulate<SF_NG>(g, a.gacc, a.total_tiles, w, red);
 }
 
-// Kernel 3: lam_phi, lam_T of the state before the step.
-template <int TS>
-__global__ __launch_bounds__(256) void sf_adj3_kernel(AdjArgs a) {
-    constexpr int PER = TS * TS / WG;
-    const int w = blockIdx.x;
-    const InstDesc& D = a.inst[a.tile_inst[w]];
-    const size_t TC = a.total_cells;
-    const double* phi = a.u + D.cell_base;
-    const double* T = a.u + TC + D.cell_base;
-    const double* lamT1 = a.lam_n + TC + D.cell_base;
-    const double* mu = a.w0 + D.cell_base;
-    const double* lgx = a.w1 + D.cell_base;
-    const double* lgy = a.w2 + D.cell_base;
-    const double* z = a.w3 + D.cell_base;
+// The stages after staging: the gradient's cotangents on the tile and S
+// cells around it, then the tile's lam_phi and lam_T.
+template <int TS, int NT, int S, bool MIRROR, int OWN = TS * TS / NT>
+__device__ inline void sf_adj_out(SfAdjLds<TS, NT, S>& L, const AdjArgs& a, const InstDesc& D, const AdjEdge& ed,
+                                  const int (&cell)[OWN], const double (&lp0)[OWN], const double (&tv)[OWN],
+                                  double (&g)[SF_NG]) {
+    using W = AdjBox<TS, S>;
+    static_assert(W::NF <= NT, "one frame cell per thread");
+    const int tid = threadIdx.x;
     const bool ref = D.stencil == AMPS_STENCIL_REF;
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        const int e = tid + i * NT;
+        sf_adj_grad<TS, NT, S, MIRROR, true>(L, D, ed, e / TS, e % TS, ref, g);
+    }
+    if (tid < W::NF) {
+        int y, x;
+        W::frame(tid, y, x);
+        sf_adj_grad<TS, NT, S, MIRROR, false>(L, D, ed, y, x, ref, g);
+    }
+    __syncthreads();
     const double inv2dx = D.k[SFK_INV_2DX], inv2dy = D.k[SFK_INV_2DY], inv = D.k[SFK_INV_DXDY];
     const double dt = D.k[SFK_DT], aop = D.k[SFK_ALPHA_OVER_PI], gam = D.k[SFK_GAMMA], teq = D.k[SFK_TEQ];
     const double noise = D.k[SFK_NOISE];
     const uint32_t key = noise_key(D.seed, (uint64_t)(*a.step_ctr + a.step_add));
-    for (int i = 0; i < PER; ++i) {
-        int x, y;
-        tile_cell<TS>(D, w, i, x, y);
-        const size_t cl = (size_t)y * D.nx + x;
-        const double p = phi[cl], t = T[cl], m_u = mu[cl];
+    double* lam = a.lam + D.cell_base;
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        const int e = tid + i * NT, y = e / TS, x = e % TS;
+        const double p = L.phi[AdjBox<TS, 2 * S>::at(y, x)], t = tv[i];
+        const double m_u = L.mu[AdjBox<TS, S + 1>::at(y, x)];
         const double arg = gam * (teq - t);
         const double m = aop * atan(arg);
         const double pp = p * (1.0 - p);
         double dR = (1.0 - 2.0 * p) * (p - 0.5 + m) + pp;
         if (noise != 0.0) {
-            const double u = (double)noise_u24(key, (uint32_t)cl);
+            const double u = (double)noise_u24(key, (uint32_t)cell[i]);
             dR += noise * (1.0 - 2.0 * p) * (u - 0.5);
         }
-        double lp = a.lam_n[D.cell_base + cl] + m_u * dR;
-        lp += inv2dx * (gather_x(lgx, x, y, 1, D) - gather_x(lgx, x, y, -1, D));
-        lp += inv2dy * (gather_y(lgy, x, y, 1, D) - gather_y(lgy, x, y, -1, D));
-        lp += inv * lapT(z, x, y, ref, D);
+        double lp = lp0[i] + m_u * dR;
+        lp += inv2dx * (adj_gather_x<TS, S, MIRROR>(L.w1, y, x, 1, ed) - adj_gather_x<TS, S, MIRROR>(L.w1, y, x, -1, ed));
+        lp += inv2dy * (adj_gather_y<TS, S, MIRROR>(L.w2, y, x, 1, ed) - adj_gather_y<TS, S, MIRROR>(L.w2, y, x, -1, ed));
+        lp += inv * adj_lapT<TS, S, MIRROR>(L.w3, y, x, ref, ed);
         const double dmdT = aop * (-gam) / (1.0 + arg * arg);
-        const double lt = lamT1[cl] + m_u * pp * dmdT + dt * inv * lapT(lamT1, x, y, ref, D);
-        a.lam[D.cell_base + cl] = lp;
-        a.lam[TC + D.cell_base + cl] = lt;
+        const double lt = L.lt[AdjBox<TS, S + 1>::at(y, x)] + m_u * pp * dmdT +
+                          dt * inv * adj_lapT<TS, S + 1, MIRROR>(L.lt, y, x, ref, ed);
+        lam[cell[i]] = lp;
+        lam[a.total_cells + cell[i]] = lt;
     }
+}
+
+// One reverse step: a workgroup stages phi and both cotangents of its tile
+// with their halos, forms mu = dt/tau (lam_phi' + K lam_T') on the way in,
+// and writes the tile's lam_phi and lam_T: 56 B of state traffic per cell
+// where three kernels over full-grid work arrays moved about 130.  512^2,
+// tile 16, reach 2: 11.1 us a step against 25.4 for the three kernels (3.5 us
+// of it a launch's fixed cost; the tiles' chains of rcp, ldexp and atan
+// otherwise).
+template <int TS, int NT, int S>
+__global__ __launch_bounds__(NT, 4) void sf_adj_kernel(AdjArgs a) {
+    using P = AdjBox<TS, 2 * S>;
+    using M = AdjBox<TS, S + 1>;
+    constexpr int OWN = TS * TS / NT, FP = (P::NF + NT - 1) / NT;
+    static_assert(M::NF <= NT, "one frame cell per thread");
+    __shared__ SfAdjLds<TS, NT, S> L;
+    const int w = xcd_remap(blockIdx.x, gridDim.x);
+    const InstDesc& D = a.inst[a.tile_inst[w]];
+    const int lti = w - D.tile_base, tyi = lti / D.tx;
+    const int oy = tyi * TS, ox = (lti - tyi * D.tx) * TS;
+    const size_t TC = a.total_cells;
+    const double* u = a.u + D.cell_base;
+    const double* un = a.un + D.cell_base;
+    const double* ln = a.lam_n + D.cell_base;
+    const int tid = threadIdx.x;
+    const double dtt = D.k[SFK_DT_OVER_TAU], K = D.k[SFK_KAPPA], tau = D.p[AMPS_SF_TAU];
+    // every load of the tile in flight before the first LDS store
+    double pv[OWN], pn[OWN], tv[OWN], lp[OWN], lt[OWN], fp[FP], fl, ft;
+    int cell[OWN], py[FP], px[FP], my, mx;
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        const int e = tid + i * NT;
+        cell[i] = (oy + e / TS) * D.nx + ox + e % TS;
+        lp[i] = ln[cell[i]];
+        lt[i] = ln[TC + cell[i]];
+        pv[i] = u[cell[i]];
+        pn[i] = un[cell[i]];
+        tv[i] = u[TC + cell[i]];
+    }
+#pragma unroll
+    for (int k = 0; k < FP; ++k) {
+        P::frame(tid + k * NT < P::NF ? tid + k * NT : 0, py[k], px[k]);
+        fp[k] = u[adj_cell(D, oy + py[k], ox + px[k])];
+    }
+    M::frame(tid < M::NF ? tid : 0, my, mx);
+    {
+        const int c = adj_cell(D, oy + my, ox + mx);
+        fl = ln[c];
+        ft = ln[TC + c];
+    }
+    double g[SF_NG] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        const int e = tid + i * NT, y = e / TS, x = e % TS;
+        const double big = lp[i] + K * lt[i];
+        L.phi[P::at(y, x)] = pv[i];
+        L.mu[M::at(y, x)] = dtt * big;
+        L.lt[M::at(y, x)] = lt[i];
+        const double dphi = pn[i] - pv[i];
+        g[1] += lt[i] * dphi;
+        g[3] -= big * dphi / tau;
+    }
+#pragma unroll
+    for (int k = 0; k < FP; ++k)
+        if (tid + k * NT < P::NF) L.phi[P::at(py[k], px[k])] = fp[k];
+    if (tid < M::NF) {
+        const double big = fl + K * ft;
+        L.mu[M::at(my, mx)] = dtt * big;
+        L.lt[M::at(my, mx)] = ft;
+    }
+    __syncthreads();
+    const AdjEdge ed{oy, ox, D.ny, D.nx};
+    if (adj_mirror(D, oy, ox, TS)) sf_adj_out<TS, NT, S, true>(L, a, D, ed, cell, lp, tv, g);
+    else sf_adj_out<TS, NT, S, false>(L, a, D, ed, cell, lp, tv, g);
+    block_accumulate<SF_NG, NT / 64>(g, a.gacc, a.total_tiles, w, L.red);
 }
 
 // ============================================================== sintering
 // gradient slots: 0 Dsurf, 1 Dgb, 2 kappa_c, 3 kappa_eta, 4 L, 5 Dvol
 constexpr int SN_NG = 6;
 
-__device__ inline double sn_mu(const double* c, const double* e1, const double* e2, int x, int y,
-                               const InstDesc& D) {
-    const size_t cl = (size_t)y * D.nx + x;
-    const double cv = c[cl], a1 = e1[cl], a2 = e2[cl];
-    const double con_lap = lap_fwd(c, x, y, false, D.k[SNK_INV_DXDY], D);
+// Boxes of the fused reverse step in LDS, by halo: c 4, etas and mu 3, Y 2,
+// nu 1; lam_mu (halo 1) takes mu's place once every mu_lap is formed.  At
+// tile 32: 76.8 KB, two 512-thread workgroups per CU.
+template <int TS, int NT>
+struct SnAdjLds {
+    using C = AdjBox<TS, 4>;
+    using E = AdjBox<TS, 3>;
+    using Y2 = AdjBox<TS, 2>;
+    using N1 = AdjBox<TS, 1>;
+    double c[C::SZ];
+    double e[2][E::SZ];
+    double mu[E::SZ];
+    double Y[Y2::SZ];
+    double nu[2][N1::SZ];
+    double red[NT / 64 * SN_NG];
+};
+
+// What a tile cell keeps from the mu_lap stage for the last one.
+struct SnAdjOwn {
+    double mu_lap, cn, kap;
+};
+
+// mu at box cell (y, x) (sintering/function.h:67-72).
+template <int TS, int NT>
+__device__ inline double sn_adj_mu(const SnAdjLds<TS, NT>& L, const InstDesc& D, int y, int x) {
+    using C = AdjBox<TS, 4>;
+    using E = AdjBox<TS, 3>;
+    const int i = C::at(y, x), k = E::at(y, x);
+    const double cv = L.c[i], a1 = L.e[0][k], a2 = L.e[1][k];
+    const double con_lap =
+        (L.c[i - 1] + L.c[i + 1] + L.c[i - C::LW] + L.c[i + C::LW] - 4.0 * cv) * D.k[SNK_INV_DXDY];
     const double sum2 = a1 * a1 + a2 * a2, sum3 = a1 * a1 * a1 + a2 * a2 * a2, om = 1.0 - cv;
     const double B = D.k[SNK_B], A2 = D.k[SNK_A2];
     const double df = B * (2.0 * cv + 4.0 * sum3 - 6.0 * sum2) - A2 * (cv * cv) * om + A2 * cv * (om * om);
     return df - D.k[SNK_HALF_KC] * con_lap;
 }
 
-// Kernel 0: mu of the state before the step (w0).
-template <int TS>
-__global__ __launch_bounds__(256) void sn_adj0_kernel(AdjArgs a) {
-    constexpr int PER = TS * TS / WG;
-    const int w = blockIdx.x;
-    const InstDesc& D = a.inst[a.tile_inst[w]];
-    const size_t TC = a.total_cells;
-    const double* c = a.u + D.cell_base;
-    const double* e1 = a.u + TC + D.cell_base;
-    const double* e2 = a.u + 2 * TC + D.cell_base;
-    for (int i = 0; i < PER; ++i) {
-        int x, y;
-        tile_cell<TS>(D, w, i, x, y);
-        a.w0[D.cell_base + (size_t)y * D.nx + x] = sn_mu(c, e1, e2, x, y, D);
-    }
-}
-
-// Kernel 1: clamp masks, the cotangent kappa of c's pre-clamp update, nu_i of
-// the etas', Y = kappa dt M (for lap^T into mu); partials of Dsurf, Dgb, Dvol,
-// kappa_eta, L.
-template <int TS>
-__global__ __launch_bounds__(256) void sn_adj1_kernel(AdjArgs a) {
-    constexpr int PER = TS * TS / WG;
-    __shared__ double red[4 * SN_NG];
-    const int w = blockIdx.x;
-    const InstDesc& D = a.inst[a.tile_inst[w]];
-    const size_t TC = a.total_cells;
-    const double* c = a.u + D.cell_base;
-    const double* e[2] = {a.u + TC + D.cell_base, a.u + 2 * TC + D.cell_base};
-    const double* mu = a.w0 + D.cell_base;
+// The stage of the clamp masks at box cell (y, x) (halo 2): Y = kappa dt M
+// with kappa the cotangent of c's pre-clamp update, and nu_k of the etas'
+// (halo 1).  ln: the three cotangents of the state after the step there.
+// OWN: a tile cell, whose parameter partials are added to g and whose
+// mu_lap, c' and kappa are kept.
+template <int TS, int NT, bool OWN>
+__device__ inline void sn_adj_mask(SnAdjLds<TS, NT>& L, const InstDesc& D, int y, int x, const double (&ln)[3],
+                                   double (&g)[SN_NG], SnAdjOwn& own) {
+    using E = AdjBox<TS, 3>;
+    const int i = E::at(y, x);
+    const double cv = L.c[AdjBox<TS, 4>::at(y, x)], a1 = L.e[0][i], a2 = L.e[1][i];
     const double inv = D.k[SNK_INV_DXDY], dt = D.k[SNK_DT], B = D.k[SNK_B];
-    const double dvol = D.k[SNK_DVOL], dvap = D.k[SNK_DVAP], dsur = D.k[SNK_DSURF], dgb = D.k[SNK_DGB];
     const double dtl = D.k[SNK_DT_L], hke = D.k[SNK_HALF_KE];
-    double g[SN_NG] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int i = 0; i < PER; ++i) {
-        int x, y;
-        tile_cell<TS>(D, w, i, x, y);
-        const size_t cl = (size_t)y * D.nx + x;
-        const double cv = c[cl], a1 = e[0][cl], a2 = e[1][cl];
-        const double mu_lap = lap_fwd(mu, x, y, false, inv, D);
-        const double h = cv * cv * cv * (10.0 - 15.0 * cv + 6.0 * (cv * cv));
-        const double mob = dvol * h + dvap * (1.0 - h) + dsur * cv * (1.0 - cv) + dgb * (a1 * a2 * 2.0);
-        const double v = cv + dt * mob * mu_lap;
-        const double cn = v >= 1.0 ? 1.0 : (v < 0.0 ? 0.0 : v);
-        const double gc = (v >= 0.0 && v < 1.0) ? 1.0 : 0.0;
-        const double sum2 = a1 * a1 + a2 * a2;
-        double lcn = a.lam_n[D.cell_base + cl];
-        double nu[2];
-        for (int k = 0; k < 2; ++k) {
-            const double ak = k == 0 ? a1 : a2;
-            const double l = lap_fwd(e[k], x, y, false, inv, D);
-            const double dk = B * (-12.0 * (ak * ak) * (2.0 - cn) + 12.0 * ak * (1.0 - cn) + 12.0 * ak * sum2);
-            const double wk = ak - dtl * (dk - hke * l);
-            const double gk = (wk >= 0.0 && wk < 1.0) ? 1.0 : 0.0;
-            nu[k] = a.lam_n[(size_t)(1 + k) * TC + D.cell_base + cl] * gk;
-            lcn += nu[k] * (-dtl) * B * (12.0 * ak * ak - 12.0 * ak);
-            g[3] += nu[k] * dtl * 0.5 * l;                 // d w_k / d kappa_eta
-            g[4] += nu[k] * (-dt) * (dk - hke * l);        // d w_k / d L
+    const double mu_lap = (L.mu[i - 1] + L.mu[i + 1] + L.mu[i - E::LW] + L.mu[i + E::LW] - 4.0 * L.mu[i]) * inv;
+    const double h = cv * cv * cv * (10.0 - 15.0 * cv + 6.0 * (cv * cv));
+    const double mob = D.k[SNK_DVOL] * h + D.k[SNK_DVAP] * (1.0 - h) + D.k[SNK_DSURF] * cv * (1.0 - cv) +
+                       D.k[SNK_DGB] * (a1 * a2 * 2.0);
+    const double v = cv + dt * mob * mu_lap;
+    const double cn = v >= 1.0 ? 1.0 : (v < 0.0 ? 0.0 : v);
+    const double gc = (v >= 0.0 && v < 1.0) ? 1.0 : 0.0;
+    const double sum2 = a1 * a1 + a2 * a2;
+    double lcn = ln[0];
+    const bool ring1 = OWN || (y >= -1 && y <= TS && x >= -1 && x <= TS);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const double ak = k == 0 ? a1 : a2;
+        const double* e = L.e[k];
+        const double l = (e[i - 1] + e[i + 1] + e[i - E::LW] + e[i + E::LW] - 4.0 * ak) * inv;
+        const double dk = B * (-12.0 * (ak * ak) * (2.0 - cn) + 12.0 * ak * (1.0 - cn) + 12.0 * ak * sum2);
+        const double wk = ak - dtl * (dk - hke * l);
+        const double gk = (wk >= 0.0 && wk < 1.0) ? 1.0 : 0.0;
+        const double nu = ln[1 + k] * gk;
+        lcn += nu * (-dtl) * B * (12.0 * ak * ak - 12.0 * ak);
+        if (ring1) L.nu[k][AdjBox<TS, 1>::at(y, x)] = nu;
+        if (OWN) {
+            g[3] += nu * dtl * 0.5 * l;             // d w_k / d kappa_eta
+            g[4] += nu * (-dt) * (dk - hke * l);    // d w_k / d L
         }
-        const double kap = lcn * gc;
-        a.w1[D.cell_base + cl] = kap * dt * mob;
-        a.w2[D.cell_base + cl] = kap;
-        a.w3[D.cell_base + cl] = nu[0];
-        a.w4[D.cell_base + cl] = nu[1];
+    }
+    const double kap = lcn * gc;
+    L.Y[AdjBox<TS, 2>::at(y, x)] = kap * dt * mob;
+    if (OWN) {
+        own.mu_lap = mu_lap;
+        own.cn = cn;
+        own.kap = kap;
         const double q = kap * dt * mu_lap;
         g[0] += q * cv * (1.0 - cv);
         g[1] += q * (a1 * a2 * 2.0);
         g[5] += q * h;
     }
-    block_accumulate<SN_NG>(g, a.gacc, a.total_tiles, w, red);
 }
 
-// Kernel 2: lam_mu = lap^T(Y) (w5); partial of kappa_c.
-template <int TS>
-__global__ __launch_bounds__(256) void sn_adj2_kernel(AdjArgs a) {
-    constexpr int PER = TS * TS / WG;
-    __shared__ double red[4 * SN_NG];
-    const int w = blockIdx.x;
-    const InstDesc& D = a.inst[a.tile_inst[w]];
-    const double* c = a.u + D.cell_base;
-    const double* Y = a.w1 + D.cell_base;
-    const double inv = D.k[SNK_INV_DXDY];
-    double g[SN_NG] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int i = 0; i < PER; ++i) {
-        int x, y;
-        tile_cell<TS>(D, w, i, x, y);
-        const size_t cl = (size_t)y * D.nx + x;
-        const double lmu = inv * lapT(Y, x, y, false, D);
-        a.w5[D.cell_base + cl] = lmu;
-        g[2] += lmu * (-0.5) * lap_fwd(c, x, y, false, inv, D);
+// The last two stages: lam_mu = lap^T(Y) on the tile and its ring, in mu's
+// place, then the tile's cotangents; adds the kappa_c partial to g2.
+template <int TS, int NT, bool MIRROR, int OWN = TS * TS / NT>
+__device__ inline void sn_adj_out(SnAdjLds<TS, NT>& L, const InstDesc& D, const AdjEdge& ed,
+                                  const SnAdjOwn (&own)[OWN], const int (&cell)[OWN], double& g2, double* lam,
+                                  size_t TC) {
+    using C = AdjBox<TS, 4>;
+    using E = AdjBox<TS, 3>;
+    using N1 = AdjBox<TS, 1>;
+    const int tid = threadIdx.x;
+    const double inv = D.k[SNK_INV_DXDY], dt = D.k[SNK_DT];
+    double* lmu = L.mu;
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        const int e = tid + i * NT, y = e / TS, x = e % TS;
+        const double lm = inv * adj_lapT<TS, 2, MIRROR>(L.Y, y, x, false, ed);
+        lmu[N1::at(y, x)] = lm;
+        const int k = C::at(y, x);
+        const double l = (L.c[k - 1] + L.c[k + 1] + L.c[k - C::LW] + L.c[k + C::LW] - 4.0 * L.c[k]) * inv;
+        g2 += lm * (-0.5) * l;
     }
-    block_accumulate<SN_NG>(g, a.gacc, a.total_tiles, w, red);
-}
-
-// Kernel 3: lam_c, lam_eta1, lam_eta2 of the state before the step.
-template <int TS>
-__global__ __launch_bounds__(256) void sn_adj3_kernel(AdjArgs a) {
-    constexpr int PER = TS * TS / WG;
-    const int w = blockIdx.x;
-    const InstDesc& D = a.inst[a.tile_inst[w]];
-    const size_t TC = a.total_cells;
-    const double* c = a.u + D.cell_base;
-    const double* e1 = a.u + TC + D.cell_base;
-    const double* e2 = a.u + 2 * TC + D.cell_base;
-    const double* mu = a.w0 + D.cell_base;
-    const double* kapa = a.w2 + D.cell_base;
-    const double* nua[2] = {a.w3 + D.cell_base, a.w4 + D.cell_base};
-    const double* lmua = a.w5 + D.cell_base;
-    const double inv = D.k[SNK_INV_DXDY], dt = D.k[SNK_DT], B = D.k[SNK_B], A2 = D.k[SNK_A2];
-    const double dvol = D.k[SNK_DVOL], dvap = D.k[SNK_DVAP], dsur = D.k[SNK_DSURF], dgb = D.k[SNK_DGB];
+    if (tid < N1::NF) {
+        int y, x;
+        N1::frame(tid, y, x);
+        lmu[N1::at(y, x)] = inv * adj_lapT<TS, 2, MIRROR>(L.Y, y, x, false, ed);
+    }
+    __syncthreads();
+    const double B = D.k[SNK_B], A2 = D.k[SNK_A2];
     const double dtl = D.k[SNK_DT_L], hke = D.k[SNK_HALF_KE], hkc = D.k[SNK_HALF_KC];
-    for (int i = 0; i < PER; ++i) {
-        int x, y;
-        tile_cell<TS>(D, w, i, x, y);
-        const size_t cl = (size_t)y * D.nx + x;
-        const double cv = c[cl], a1 = e1[cl], a2 = e2[cl], om = 1.0 - cv;
-        const double cn = a.un[D.cell_base + cl];
-        const double mu_lap = lap_fwd(mu, x, y, false, inv, D);
-        const double kap = kapa[cl], lmu = lmua[cl];
-        const double h = cv * cv * cv * (10.0 - 15.0 * cv + 6.0 * (cv * cv));
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        const int e = tid + i * NT, y = e / TS, x = e % TS;
+        const int k = E::at(y, x), r = N1::at(y, x);
+        const double cv = L.c[C::at(y, x)], a1 = L.e[0][k], a2 = L.e[1][k], om = 1.0 - cv;
+        const double cn = own[i].cn, kap = own[i].kap, lm = lmu[r];
         const double hp = 3.0 * cv * cv * (10.0 - 15.0 * cv + 6.0 * (cv * cv)) + cv * cv * cv * (-15.0 + 12.0 * cv);
-        (void)h;
-        const double dMdc = (dvol - dvap) * hp + dsur * (1.0 - 2.0 * cv);
+        const double dMdc = (D.k[SNK_DVOL] - D.k[SNK_DVAP]) * hp + D.k[SNK_DSURF] * (1.0 - 2.0 * cv);
         const double dfdc = 2.0 * B - A2 * (2.0 * cv * om - cv * cv) + A2 * (om * om - 2.0 * cv * om);
-        const double q = kap * dt * mu_lap;
-        const double lc = kap + q * dMdc + lmu * dfdc - hkc * inv * lapT(lmua, x, y, false, D);
-        a.lam[D.cell_base + cl] = lc;
+        const double q = kap * dt * own[i].mu_lap;
+        lam[cell[i]] = kap + q * dMdc + lm * dfdc - hkc * inv * adj_lapT<TS, 1, MIRROR>(lmu, y, x, false, ed);
         const double sum2 = a1 * a1 + a2 * a2;
-        for (int k = 0; k < 2; ++k) {
-            const double ak = k == 0 ? a1 : a2, aj = k == 0 ? a2 : a1;
-            const double nuk = nua[k][cl], nuj = nua[1 - k][cl];
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            const double ak = f == 0 ? a1 : a2, aj = f == 0 ? a2 : a1;
+            const double nuk = L.nu[f][r], nuj = L.nu[1 - f][r];
             const double ddk = B * (-24.0 * ak * (2.0 - cn) + 12.0 * (1.0 - cn) + 12.0 * sum2 + 24.0 * ak * ak);
             double la = nuk * (1.0 - dtl * ddk) + nuj * (-dtl) * B * 24.0 * aj * ak;
-            la += q * dgb * 2.0 * aj + lmu * B * (12.0 * ak * ak - 12.0 * ak);
-            la += dtl * hke * inv * lapT(nua[k], x, y, false, D);
-            a.lam[(size_t)(1 + k) * TC + D.cell_base + cl] = la;
+            la += q * D.k[SNK_DGB] * 2.0 * aj + lm * B * (12.0 * ak * ak - 12.0 * ak);
+            la += dtl * hke * inv * adj_lapT<TS, 1, MIRROR>(L.nu[f], y, x, false, ed);
+            lam[(size_t)(1 + f) * TC + cell[i]] = la;
         }
     }
+}
+
+// One reverse step: a workgroup stages c (halo 4), the etas (3) and the
+// cotangents (2), evaluates mu on the tile and 3 cells around it, Y on 2, nu
+// and lam_mu on 1, and writes the tile's three cotangents: 72 B of state
+// traffic per cell where four kernels over full-grid work arrays moved about
+// 250.  The re-evaluated rings cost 1.41x (mu), 1.27x (masks) and 1.13x
+// (lam_mu) of a tile's arithmetic at tile 32.  1024^2: 32 us a step against
+// 78 for the four kernels; bound by the latency of its five stages at 16
+// waves per CU (LDS and 126 VGPRs), about 14 us of VALU issue.  Tile 16 (5
+// waves per SIMD, rings 1.89x/1.56x/1.27x): 37 us.
+template <int TS, int NT>
+__global__ __launch_bounds__(NT, 4) void sn_adj_kernel(AdjArgs a) {
+    using C = AdjBox<TS, 4>;
+    using E = AdjBox<TS, 3>;
+    using Y2 = AdjBox<TS, 2>;
+    constexpr int OWN = TS * TS / NT, FC = (C::NF + NT - 1) / NT;
+    static_assert(E::NF <= NT, "one frame cell per thread");
+    __shared__ SnAdjLds<TS, NT> L;
+    const int w = xcd_remap(blockIdx.x, gridDim.x);
+    const InstDesc& D = a.inst[a.tile_inst[w]];
+    const int lt = w - D.tile_base, tyi = lt / D.tx;
+    const int oy = tyi * TS, ox = (lt - tyi * D.tx) * TS;
+    const size_t TC = a.total_cells;
+    const double* u = a.u + D.cell_base;
+    const double* ln = a.lam_n + D.cell_base;
+    const int tid = threadIdx.x;
+    // the boxes' loads in flight together before the first LDS store
+    double vc[OWN], ve[2][OWN], vl[OWN][3], fc[FC], fe[2], fl[3];
+    int cell[OWN];
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        const int e = tid + i * NT;
+        cell[i] = (oy + e / TS) * D.nx + ox + e % TS;
+        vc[i] = u[cell[i]];
+        ve[0][i] = u[TC + cell[i]];
+        ve[1][i] = u[2 * TC + cell[i]];
+    }
+    int cy[FC], cx[FC], ey, ex, yy, yx;
+#pragma unroll
+    for (int k = 0; k < FC; ++k) {
+        C::frame(tid + k * NT < C::NF ? tid + k * NT : 0, cy[k], cx[k]);
+        fc[k] = u[adj_cell(D, oy + cy[k], ox + cx[k])];
+    }
+    {
+        E::frame(tid < E::NF ? tid : 0, ey, ex);
+        const int g = adj_cell(D, oy + ey, ox + ex);
+        fe[0] = u[TC + g];
+        fe[1] = u[2 * TC + g];
+    }
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        const int e = tid + i * NT, y = e / TS, x = e % TS;
+        L.c[C::at(y, x)] = vc[i];
+        L.e[0][E::at(y, x)] = ve[0][i];
+        L.e[1][E::at(y, x)] = ve[1][i];
+    }
+#pragma unroll
+    for (int k = 0; k < FC; ++k)
+        if (tid + k * NT < C::NF) L.c[C::at(cy[k], cx[k])] = fc[k];
+    if (tid < E::NF) {
+        L.e[0][E::at(ey, ex)] = fe[0];
+        L.e[1][E::at(ey, ex)] = fe[1];
+    }
+    // the cotangents arrive during the mu stage
+#pragma unroll
+    for (int i = 0; i < OWN; ++i)
+#pragma unroll
+        for (int f = 0; f < 3; ++f) vl[i][f] = ln[f * TC + cell[i]];
+    {
+        Y2::frame(tid < Y2::NF ? tid : 0, yy, yx);
+        const int g = adj_cell(D, oy + yy, ox + yx);
+#pragma unroll
+        for (int f = 0; f < 3; ++f) fl[f] = ln[f * TC + g];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        const int e = tid + i * NT, y = e / TS, x = e % TS;
+        L.mu[E::at(y, x)] = sn_adj_mu<TS, NT>(L, D, y, x);
+    }
+    if (tid < E::NF) L.mu[E::at(ey, ex)] = sn_adj_mu<TS, NT>(L, D, ey, ex);
+    __syncthreads();
+    double g[SN_NG] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    SnAdjOwn own[OWN];
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        const int e = tid + i * NT;
+        sn_adj_mask<TS, NT, true>(L, D, e / TS, e % TS, vl[i], g, own[i]);
+    }
+    if (tid < Y2::NF) {
+        SnAdjOwn unused;
+        sn_adj_mask<TS, NT, false>(L, D, yy, yx, fl, g, unused);
+    }
+    __syncthreads();
+    const AdjEdge ed{oy, ox, D.ny, D.nx};
+    double* lam = a.lam + D.cell_base;
+    if (adj_mirror(D, oy, ox, TS)) sn_adj_out<TS, NT, true>(L, D, ed, own, cell, g[2], lam, TC);
+    else sn_adj_out<TS, NT, false>(L, D, ed, own, cell, g[2], lam, TC);
+    block_accumulate<SN_NG, NT / 64>(g, a.gacc, a.total_tiles, w, L.red);
 }
 
 // ------------------------------------------------------------ host launch
 int launch_adjoint_step(const AdjArgs& a, int model, int tile, hipStream_t s) {
-    const dim3 g(a.total_tiles), b(WG);
+    const dim3 g(a.total_tiles);
     if (tile != 16 && tile != 32) return AMPS_E_UNSUPPORTED;
     if (model == AMPS_SNOWFLAKE) {
+        // S: the reach of the widest Laplacian among the instances
         if (tile == 16) {
-            hipLaunchKernelGGL(sf_adj1_kernel<16>, g, b, 0, s, a);
-            hipLaunchKernelGGL(sf_adj2_kernel<16>, g, b, 0, s, a);
-            hipLaunchKernelGGL(sf_adj3_kernel<16>, g, b, 0, s, a);
+            if (a.t_halo == 2) hipLaunchKernelGGL((sf_adj_kernel<16, 256, 2>), g, dim3(256), 0, s, a);
+            else hipLaunchKernelGGL((sf_adj_kernel<16, 256, 1>), g, dim3(256), 0, s, a);
         } else {
-            hipLaunchKernelGGL(sf_adj1_kernel<32>, g, b, 0, s, a);
-            hipLaunchKernelGGL(sf_adj2_kernel<32>, g, b, 0, s, a);
-            hipLaunchKernelGGL(sf_adj3_kernel<32>, g, b, 0, s, a);
+            if (a.t_halo == 2) hipLaunchKernelGGL((sf_adj_kernel<32, 512, 2>), g, dim3(512), 0, s, a);
+            else hipLaunchKernelGGL((sf_adj_kernel<32, 512, 1>), g, dim3(512), 0, s, a);
         }
     } else if (model == AMPS_SINTERING) {
-        if (tile == 16) {
-            hipLaunchKernelGGL(sn_adj0_kernel<16>, g, b, 0, s, a);
-            hipLaunchKernelGGL(sn_adj1_kernel<16>, g, b, 0, s, a);
-            hipLaunchKernelGGL(sn_adj2_kernel<16>, g, b, 0, s, a);
-            hipLaunchKernelGGL(sn_adj3_kernel<16>, g, b, 0, s, a);
-        } else {
-            hipLaunchKernelGGL(sn_adj0_kernel<32>, g, b, 0, s, a);
-            hipLaunchKernelGGL(sn_adj1_kernel<32>, g, b, 0, s, a);
-            hipLaunchKernelGGL(sn_adj2_kernel<32>, g, b, 0, s, a);
-            hipLaunchKernelGGL(sn_adj3_kernel<32>, g, b, 0, s, a);
-        }
+        if (tile == 16) hipLaunchKernelGGL((sn_adj_kernel<16, 256>), g, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((sn_adj_kernel<32, 512>), g, dim3(512), 0, s, a);
     } else {
         return AMPS_E_UNSUPPORTED;
     }

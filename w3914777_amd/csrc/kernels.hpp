@@ -56,7 +56,7 @@ int launch_gg_aux(const StepArgs& a, int tile, const int* type_old, hipStream_t 
 int launch_sn_step(const StepArgs& a, int tile, bool adaptive, int grid, hipStream_t s, const hipEvent_t* ev = nullptr);
 
 // Reverse-time adjoint of one FP64 step (snowflake, sintering).  Arrays are
-// [field][total_cells] like the FP64 state; work arrays hold total_cells.
+// [field][total_cells] like the FP64 state.
 struct AdjArgs {
     const InstDesc* inst;
     const int* tile_inst;
@@ -66,15 +66,10 @@ struct AdjArgs {
     const double* un;      // state after the step
     const double* lam_n;   // dJ/d(state after)
     double* lam;           // dJ/d(state before), written
-    double* w0;            // work arrays, one value per cell
-    double* w1;
-    double* w2;
-    double* w3;
-    double* w4;
-    double* w5;
     double* gacc;          // [gradient slot][total_tiles] accumulators
     const long long* step_ctr;  // step index of the forward step = *step_ctr + step_add
     int step_add;
+    int t_halo;            // snowflake: reach of the widest Laplacian among the instances
 };
 int launch_adjoint_step(const AdjArgs& a, int model, int tile, hipStream_t s);
 
