@@ -61,6 +61,13 @@ __host__ __device__ inline int bmap(int i, int n, int bc) {
     return i < 0 ? -i : 2 * (n - 1) - i;
 }
 
+// The same map by selects (a branch around a load's address would split the
+// loads of a box into rounds).
+__device__ inline int map_cell(int i, int n, bool per) {
+    const int lo = per ? i + n : -i, hi = per ? i - n : 2 * (n - 1) - i;
+    return i < 0 ? lo : (i >= n ? hi : i);
+}
+
 // ------------------------------------------------------------- counter RNG
 // SplitMix64 finaliser keyed by (seed, stream, index); bit-identical to the
 // host implementation so seeded noise is reproducible on any device.
@@ -137,6 +144,18 @@ struct StepArgs {
     Buf in, out;
     double* aux_in;             // model auxiliary per-cell array (grain growth: sum of squares)
     double* aux_out;
+};
+
+// Plan of a PURE_FP64 context's multi-step launches: k steps (0: single steps
+// only) on square blocks whose edge (16 or 32) divides every instance's
+// sides; block b of the launch belongs to instance inst[b], whose blocks
+// start at base[instance].
+struct BlockMap {
+    int k;
+    int edge;
+    int nblocks;
+    const int* inst;
+    const int* base;
 };
 
 // NO_SKIP list of the snowflake's flat sweep: NSK_SEGS segments (list

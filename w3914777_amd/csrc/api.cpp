@@ -106,6 +106,10 @@ struct amps_ctx {
     int pending_adv = 0;
     bool initialised = false;
 
+    BlockMap bm{};                         // PURE_FP64: several steps a launch where that is faster
+    int* d_blk_inst = nullptr;
+    int* d_blk_base = nullptr;
+
     // graphs: one per starting buffer parity
     bool use_graph = true;
     int graph_period = 0;
@@ -428,6 +432,21 @@ int enqueue_one(amps_ctx* c) {
     return AMPS_OK;
 }
 
+// Whether amps_step may advance several steps a launch: nothing then looks at
+// the state, or times a sweep, between them.
+bool use_multi(const amps_ctx* c) { return c->bm.k > 1 && !c->taping && !c->ktiming; }
+
+// One launch of bm.k steps (PURE_FP64).
+int enqueue_multi(amps_ctx* c) {
+    StepArgs a = step_args(c, c->cur);
+    a.step_add = c->pending_adv;
+    RCCHK(launch_sf_multi(a, c->bm, c->stream));
+    c->pending_adv += c->bm.k;
+    c->cur ^= 1;
+    c->steps_done += c->bm.k;
+    return AMPS_OK;
+}
+
 // Capture `period` steps (monitor pass included) starting from buffer parity p.
 int build_graph(amps_ctx* c, int p) {
     hipGraph_t g = nullptr;
@@ -449,6 +468,59 @@ int build_graph(amps_ctx* c, int p) {
     return AMPS_OK;
 }
 
+}  // namespace
+
+namespace {
+// Number of edge x edge blocks of the context's grids; 0 if edge does not
+// divide every side (16 divides every tile edge).
+long long block_count(const amps_ctx* c, int edge) {
+    long long n = 0;
+    for (const InstDesc& d : c->desc) {
+        if (d.nx % edge || d.ny % edge) return 0;
+        n += (long long)(d.nx / edge) * (d.ny / edge);
+    }
+    return n;
+}
+
+// Steps per launch of a PURE_FP64 snowflake context.
+//
+// A single step of a small grid is its launch and one tile's chain of
+// dependent operations (5 us from 64^2 to 256^2, 6.3 at 512^2), so K steps
+// share a launch and the halo's redundant cells are paid from idle compute
+// units: worth it while there are few blocks per CU.  Measured on 256 CUs, us
+// a step against the single step's, reference physics (workload physics in
+// brackets):
+//   16^2 blocks, K = 4:  256^2 (256 blocks) 2.2 : 5.0 (2.5 : 4.9); 320^2 (400) 3.0 : 5.3 (3.3 : 5.2)
+//   16^2 blocks, K = 3:  320^2 (400) 3.0 (3.2); 384^2 (576) 3.6 : 5.6 (3.9 : 5.5)
+//   32^2 blocks, K = 3:  384^2 (144) 3.5 (4.0); 512^2 (256) 3.6 : 6.3 (4.1 : 6.1); 640^2 (400) 6.6 : 7.8 (7.1 : 7.6)
+//   16^2 blocks, K = 2:  512^2 (1024) 4.6 (5.1); 640^2 (1600) 6.6 (7.0); 768^2 (2304) 8.1 : 9.7 (8.5 : 9.4)
+// Larger grids fill the chip with single steps and lose by the redundancy
+// (1024^2: 13.1 : 13.2 and 12.6 : 12.5; 2048^2: 43 : 36).
+int plan_multi(amps_ctx* c) {
+    if (c->mode != AMPS_PURE_FP64 || c->model != AMPS_SNOWFLAKE) return AMPS_OK;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
+    const long long b16 = block_count(c, 16), b32 = block_count(c, 32);
+    int k = 0, edge = 16;
+    if (b16 <= cus + cus / 4) k = 4;
+    else if (b32 > 0 && b32 <= cus && b16 > 2 * cus) { k = 3; edge = 32; }
+    else if (b16 <= 2 * cus + cus / 4) k = 3;
+    else if (b16 <= 9 * cus) k = 2;
+    if (k == 0) return AMPS_OK;
+    std::vector<int> inst, base;
+    for (int i = 0; i < c->ninst; ++i) {
+        base.push_back((int)inst.size());
+        inst.insert(inst.end(), (size_t)(c->desc[i].nx / edge) * (c->desc[i].ny / edge), i);
+    }
+    RCCHK(dmalloc(c, (void**)&c->d_blk_inst, inst.size() * sizeof(int)));
+    RCCHK(dmalloc(c, (void**)&c->d_blk_base, base.size() * sizeof(int)));
+    HIPCHK(hipMemcpy(c->d_blk_inst, inst.data(), inst.size() * sizeof(int), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(c->d_blk_base, base.data(), base.size() * sizeof(int), hipMemcpyHostToDevice));
+    c->bm = BlockMap{k, edge, (int)inst.size(), c->d_blk_inst, c->d_blk_base};
+    return AMPS_OK;
+}
 }  // namespace
 
 // ============================================================ tape helpers
@@ -652,6 +724,8 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
         c->grid_cap = cfgs[0].wg_per_cu * cus;
     }
     c->graph_period = c->mode == AMPS_ADAPTIVE ? (c->every % 2 ? 2 * c->every : c->every) : 10;
+    rc = plan_multi(c);
+    if (rc != AMPS_OK) { std::string m = g_last_error; amps_destroy(c); return fail(rc, m); }
     *out = c;
     return AMPS_OK;
 }
@@ -724,7 +798,12 @@ int amps_step(amps_ctx* c, int nsteps) {
     const bool graphs = c->use_graph && !c->taping && !c->ktiming;
     while (left > 0) {
         const long long s = c->steps_done;
-        if (graphs && left >= c->graph_period && s % c->graph_period == 0) {
+        if (use_multi(c) && left >= c->bm.k) {
+            // not captured: a launch runs longer than its enqueue takes, and a
+            // graph of these adds a gap of its own per replay
+            RCCHK(enqueue_multi(c));
+            left -= c->bm.k;
+        } else if (graphs && left >= c->graph_period && s % c->graph_period == 0) {
             RCCHK(flush_adv(c));
             if (!c->gexec[c->cur]) RCCHK(build_graph(c, c->cur));
             HIPCHK(hipGraphLaunch(c->gexec[c->cur], c->stream));

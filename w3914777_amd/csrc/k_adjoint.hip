@@ -75,15 +75,10 @@ struct AdjBox {
     }
 };
 
-// Cell (gy, gx) of instance D, boundary-mapped (bmap by selects: a branch
-// around a load's address would split the loads of a tile into rounds).
-__device__ inline int adj_map(int i, int n, bool per) {
-    const int lo = per ? i + n : -i, hi = per ? i - n : 2 * (n - 1) - i;
-    return i < 0 ? lo : (i >= n ? hi : i);
-}
+// Cell (gy, gx) of instance D, boundary-mapped.
 __device__ inline int adj_cell(const InstDesc& D, int gy, int gx) {
     const bool per = D.bc == AMPS_BC_PERIODIC;
-    return adj_map(gy, D.ny, per) * D.nx + adj_map(gx, D.nx, per);
+    return map_cell(gy, D.ny, per) * D.nx + map_cell(gx, D.nx, per);
 }
 
 // Tile origin of the transposed reads.  MIRROR: the tile meets a zero-flux

@@ -1575,6 +1575,210 @@ __global__ __launch_bounds__(FLAT_NT) void sf_flat_kernel(StepArgs a, const Inst
     }
 }
 
+// ------------------------------------------------------ several FP64 steps
+// PURE_FP64: K explicit-Euler steps in one launch.  A workgroup stages phi
+// and T of a BS x BS block with a halo of 2K cells (a step's reach is 2) and
+// advances them K times in LDS, each step on a region 2 cells smaller on
+// every side; the last one writes the block.  The cells of the halo are
+// advanced by every block that holds them, with the same operations on the
+// same values, so the result is that of K single steps, bit for bit.
+//
+// Outside a zero-flux domain a cell takes what its mirror image inside the
+// domain gets (values and ring intermediates alike, as the index map of the
+// single step does), evaluated again in its place: no pass to refill ghosts.
+template <int BS, int K>
+struct SfMultiLds {
+    static constexpr int W0 = BS + 4 * K, WR = W0 - 2;
+    double f[2][2][W0 * W0];  // [generation][phi, T]
+    double P[WR * WR], Q[WR * WR], E2[WR * WR];
+};
+
+// Box coordinate of the mirror image of box coordinate b (origin o of the
+// block, halo h) on a zero-flux axis of n cells.
+__device__ inline int sf_mirror(int b, int o, int h, int n) {
+    const int g = o - h + b;
+    return g < 0 ? b - 2 * g : (g >= n ? b + 2 * (n - 1 - g) : b);
+}
+
+// Calls compute(e, r) for the cells e = tid + k NT < N of a region, then
+// store(e, r): the full passes of a thread are computed side by side (their
+// chains of dependent operations overlap), the last, partial one after them.
+template <int N, int NT, typename R, typename C, typename W>
+__device__ inline void for_cells(C&& compute, W&& store) {
+    constexpr int FULL = N / NT;
+    if constexpr (FULL > 0) {
+        R r[FULL];
+#pragma unroll
+        for (int k = 0; k < FULL; ++k) compute((int)threadIdx.x + k * NT, r[k]);
+#pragma unroll
+        for (int k = 0; k < FULL; ++k) store((int)threadIdx.x + k * NT, r[k]);
+    }
+    if constexpr (N % NT != 0) {
+        if ((int)threadIdx.x + FULL * NT < N) {
+            R r;
+            compute((int)threadIdx.x + FULL * NT, r);
+            store((int)threadIdx.x + FULL * NT, r);
+        }
+    }
+}
+
+// Step S of K: ring intermediates on the region and one cell around it, then
+// the new phi and T of the region.
+template <int BS, int K, int S, int NT, bool EDGE>
+__device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepArgs& a, const InstDesc& d, int ox, int oy,
+                                     uint32_t key) {
+    using M = SfMultiLds<BS, K>;
+    constexpr int H = 2 * K, W0 = M::W0, WR = M::WR;
+    constexpr int HS = 2 * (K - 1 - S), W = BS + 2 * HS, B0 = H - HS;  // region: box coordinates B0 .. B0 + W - 1
+    const double* F = L.f[S & 1][0];
+    const double* G = L.f[S & 1][1];
+    const double inv2dx = d.k[SFK_INV_2DX], inv2dy = d.k[SFK_INV_2DY];
+    {
+        const int n = (int)d.k[SFK_ANISO_N];
+        const double cth0 = d.k[SFK_COS_N_THETA0], sth0 = d.k[SFK_SIN_N_THETA0];
+        const double epsb = d.k[SFK_EPSB], epsbd = d.k[SFK_EPSB_DELTA], mend = d.k[SFK_MEPSB_ANISO_DELTA];
+        constexpr int WP = W + 2;
+        struct Ring { double p, q, e2; };
+        for_cells<WP * WP, NT, Ring>(
+            [&](int e, Ring& r) {
+                const int y = e / WP, by = B0 - 1 + y, bx = B0 - 1 + e - y * WP;
+                int sy = by, sx = bx;
+                if (EDGE) {
+                    sy = sf_mirror(by, oy, H, d.ny);
+                    sx = sf_mirror(bx, ox, H, d.nx);
+                }
+                const int c = sy * W0 + sx;
+                const double gx = (F[c + 1] - F[c - 1]) * inv2dx;
+                const double gy = (F[c + W0] - F[c - W0]) * inv2dy;
+                double eps, epsd;
+                sf_aniso<double>(gx, gy, n, cth0, sth0, epsb, epsbd, mend, eps, epsd);
+                const double A = eps * epsd;
+                r.p = A * gx;
+                r.q = A * gy;
+                r.e2 = eps * eps;
+            },
+            [&](int e, const Ring& r) {
+                const int y = e / WP, o = (B0 - 2 + y) * WR + B0 - 2 + e - y * WP;
+                L.P[o] = r.p;
+                L.Q[o] = r.q;
+                L.E2[o] = r.e2;
+            });
+    }
+    __syncthreads();
+    const bool ref = d.stencil == AMPS_STENCIL_REF;
+    const double inv = d.k[SFK_INV_DXDY], dtt = d.k[SFK_DT_OVER_TAU], dt = d.k[SFK_DT], kap = d.k[SFK_KAPPA];
+    const double aop = d.k[SFK_ALPHA_OVER_PI], gam = d.k[SFK_GAMMA], teq = d.k[SFK_TEQ], noise = d.k[SFK_NOISE];
+    double* ophi = a.out.f64 + d.cell_base;
+    double* oT = a.out.f64 + a.total_cells + d.cell_base;
+    // the update's long part without a branch, then the noise and the stores
+    struct Part { double ph, t, lt, br; };
+    for_cells<W * W, NT, Part>(
+        [&](int e, Part& out) {
+            const int y = e / W, by = B0 + y, bx = B0 + e - y * W;
+            int sy = by, sx = bx;
+            if (EDGE) {
+                sy = sf_mirror(by, oy, H, d.ny);
+                sx = sf_mirror(bx, ox, H, d.nx);
+            }
+            const int c = sy * W0 + sx, r = (sy - 1) * WR + sx - 1;
+            double lp, lt;
+            const double ph = F[c], t = G[c];
+            if (ref) {
+                const double sp = F[c - 1] + F[c - 2] + F[c + 1] + F[c + 2] + F[c - W0] + F[c - 2 * W0] + F[c + W0] + F[c + 2 * W0];
+                const double st = G[c - 1] + G[c - 2] + G[c + 1] + G[c + 2] + G[c - W0] + G[c - 2 * W0] + G[c + W0] + G[c + 2 * W0];
+                lp = (sp - 8.0 * ph) * inv;
+                lt = (st - 8.0 * t) * inv;
+            } else {
+                lp = (F[c - 1] + F[c + 1] + F[c - W0] + F[c + W0] - 4.0 * ph) * inv;
+                lt = (G[c - 1] + G[c + 1] + G[c - W0] + G[c + W0] - 4.0 * t) * inv;
+            }
+            const double term1 = (L.P[r + WR] - L.P[r - WR]) * inv2dy;
+            const double term2 = -(L.Q[r + 1] - L.Q[r - 1]) * inv2dx;
+            const double flux = term1 + term2 + L.E2[r] * lp;
+            const double m = aop * atan(gam * (teq - t));
+            const double pp = ph * (1.0 - ph);
+            out.br = flux + pp * (ph - 0.5 + m);
+            out.ph = ph;
+            out.t = t;
+            out.lt = lt;
+        },
+        [&](int e, const Part& v) {
+            const int y = e / W, x = e - y * W;
+            const double ph = v.ph, pp = ph * (1.0 - ph);
+            double br = v.br;
+            if (noise != 0.0 && fabs(pp) > 0.0) {
+                int gy = oy - HS + y, gx = ox - HS + x;
+                if (EDGE) {
+                    gy = sf_mirror(gy, 0, 0, d.ny);
+                    gx = sf_mirror(gx, 0, 0, d.nx);
+                }
+                // a wrapped halo cell draws the noise of the cell it stands for
+                gy = gy < 0 ? gy + d.ny : (gy >= d.ny ? gy - d.ny : gy);
+                gx = gx < 0 ? gx + d.nx : (gx >= d.nx ? gx - d.nx : gx);
+                const double u = (double)noise_u24(key, (uint32_t)(gy * d.nx + gx));
+                br = br + noise * ph * (1.0 - ph) * (u - 0.5);
+            }
+            const double phn = ph + dtt * br;
+            const double tn = sf_t_update<double>(v.t, v.lt, dt, kap, phn - ph);
+            if constexpr (S == K - 1) {  // the region is the block itself
+                const int g = (oy + y) * d.nx + ox + x;
+                ophi[g] = phn;
+                oT[g] = tn;
+            } else {
+                L.f[(S + 1) & 1][0][(B0 + y) * W0 + B0 + x] = phn;
+                L.f[(S + 1) & 1][1][(B0 + y) * W0 + B0 + x] = tn;
+            }
+        });
+    if constexpr (S + 1 < K) __syncthreads();
+}
+
+template <int BS, int K, int NT, bool EDGE>
+__device__ __forceinline__ void sf_multi_steps(SfMultiLds<BS, K>& L, const StepArgs& a, const InstDesc& d, int ox,
+                                               int oy, long long step) {
+    sf_multi_step<BS, K, 0, NT, EDGE>(L, a, d, ox, oy, noise_key(d.seed, (uint64_t)step));
+    if constexpr (K > 1) sf_multi_step<BS, K, 1, NT, EDGE>(L, a, d, ox, oy, noise_key(d.seed, (uint64_t)(step + 1)));
+    if constexpr (K > 2) sf_multi_step<BS, K, 2, NT, EDGE>(L, a, d, ox, oy, noise_key(d.seed, (uint64_t)(step + 2)));
+    if constexpr (K > 3) sf_multi_step<BS, K, 3, NT, EDGE>(L, a, d, ox, oy, noise_key(d.seed, (uint64_t)(step + 3)));
+}
+
+template <int BS, int K, int NT>
+__global__ __launch_bounds__(NT) void sf_multi_kernel(StepArgs a, const InstDesc* __restrict__ inst,
+                                                      const int* __restrict__ binst, const int* __restrict__ bbase) {
+    using M = SfMultiLds<BS, K>;
+    constexpr int H = 2 * K, W0 = M::W0, NL = (W0 * W0 + NT - 1) / NT;
+    __shared__ __align__(16) M L;
+    const long long step = *a.step_ctr + a.step_add;
+    const int b = xcd_remap(blockIdx.x, gridDim.x);
+    const int in = a.ninst > 1 ? binst[b] : 0;
+    const InstDesc& d = inst[in];
+    const int lb = a.ninst > 1 ? b - bbase[in] : b, nbx = d.nx / BS;
+    const int ty = lb / nbx, oy = ty * BS, ox = (lb - ty * nbx) * BS;
+    const bool per = d.bc == AMPS_BC_PERIODIC;
+    const double* fphi = a.in.f64 + d.cell_base;
+    const double* fT = a.in.f64 + a.total_cells + d.cell_base;
+    double vp[NL], vt[NL];
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+        const int e = min((int)threadIdx.x + k * NT, W0 * W0 - 1);
+        const int y = e / W0;
+        const int g = map_cell(oy - H + y, d.ny, per) * d.nx + map_cell(ox - H + e - y * W0, d.nx, per);
+        vp[k] = fphi[g];
+        vt[k] = fT[g];
+    }
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+        const int e = threadIdx.x + k * NT;
+        if (e < W0 * W0) {
+            L.f[0][0][e] = vp[k];
+            L.f[0][1][e] = vt[k];
+        }
+    }
+    __syncthreads();
+    const bool edge = !per && (ox == 0 || oy == 0 || ox + BS == d.nx || oy + BS == d.ny);
+    if (edge) sf_multi_steps<BS, K, NT, true>(L, a, d, ox, oy, step);
+    else sf_multi_steps<BS, K, NT, false>(L, a, d, ox, oy, step);
+}
+
 // ------------------------------------------------------------ host launch
 // Persistent grid of kernel K: resident workgroups per CU (occupancy query,
 // cached per kernel) x CUs, at most one workgroup per work item.
@@ -1652,6 +1856,20 @@ int launch_sf_step(const StepArgs& a, int tile, bool adaptive, hipStream_t s, co
         return AMPS_E_UNSUPPORTED;
     }
     return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;
+}
+
+int launch_sf_multi(const StepArgs& a, const BlockMap& bm, hipStream_t s) {
+#define SF_MULTI(E, K, NT)                                                                                  \
+    if (bm.edge == E && bm.k == K) {                                                                        \
+        hipLaunchKernelGGL((sf_multi_kernel<E, K, NT>), dim3(bm.nblocks), dim3(NT), 0, s, a, a.inst, bm.inst, bm.base); \
+        return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;                                      \
+    }
+    SF_MULTI(16, 4, 768)
+    SF_MULTI(16, 3, 512)
+    SF_MULTI(16, 2, 256)
+    SF_MULTI(32, 3, 1024)
+#undef SF_MULTI
+    return AMPS_E_UNSUPPORTED;
 }
 
 }  // namespace amps

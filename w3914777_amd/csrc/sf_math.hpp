@@ -81,11 +81,24 @@ __device__ inline void sf_unit_power6(R gx, R gy, R& c, R& s) {
     s = s2 * (R(3) * cc - ss);
 }
 
+// (cos 4 theta, sin 4 theta) by sf_unit_power's operations with the power a
+// constant and no branch on the gradient (a zero one is replaced by (1, 0)
+// and gives (1, 0)): the loops over the bits of n and the branch otherwise
+// keep the cells of a thread one after the other.
+template <typename R>
+__device__ inline void sf_unit_power4(R gx, R gy, R& c, R& s) {
+    const bool nz = fmax(fabs(gx), fabs(gy)) != R(0);
+    sf_unit_power<R>(nz ? gx : R(1), nz ? gy : R(0), 4, c, s);
+    c = nz ? c : R(1);
+    s = nz ? s : R(0);
+}
+
 template <typename R>
 __device__ inline void sf_aniso(R gx, R gy, int n, R cth0, R sth0, R epsb, R epsb_delta, R m_epsb_n_delta,
                                 R& eps, R& epsd) {
     R c, s;
     if (n == 6) sf_unit_power6<R>(gx, gy, c, s);  // the snowflake's six-fold case
+    else if (n == 4) sf_unit_power4<R>(gx, gy, c, s);  // the reference's
     else sf_unit_power<R>(gx, gy, n, c, s);
     R ca = c * cth0 + s * sth0;  // cos(n (theta - theta0))
     R sa = s * cth0 - c * sth0;  // sin(n (theta - theta0))
