@@ -70,3 +70,23 @@ def test_snowflake_steps_per_launch_bitwise(amps, ny, nx, tile, bc, stencil, ani
 def test_snowflake_batches_bitwise(amps, sides):
     cfgs = [sf(amps, ny, nx, 16, i % 2, (i + 1) % 2, (4, 6, 5)[i % 3], 0.01 * (i % 2)) for i, (ny, nx) in enumerate(sides)]
     check(amps, cfgs, 10, 3)
+
+
+def gg(amps, ny, nx, tile, bc, stencil, q):
+    c = amps.Config.default(amps.GRAINGROWTH)
+    c.nx, c.ny, c.tile, c.bc, c.stencil, c.q = nx, ny, tile, bc, stencil, q
+    return c
+
+
+# every (edge, K, q) of the plan: one block, up to 1.25 blocks of 16^2 per CU, sides that divide by 32 or not
+@pytest.mark.parametrize("ny,nx,tile", [(16, 16, 16), (96, 48, 16), (256, 320, 32), (272, 336, 16), (416, 256, 32),
+                                        (608, 512, 32), (752, 400, 16)])
+@pytest.mark.parametrize("q,bc,stencil", [(2, 0, 0), (2, 1, 1), (3, 1, 0), (4, 0, 1), (5, 1, 0), (6, 0, 0), (7, 1, 1)])
+def test_graingrowth_steps_per_launch_bitwise(amps, ny, nx, tile, q, bc, stencil):
+    check(amps, [gg(amps, ny, nx, tile, bc, stencil, q)], 17, 5)
+
+
+@pytest.mark.parametrize("q", [2, 4])
+def test_graingrowth_batches_bitwise(amps, q):
+    cfgs = [gg(amps, ny, nx, 16, i % 2, (i + 1) % 2, q) for i, (ny, nx) in enumerate(((16, 48), (320, 336), (64, 64)))]
+    check(amps, cfgs, 13, 9)

@@ -440,7 +440,7 @@ bool use_multi(const amps_ctx* c) { return c->bm.k > 1 && !c->taping && !c->ktim
 int enqueue_multi(amps_ctx* c) {
     StepArgs a = step_args(c, c->cur);
     a.step_add = c->pending_adv;
-    RCCHK(launch_sf_multi(a, c->bm, c->stream));
+    RCCHK(c->model == AMPS_SNOWFLAKE ? launch_sf_multi(a, c->bm, c->stream) : launch_gg_multi(a, c->bm, c->stream));
     c->pending_adv += c->bm.k;
     c->cur ^= 1;
     c->steps_done += c->bm.k;
@@ -482,7 +482,7 @@ long long block_count(const amps_ctx* c, int edge) {
     return n;
 }
 
-// Steps per launch of a PURE_FP64 snowflake context.
+// Steps per launch of a PURE_FP64 snowflake context on 16^2 or 32^2 blocks.
 //
 // A single step of a small grid is its launch and one tile's chain of
 // dependent operations (5 us from 64^2 to 256^2, 6.3 at 512^2), so K steps
@@ -496,18 +496,46 @@ long long block_count(const amps_ctx* c, int edge) {
 //   16^2 blocks, K = 2:  512^2 (1024) 4.6 (5.1); 640^2 (1600) 6.6 (7.0); 768^2 (2304) 8.1 : 9.7 (8.5 : 9.4)
 // Larger grids fill the chip with single steps and lose by the redundancy
 // (1024^2: 13.1 : 13.2 and 12.6 : 12.5; 2048^2: 43 : 36).
+void plan_sf(long long b16, long long b32, int cus, int& k, int& edge) {
+    if (b16 <= cus + cus / 4) k = 4;
+    else if (b32 > 0 && b32 <= cus && b16 > 2 * cus) { k = 3; edge = 32; }
+    else if (b16 <= 2 * cus + cus / 4) k = 3;
+    else if (b16 <= 9 * cus) k = 2;
+}
+
+// Steps per launch of a PURE_FP64 grain-growth context (q <= 6: the fields of
+// a block, in two generations, fit the LDS).  The update is short and the
+// reach one cell, so every grid gains: with few blocks per CU the launch and
+// the latency are shared, with many the traffic is.  us a step against the
+// single step's (256 CUs, tile 16):
+//   16^2, K = 8:  256^2 q = 2 1.1 : 4.2, q = 4 1.7 : 5.2 (384^2 q = 4 3.4; 16^2, K = 4 3.0; 32^2, K = 4 2.9 : 6.0)
+//   32^2, K = 6:  512^2 q = 2 1.8 : 5.4 (16^2, K = 4 2.4), 1024^2 4.9 : 12.6 (6.3), 3072^2 41 : 131 (53)
+//   32^2, K = 4:  512^2 q = 3 2.5 : 6.2 (3.0), q = 4 3.1 : 7.0 (3.7), q = 6 4.2 : 8.2 (5.4); 2048^2 q = 6 68 : 126 (73)
+//   16^2, K = 4:  768^2 q = 4 6.8 : 11.6 (32^2, K = 4 8.0), 3072^2 88 : 214 (101); 1024^2 q = 5 13.3 : 19.7 (13.1)
+// At q = 4 and 5 a 32^2 block leaves one workgroup per CU, which pays only
+// while there is about one block per CU.
+void plan_gg(int q, long long b16, long long b32, int cus, int& k, int& edge) {
+    if (q > 6) return;
+    if (b16 <= cus + cus / 4) {
+        k = q <= 4 ? 8 : 4;
+    } else if (b32 > 0 && (q <= 3 || q == 6 || b32 <= cus)) {
+        k = q == 2 ? 6 : 4;
+        edge = 32;
+    } else {
+        k = 4;
+    }
+}
+
 int plan_multi(amps_ctx* c) {
-    if (c->mode != AMPS_PURE_FP64 || c->model != AMPS_SNOWFLAKE) return AMPS_OK;
+    if (c->mode != AMPS_PURE_FP64 || c->model == AMPS_SINTERING) return AMPS_OK;
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
     const long long b16 = block_count(c, 16), b32 = block_count(c, 32);
     int k = 0, edge = 16;
-    if (b16 <= cus + cus / 4) k = 4;
-    else if (b32 > 0 && b32 <= cus && b16 > 2 * cus) { k = 3; edge = 32; }
-    else if (b16 <= 2 * cus + cus / 4) k = 3;
-    else if (b16 <= 9 * cus) k = 2;
+    if (c->model == AMPS_SNOWFLAKE) plan_sf(b16, b32, cus, k, edge);
+    else plan_gg(c->q, b16, b32, cus, k, edge);
     if (k == 0) return AMPS_OK;
     std::vector<int> inst, base;
     for (int i = 0; i < c->ninst; ++i) {

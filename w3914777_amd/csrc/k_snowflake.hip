@@ -1593,35 +1593,6 @@ struct SfMultiLds {
     double P[WR * WR], Q[WR * WR], E2[WR * WR];
 };
 
-// Box coordinate of the mirror image of box coordinate b (origin o of the
-// block, halo h) on a zero-flux axis of n cells.
-__device__ inline int sf_mirror(int b, int o, int h, int n) {
-    const int g = o - h + b;
-    return g < 0 ? b - 2 * g : (g >= n ? b + 2 * (n - 1 - g) : b);
-}
-
-// Calls compute(e, r) for the cells e = tid + k NT < N of a region, then
-// store(e, r): the full passes of a thread are computed side by side (their
-// chains of dependent operations overlap), the last, partial one after them.
-template <int N, int NT, typename R, typename C, typename W>
-__device__ inline void for_cells(C&& compute, W&& store) {
-    constexpr int FULL = N / NT;
-    if constexpr (FULL > 0) {
-        R r[FULL];
-#pragma unroll
-        for (int k = 0; k < FULL; ++k) compute((int)threadIdx.x + k * NT, r[k]);
-#pragma unroll
-        for (int k = 0; k < FULL; ++k) store((int)threadIdx.x + k * NT, r[k]);
-    }
-    if constexpr (N % NT != 0) {
-        if ((int)threadIdx.x + FULL * NT < N) {
-            R r;
-            compute((int)threadIdx.x + FULL * NT, r);
-            store((int)threadIdx.x + FULL * NT, r);
-        }
-    }
-}
-
 // Step S of K: ring intermediates on the region and one cell around it, then
 // the new phi and T of the region.
 template <int BS, int K, int S, int NT, bool EDGE>
@@ -1644,8 +1615,8 @@ __device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepAr
                 const int y = e / WP, by = B0 - 1 + y, bx = B0 - 1 + e - y * WP;
                 int sy = by, sx = bx;
                 if (EDGE) {
-                    sy = sf_mirror(by, oy, H, d.ny);
-                    sx = sf_mirror(bx, ox, H, d.nx);
+                    sy = mirror_box(by, oy, H, d.ny);
+                    sx = mirror_box(bx, ox, H, d.nx);
                 }
                 const int c = sy * W0 + sx;
                 const double gx = (F[c + 1] - F[c - 1]) * inv2dx;
@@ -1677,8 +1648,8 @@ __device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepAr
             const int y = e / W, by = B0 + y, bx = B0 + e - y * W;
             int sy = by, sx = bx;
             if (EDGE) {
-                sy = sf_mirror(by, oy, H, d.ny);
-                sx = sf_mirror(bx, ox, H, d.nx);
+                sy = mirror_box(by, oy, H, d.ny);
+                sx = mirror_box(bx, ox, H, d.nx);
             }
             const int c = sy * W0 + sx, r = (sy - 1) * WR + sx - 1;
             double lp, lt;
@@ -1709,8 +1680,8 @@ __device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepAr
             if (noise != 0.0 && fabs(pp) > 0.0) {
                 int gy = oy - HS + y, gx = ox - HS + x;
                 if (EDGE) {
-                    gy = sf_mirror(gy, 0, 0, d.ny);
-                    gx = sf_mirror(gx, 0, 0, d.nx);
+                    gy = mirror_box(gy, 0, 0, d.ny);
+                    gx = mirror_box(gx, 0, 0, d.nx);
                 }
                 // a wrapped halo cell draws the noise of the cell it stands for
                 gy = gy < 0 ? gy + d.ny : (gy >= d.ny ? gy - d.ny : gy);

@@ -225,6 +225,36 @@ __device__ inline void box_load_dev32(float* b0, const double* f64, const __half
     }
 }
 
+// ------------------------------------------------- multi-step FP64 blocks
+// Box coordinate of the mirror image of box coordinate b (origin o of the
+// block, halo h) on a zero-flux axis of n cells.
+__device__ inline int mirror_box(int b, int o, int h, int n) {
+    const int g = o - h + b;
+    return g < 0 ? b - 2 * g : (g >= n ? b + 2 * (n - 1 - g) : b);
+}
+
+// Calls compute(e, r) for the cells e = tid + k NT < N of a region, then
+// store(e, r): the full passes of a thread are computed side by side (their
+// chains of dependent operations overlap), the last, partial one after them.
+template <int N, int NT, typename R, typename C, typename W>
+__device__ inline void for_cells(C&& compute, W&& store) {
+    constexpr int FULL = N / NT;
+    if constexpr (FULL > 0) {
+        R r[FULL];
+#pragma unroll
+        for (int k = 0; k < FULL; ++k) compute((int)threadIdx.x + k * NT, r[k]);
+#pragma unroll
+        for (int k = 0; k < FULL; ++k) store((int)threadIdx.x + k * NT, r[k]);
+    }
+    if constexpr (N % NT != 0) {
+        if ((int)threadIdx.x + FULL * NT < N) {
+            R r;
+            compute((int)threadIdx.x + FULL * NT, r);
+            store((int)threadIdx.x + FULL * NT, r);
+        }
+    }
+}
+
 // 1/x to ~1 ulp: hardware reciprocal estimate refined by two Newton steps.
 __device__ inline double rcp_nr(double x) {
     double r = __builtin_amdgcn_rcp(x);
