@@ -90,3 +90,22 @@ def test_graingrowth_steps_per_launch_bitwise(amps, ny, nx, tile, q, bc, stencil
 def test_graingrowth_batches_bitwise(amps, q):
     cfgs = [gg(amps, ny, nx, 16, i % 2, (i + 1) % 2, q) for i, (ny, nx) in enumerate(((16, 48), (320, 336), (64, 64)))]
     check(amps, cfgs, 13, 9)
+
+
+def sn(amps, ny, nx, tile, bc, flags):
+    c = amps.Config.default(amps.SINTERING)
+    c.nx, c.ny, c.tile, c.bc, c.flags = nx, ny, tile, bc, flags
+    return c
+
+
+# one block, 16^2 blocks with K = 4 and K = 2, 32^2 blocks with K = 3 and K = 2
+@pytest.mark.parametrize("ny,nx,tile", [(16, 16, 16), (48, 96, 16), (256, 320, 32), (288, 384, 32), (400, 336, 16),
+                                        (800, 1056, 32)])
+@pytest.mark.parametrize("bc,flags", [(0, 0), (1, 0), (0, 2), (1, 2)])
+def test_sintering_steps_per_launch_bitwise(amps, ny, nx, tile, bc, flags):
+    check(amps, [sn(amps, ny, nx, tile, bc, flags)], 11, 6)
+
+
+def test_sintering_batch_bitwise(amps):
+    cfgs = [sn(amps, ny, nx, 16, i % 2, 0) for i, (ny, nx) in enumerate(((16, 48), (320, 336), (64, 64)))]
+    check(amps, cfgs, 9, 8)

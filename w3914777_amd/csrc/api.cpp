@@ -440,7 +440,9 @@ bool use_multi(const amps_ctx* c) { return c->bm.k > 1 && !c->taping && !c->ktim
 int enqueue_multi(amps_ctx* c) {
     StepArgs a = step_args(c, c->cur);
     a.step_add = c->pending_adv;
-    RCCHK(c->model == AMPS_SNOWFLAKE ? launch_sf_multi(a, c->bm, c->stream) : launch_gg_multi(a, c->bm, c->stream));
+    RCCHK(c->model == AMPS_SNOWFLAKE     ? launch_sf_multi(a, c->bm, c->stream)
+          : c->model == AMPS_GRAINGROWTH ? launch_gg_multi(a, c->bm, c->stream)
+                                         : launch_sn_multi(a, c->bm, c->stream));
     c->pending_adv += c->bm.k;
     c->cur ^= 1;
     c->steps_done += c->bm.k;
@@ -526,8 +528,26 @@ void plan_gg(int q, long long b16, long long b32, int cus, int& k, int& edge) {
     }
 }
 
+// Steps per launch of a PURE_FP64 sintering context.  us a step against the
+// single step's (256 CUs, tile 32, workload physics):
+//   16^2, K = 4:  64^2 to 256^2 1.8 : 7.5
+//   32^2, K = 3:  384^2 3.0 : 7.9 (16^2, K = 2 3.6); 512^2 3.1 : 8.2 (4.4); 768^2 7.5 : 10.5
+//   16^2, K = 2:  768^2 (2304 blocks) 6.9 : 10.5 (32^2, K = 2 7.4); 1024^2 10.8; 3072^2 82
+//   32^2, K = 2:  1024^2 (1024 blocks) 9.7 : 13.7; 2048^2 34.6 : 40; 3072^2 77 : 99
+void plan_sn(long long b16, long long b32, int cus, int& k, int& edge) {
+    k = 2;
+    if (b16 <= cus + cus / 4) {
+        k = 4;
+    } else if (b32 > 0 && b32 <= cus) {
+        k = 3;
+        edge = 32;
+    } else if (b32 > 3 * cus) {
+        edge = 32;
+    }
+}
+
 int plan_multi(amps_ctx* c) {
-    if (c->mode != AMPS_PURE_FP64 || c->model == AMPS_SINTERING) return AMPS_OK;
+    if (c->mode != AMPS_PURE_FP64) return AMPS_OK;
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
@@ -535,7 +555,8 @@ int plan_multi(amps_ctx* c) {
     const long long b16 = block_count(c, 16), b32 = block_count(c, 32);
     int k = 0, edge = 16;
     if (c->model == AMPS_SNOWFLAKE) plan_sf(b16, b32, cus, k, edge);
-    else plan_gg(c->q, b16, b32, cus, k, edge);
+    else if (c->model == AMPS_GRAINGROWTH) plan_gg(c->q, b16, b32, cus, k, edge);
+    else plan_sn(b16, b32, cus, k, edge);
     if (k == 0) return AMPS_OK;
     std::vector<int> inst, base;
     for (int i = 0; i < c->ninst; ++i) {

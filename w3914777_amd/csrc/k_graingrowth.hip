@@ -782,7 +782,7 @@ __device__ __forceinline__ void gg_multi_step(GgMultiLds<BS, K, Q>& L, const Ste
     struct New {
         double e[Q];
     };
-    for_cells<W * W, NT, New>(
+    for_cells<W * W, NT, false, New>(
         [&](int e, New& n) {
             const int y = e / W;
             int sy = B0 + y, sx = B0 + e - y * W;

@@ -1610,7 +1610,7 @@ __device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepAr
         const double epsb = d.k[SFK_EPSB], epsbd = d.k[SFK_EPSB_DELTA], mend = d.k[SFK_MEPSB_ANISO_DELTA];
         constexpr int WP = W + 2;
         struct Ring { double p, q, e2; };
-        for_cells<WP * WP, NT, Ring>(
+        for_cells<WP * WP, NT, false, Ring>(
             [&](int e, Ring& r) {
                 const int y = e / WP, by = B0 - 1 + y, bx = B0 - 1 + e - y * WP;
                 int sy = by, sx = bx;
@@ -1643,7 +1643,7 @@ __device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepAr
     double* oT = a.out.f64 + a.total_cells + d.cell_base;
     // the update's long part without a branch, then the noise and the stores
     struct Part { double ph, t, lt, br; };
-    for_cells<W * W, NT, Part>(
+    for_cells<W * W, NT, false, Part>(
         [&](int e, Part& out) {
             const int y = e / W, by = B0 + y, bx = B0 + e - y * W;
             int sy = by, sx = bx;

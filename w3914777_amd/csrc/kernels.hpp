@@ -47,6 +47,7 @@ int launch_sf_step(const StepArgs& a, int tile, bool adaptive, hipStream_t s, co
 // PURE_FP64: bm.k steps in one launch on the blocks of bm (a.in to a.out).
 int launch_sf_multi(const StepArgs& a, const BlockMap& bm, hipStream_t s);
 int launch_gg_multi(const StepArgs& a, const BlockMap& bm, hipStream_t s);
+int launch_sn_multi(const StepArgs& a, const BlockMap& bm, hipStream_t s);
 // same_flags[f][tile] = 0 and bit f of zmask[tile] cleared for every field f whose
 // type group changed type on the tile.
 int launch_clear_changed(const int* type_old, const int* type, const GroupMap& gm, int nfields, int total_tiles,

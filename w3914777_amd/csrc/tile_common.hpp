@@ -236,21 +236,32 @@ __device__ inline int mirror_box(int b, int o, int h, int n) {
 // Calls compute(e, r) for the cells e = tid + k NT < N of a region, then
 // store(e, r): the full passes of a thread are computed side by side (their
 // chains of dependent operations overlap), the last, partial one after them.
-template <int N, int NT, typename R, typename C, typename W>
-__device__ inline void for_cells(C&& compute, W&& store) {
+// SYNC: every store of the workgroup follows every compute (the stores
+// overwrite what the computes read).
+template <int N, int NT, bool SYNC, typename R, typename C, typename W>
+__device__ __forceinline__ void for_cells(C&& compute, W&& store) {
     constexpr int FULL = N / NT;
-    if constexpr (FULL > 0) {
-        R r[FULL];
+    constexpr bool PART = N % NT != 0;
+    R r[FULL > 0 ? FULL : 1], rp;
+    const int ep = (int)threadIdx.x + FULL * NT;
 #pragma unroll
-        for (int k = 0; k < FULL; ++k) compute((int)threadIdx.x + k * NT, r[k]);
+    for (int k = 0; k < FULL; ++k) compute((int)threadIdx.x + k * NT, r[k]);
+    if constexpr (!SYNC) {
 #pragma unroll
         for (int k = 0; k < FULL; ++k) store((int)threadIdx.x + k * NT, r[k]);
     }
-    if constexpr (N % NT != 0) {
-        if ((int)threadIdx.x + FULL * NT < N) {
-            R r;
-            compute((int)threadIdx.x + FULL * NT, r);
-            store((int)threadIdx.x + FULL * NT, r);
+    if constexpr (PART) {
+        if (ep < N) {
+            compute(ep, rp);
+            if constexpr (!SYNC) store(ep, rp);
+        }
+    }
+    if constexpr (SYNC) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < FULL; ++k) store((int)threadIdx.x + k * NT, r[k]);
+        if constexpr (PART) {
+            if (ep < N) store(ep, rp);
         }
     }
 }
