@@ -120,6 +120,9 @@ struct amps_ctx {
     bool taping = false;
     long long tape_step0 = 0;
     std::vector<double*> tape;              // device checkpoints (all fields)
+    std::vector<void*> tape_blocks;         // their allocations: 1, 2, 4, ... checkpoints each
+    double* tape_free = nullptr;            // free part of the last one
+    size_t tape_free_n = 0;                 // checkpoints that fit in it
     std::vector<long long> tape_steps;
 
     // sweep-kernel timing (events around each step-kernel launch)
@@ -131,21 +134,43 @@ struct amps_ctx {
     double kms = 0.0;                      // all sweep kernels
     double kms_part[2] = {0.0, 0.0};       // snowflake adaptive: FP64 sweep, low sweep
 
-    std::vector<void*> allocs;
+    void* memory = nullptr;                 // every device buffer above
 };
 
 int tape_push(amps_ctx* c);
 
 namespace {
 
-int dmalloc(amps_ctx* c, void** p, size_t bytes) {
-    if (bytes == 0) bytes = 8;
-    hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess) return fail(AMPS_E_NOMEM, "hipMalloc(" + std::to_string(bytes) + "): " + hipGetErrorString(e));
-    c->allocs.push_back(*p);
-    HIPCHK(hipMemset(*p, 0, bytes));
-    return AMPS_OK;
-}
+// Device memory of a context: the buffers are asked for one by one and come
+// from one zeroed allocation (an allocation costs 30 us to make and 250 us to
+// free, whatever its size).
+struct DeviceArena {
+    struct Ask {
+        void** p;
+        size_t bytes;
+    };
+    std::vector<Ask> asks;
+    template <typename T>
+    void ask(T** p, size_t bytes) {
+        asks.push_back({reinterpret_cast<void**>(p), (std::max<size_t>(bytes, 8) + 255) & ~(size_t)255});
+    }
+    int get(amps_ctx* c) {
+        size_t total = 0;
+        for (const Ask& k : asks) total += k.bytes;
+        void* base = nullptr;
+        const hipError_t e = hipMalloc(&base, total);
+        if (e != hipSuccess)
+            return fail(AMPS_E_NOMEM, "hipMalloc(" + std::to_string(total) + "): " + hipGetErrorString(e));
+        c->memory = base;
+        HIPCHK(hipMemset(base, 0, total));
+        char* at = static_cast<char*>(base);
+        for (const Ask& k : asks) {
+            *k.p = at;
+            at += k.bytes;
+        }
+        return AMPS_OK;
+    }
+};
 
 bool finite_params(const amps_config& c) {
     for (int i = 0; i < AMPS_NPARAMS; ++i)
@@ -546,8 +571,10 @@ void plan_sn(long long b16, long long b32, int cus, int& k, int& edge) {
     }
 }
 
-int plan_multi(amps_ctx* c) {
-    if (c->mode != AMPS_PURE_FP64) return AMPS_OK;
+// Chooses a PURE_FP64 context's steps per launch and blocks (bm.k = 0: single
+// steps only); inst and base receive the block map's tables.
+void plan_multi(amps_ctx* c, std::vector<int>& inst, std::vector<int>& base) {
+    if (c->mode != AMPS_PURE_FP64) return;
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
@@ -557,37 +584,46 @@ int plan_multi(amps_ctx* c) {
     if (c->model == AMPS_SNOWFLAKE) plan_sf(b16, b32, cus, k, edge);
     else if (c->model == AMPS_GRAINGROWTH) plan_gg(c->q, b16, b32, cus, k, edge);
     else plan_sn(b16, b32, cus, k, edge);
-    if (k == 0) return AMPS_OK;
-    std::vector<int> inst, base;
+    if (k == 0) return;
     for (int i = 0; i < c->ninst; ++i) {
         base.push_back((int)inst.size());
         inst.insert(inst.end(), (size_t)(c->desc[i].nx / edge) * (c->desc[i].ny / edge), i);
     }
-    RCCHK(dmalloc(c, (void**)&c->d_blk_inst, inst.size() * sizeof(int)));
-    RCCHK(dmalloc(c, (void**)&c->d_blk_base, base.size() * sizeof(int)));
-    HIPCHK(hipMemcpy(c->d_blk_inst, inst.data(), inst.size() * sizeof(int), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->d_blk_base, base.data(), base.size() * sizeof(int), hipMemcpyHostToDevice));
-    c->bm = BlockMap{k, edge, (int)inst.size(), c->d_blk_inst, c->d_blk_base};
-    return AMPS_OK;
+    c->bm = BlockMap{k, edge, (int)inst.size(), nullptr, nullptr};
 }
 }  // namespace
 
 // ============================================================ tape helpers
 int tape_push(amps_ctx* c) {
-    const size_t bytes = (size_t)c->nfields * c->total_cells * sizeof(double);
-    double* p = nullptr;
-    hipError_t e = hipMalloc((void**)&p, bytes);
-    if (e != hipSuccess) return fail(AMPS_E_NOMEM, "checkpoint allocation failed");
-    e = hipMemcpyAsync(p, c->buf[c->cur].f64, bytes, hipMemcpyDeviceToDevice, c->stream);
-    if (e != hipSuccess) { (void)hipFree(p); return fail(AMPS_E_HIP, "checkpoint copy failed"); }
-    c->tape.push_back(p);
+    const size_t words = (size_t)c->nfields * c->total_cells, bytes = words * sizeof(double);
+    if (c->tape_free_n == 0) {
+        // room for as many checkpoints as there are (up to 1 GiB), or for one
+        size_t n = std::max<size_t>(1, std::min(c->tape.size(), ((size_t)1 << 30) / bytes));
+        void* p = nullptr;
+        if (hipMalloc(&p, n * bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            n = 1;
+            if (hipMalloc(&p, bytes) != hipSuccess) return fail(AMPS_E_NOMEM, "checkpoint allocation failed");
+        }
+        c->tape_blocks.push_back(p);
+        c->tape_free = static_cast<double*>(p);
+        c->tape_free_n = n;
+    }
+    if (hipMemcpyAsync(c->tape_free, c->buf[c->cur].f64, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
+        return fail(AMPS_E_HIP, "checkpoint copy failed");
+    c->tape.push_back(c->tape_free);
     c->tape_steps.push_back(c->steps_done);
+    c->tape_free += words;
+    c->tape_free_n--;
     return AMPS_OK;
 }
 
 namespace {
 void tape_clear(amps_ctx* c) {
-    for (double* p : c->tape) (void)hipFree(p);
+    for (void* p : c->tape_blocks) (void)hipFree(p);
+    c->tape_blocks.clear();
+    c->tape_free = nullptr;
+    c->tape_free_n = 0;
     c->tape.clear();
     c->tape_steps.clear();
     c->taping = false;
@@ -724,44 +760,58 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     c->total_tiles = tiles;
 
     int rc = AMPS_OK;
-    auto A = [&](void** p, size_t bytes) { if (rc == AMPS_OK) rc = dmalloc(c, p, bytes); };
+    DeviceArena mem;
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e != hipSuccess) { delete c; return fail(AMPS_E_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e)); }
     if (hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
         amps_destroy(c);
         return fail(AMPS_E_HIP, "hipEventCreate failed");
     }
-    A((void**)&c->d_desc, sizeof(InstDesc) * n);
-    A((void**)&c->d_tile_inst, sizeof(int) * tiles);
+    mem.ask(&c->d_desc, sizeof(InstDesc) * n);
+    mem.ask(&c->d_tile_inst, sizeof(int) * tiles);
     const size_t nf = (size_t)c->nfields;
     for (int b = 0; b < 2; ++b) {
-        A((void**)&c->buf[b].f64, nf * cells * sizeof(double));
+        mem.ask(&c->buf[b].f64, nf * cells * sizeof(double));
         if (has_low(c)) {
-            A((void**)&c->buf[b].f16, nf * cells * sizeof(__half));
-            A((void**)&c->buf[b].off, nf * tiles * sizeof(double));
-            A((void**)&c->buf[b].scl, nf * tiles * sizeof(float));
-            if (c->model == AMPS_GRAINGROWTH) A((void**)&c->buf[b].zmask, tiles * sizeof(unsigned long long));
+            mem.ask(&c->buf[b].f16, nf * cells * sizeof(__half));
+            mem.ask(&c->buf[b].off, nf * tiles * sizeof(double));
+            mem.ask(&c->buf[b].scl, nf * tiles * sizeof(float));
+            if (c->model == AMPS_GRAINGROWTH) mem.ask(&c->buf[b].zmask, tiles * sizeof(unsigned long long));
         }
-        if (c->model == AMPS_GRAINGROWTH) A((void**)&c->d_aux[b], cells * sizeof(double));
+        if (c->model == AMPS_GRAINGROWTH) mem.ask(&c->d_aux[b], cells * sizeof(double));
     }
     const size_t gt = (size_t)c->ngroups * tiles;
-    A((void**)&c->d_type, gt * sizeof(int));
-    A((void**)&c->d_type_old, gt * sizeof(int));
-    A((void**)&c->d_md, gt * sizeof(double));
-    if (c->mode == AMPS_ADAPTIVE && c->monitor == AMPS_MON_TEMPORAL) A((void**)&c->d_last, gt * 16 * sizeof(double));
-    A((void**)&c->d_stats, 8 * sizeof(unsigned long long));
-    A((void**)&c->d_step, sizeof(long long));
-    A((void**)&c->d_scratch, (size_t)c->max_inst_cells * sizeof(double));
-    A((void**)&c->d_wl, 2 * (size_t)tiles * sizeof(int));
-    A((void**)&c->d_wl_count, 2 * sizeof(int));
+    mem.ask(&c->d_type, gt * sizeof(int));
+    mem.ask(&c->d_type_old, gt * sizeof(int));
+    mem.ask(&c->d_md, gt * sizeof(double));
+    if (c->mode == AMPS_ADAPTIVE && c->monitor == AMPS_MON_TEMPORAL) mem.ask(&c->d_last, gt * 16 * sizeof(double));
+    mem.ask(&c->d_stats, 8 * sizeof(unsigned long long));
+    mem.ask(&c->d_step, sizeof(long long));
+    mem.ask(&c->d_scratch, (size_t)c->max_inst_cells * sizeof(double));
+    mem.ask(&c->d_wl, 2 * (size_t)tiles * sizeof(int));
+    mem.ask(&c->d_wl_count, 2 * sizeof(int));
     c->same_flags_n = (size_t)(c->model == AMPS_GRAINGROWTH ? c->q : 1) * tiles;
-    A((void**)&c->d_same_flags, c->same_flags_n * sizeof(int));
+    mem.ask(&c->d_same_flags, c->same_flags_n * sizeof(int));
     c->full_cap = (tiles + 7) / 8;
-    A((void**)&c->d_full_seg, std::max(8 * (size_t)c->full_cap, (size_t)NSK_SEGS * nsk_cap(tiles)) * sizeof(int));
-    A((void**)&c->d_full_cnt, FULL_CNT_INTS * sizeof(int));
+    mem.ask(&c->d_full_seg, std::max(8 * (size_t)c->full_cap, (size_t)NSK_SEGS * nsk_cap(tiles)) * sizeof(int));
+    mem.ask(&c->d_full_cnt, FULL_CNT_INTS * sizeof(int));
+    std::vector<int> blk_inst, blk_base;
+    plan_multi(c, blk_inst, blk_base);
+    if (c->bm.k > 0) {
+        mem.ask(&c->d_blk_inst, blk_inst.size() * sizeof(int));
+        mem.ask(&c->d_blk_base, blk_base.size() * sizeof(int));
+    }
+    rc = mem.get(c);
     if (rc != AMPS_OK) { std::string m = g_last_error; amps_destroy(c); return fail(rc, m); }
     e = hipMemcpy(c->d_desc, c->desc.data(), sizeof(InstDesc) * n, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->d_tile_inst, c->tile_inst.data(), sizeof(int) * tiles, hipMemcpyHostToDevice);
+    if (e == hipSuccess && c->bm.k > 0) {
+        e = hipMemcpy(c->d_blk_inst, blk_inst.data(), blk_inst.size() * sizeof(int), hipMemcpyHostToDevice);
+        if (e == hipSuccess)
+            e = hipMemcpy(c->d_blk_base, blk_base.data(), blk_base.size() * sizeof(int), hipMemcpyHostToDevice);
+        c->bm.inst = c->d_blk_inst;
+        c->bm.base = c->d_blk_base;
+    }
     if (e != hipSuccess) { amps_destroy(c); return fail(AMPS_E_HIP, std::string("upload: ") + hipGetErrorString(e)); }
     const char* ng = std::getenv("AMPS_NO_GRAPH");
     c->use_graph = !(ng && ng[0] == '1');
@@ -773,8 +823,6 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
         c->grid_cap = cfgs[0].wg_per_cu * cus;
     }
     c->graph_period = c->mode == AMPS_ADAPTIVE ? (c->every % 2 ? 2 * c->every : c->every) : 10;
-    rc = plan_multi(c);
-    if (rc != AMPS_OK) { std::string m = g_last_error; amps_destroy(c); return fail(rc, m); }
     *out = c;
     return AMPS_OK;
 }
@@ -788,7 +836,7 @@ void amps_destroy(amps_ctx* c) {
     for (hipEvent_t e : c->kev) (void)hipEventDestroy(e);
     for (int p = 0; p < 2; ++p)
         if (c->gexec[p]) (void)hipGraphExecDestroy(c->gexec[p]);
-    for (void* p : c->allocs) (void)hipFree(p);
+    if (c->memory) (void)hipFree(c->memory);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1100,17 +1148,12 @@ int grad_slot(int model, int id) {
     return -1;
 }
 
-// Device allocations of one adjoint call, released on every exit path.
+// Device memory of one adjoint call, one allocation (see DeviceArena),
+// released on every exit path.
 struct AdjMem {
-    std::vector<void*> p;
+    void* p = nullptr;
     ~AdjMem() {
-        for (void* q : p) (void)hipFree(q);
-    }
-    int get(void** out, size_t bytes) {
-        *out = nullptr;
-        if (hipMalloc(out, bytes) != hipSuccess) return fail(AMPS_E_NOMEM, "adjoint work memory");
-        p.push_back(*out);
-        return AMPS_OK;
+        if (p) (void)hipFree(p);
     }
 };
 }  // namespace
@@ -1130,17 +1173,19 @@ extern "C" int amps_adjoint(amps_ctx* c, const double* dJ_du, const int32_t* par
     const int NG = 6;
     const int F = c->nfields;
     const size_t TC = (size_t)c->total_cells, state = (size_t)F * TC;
-    const int k_every = c->tape_every;
+    // states of a segment between its checkpoint and the next one, which ends
+    // it (the last segment ends at the context's own state)
+    const int nseg = (int)c->tape.size();
+    const auto seg_end = [&](int s) { return s + 1 < nseg ? c->tape_steps[s + 1] : c->steps_done; };
+    long long mmax = 1;
+    for (int s = 0; s < nseg; ++s) mmax = std::max(mmax, seg_end(s) - c->tape_steps[s]);
     AdjMem mem;
-    double* lam[2];
-    double* gacc;
-    long long* dstep;
-    std::vector<double*> seg(k_every + 1);
-    RCCHK(mem.get((void**)&lam[0], state * 8));
-    RCCHK(mem.get((void**)&lam[1], state * 8));
-    RCCHK(mem.get((void**)&gacc, (size_t)NG * c->total_tiles * 8));
-    RCCHK(mem.get((void**)&dstep, 8));
-    for (int j = 1; j <= k_every; ++j) RCCHK(mem.get((void**)&seg[j], state * 8));
+    const size_t words = 2 * state + (size_t)NG * c->total_tiles + 1 + (size_t)(mmax - 1) * state;
+    if (hipMalloc(&mem.p, words * 8) != hipSuccess) return fail(AMPS_E_NOMEM, "adjoint work memory");
+    double* lam[2] = {static_cast<double*>(mem.p), static_cast<double*>(mem.p) + state};
+    double* mid = lam[1] + state;  // [mmax - 1] states
+    double* gacc = mid + (size_t)(mmax - 1) * state;
+    long long* dstep = reinterpret_cast<long long*>(gacc + (size_t)NG * c->total_tiles);
     // cotangent of the final state: host [inst][field][ny][nx] -> device [field][cells]
     size_t hoff = 0;
     for (int i = 0; i < c->ninst; ++i) {
@@ -1152,18 +1197,20 @@ extern "C" int amps_adjoint(amps_ctx* c, const double* dJ_du, const int32_t* par
     }
     HIPCHK(hipMemsetAsync(gacc, 0, (size_t)NG * c->total_tiles * 8, c->stream));
     int cur = 0;
-    for (int s = (int)c->tape.size() - 1; s >= 0; --s) {
+    for (int s = nseg - 1; s >= 0; --s) {
         const long long S0 = c->tape_steps[s];
-        const long long S1 = s + 1 < (int)c->tape.size() ? c->tape_steps[s + 1] : c->steps_done;
-        const int m = (int)(S1 - S0);
+        const int m = (int)(seg_end(s) - S0);
         if (m <= 0) continue;
-        // recompute the segment's states from its checkpoint
-        seg[0] = c->tape[s];
+        const auto at = [&](int j) -> double* {  // state j of the segment
+            return j == 0 ? c->tape[s]
+                          : (j < m ? mid + (size_t)(j - 1) * state : (s + 1 < nseg ? c->tape[s + 1] : c->buf[c->cur].f64));
+        };
+        // recompute the segment's inner states from its checkpoint
         RCCHK(launch_fill_u64((unsigned long long*)dstep, 1, (unsigned long long)S0, c->stream));
-        for (int j = 0; j < m; ++j) {
+        for (int j = 0; j + 1 < m; ++j) {
             StepArgs a = step_args(c, 0);
-            a.in.f64 = seg[j];
-            a.out.f64 = seg[j + 1];
+            a.in.f64 = at(j);
+            a.out.f64 = at(j + 1);
             a.step_ctr = dstep;
             a.step_add = j;
             RCCHK(launch_step_kernel(c, a));
@@ -1174,8 +1221,8 @@ extern "C" int amps_adjoint(amps_ctx* c, const double* dJ_du, const int32_t* par
             a.tile_inst = c->d_tile_inst;
             a.total_tiles = c->total_tiles;
             a.total_cells = c->total_cells;
-            a.u = seg[j];
-            a.un = seg[j + 1];
+            a.u = at(j);
+            a.un = at(j + 1);
             a.lam_n = lam[cur];
             a.lam = lam[cur ^ 1];
             a.gacc = gacc;
