@@ -441,6 +441,39 @@ bool monitor_due(const amps_ctx* c, long long step) {
     return c->mode == AMPS_ADAPTIVE && step % c->every == 0;
 }
 
+// Steps amps_step may take in one launch now (0: single steps): nothing may
+// look at the state, or time a sweep, between them, so a launch ends at a
+// checkpoint of the tape at the latest.
+int multi_steps(const amps_ctx* c, int left) {
+    if (c->bm.k < 2 || c->ktiming) return 0;
+    if (c->taping) left = (int)std::min<long long>(left, c->tape_every - (c->steps_done - c->tape_step0) % c->tape_every);
+    return left >= c->bm.k ? c->bm.k : 0;
+}
+
+int launch_multi(const amps_ctx* c, const StepArgs& a) {
+    if (c->model == AMPS_SNOWFLAKE) return launch_sf_multi(a, c->bm, c->stream);
+    if (c->model == AMPS_GRAINGROWTH) return launch_gg_multi(a, c->bm, c->stream);
+    return launch_sn_multi(a, c->bm, c->stream);
+}
+
+// Push a checkpoint of the tape if the step count has reached one.
+int tape_due(amps_ctx* c) {
+    if (!c->taping || c->tape_every <= 0 || (c->steps_done - c->tape_step0) % c->tape_every != 0) return AMPS_OK;
+    RCCHK(flush_adv(c));
+    return tape_push(c);
+}
+
+// One launch of bm.k steps (PURE_FP64).
+int enqueue_multi(amps_ctx* c) {
+    StepArgs a = step_args(c, c->cur);
+    a.step_add = c->pending_adv;
+    RCCHK(launch_multi(c, a));
+    c->pending_adv += c->bm.k;
+    c->cur ^= 1;
+    c->steps_done += c->bm.k;
+    return tape_due(c);
+}
+
 int enqueue_one(amps_ctx* c) {
     if (monitor_due(c, c->steps_done)) {
         RCCHK(enqueue_monitor(c, c->cur));
@@ -450,28 +483,7 @@ int enqueue_one(amps_ctx* c) {
     c->pending_adv++;
     c->cur ^= 1;
     c->steps_done++;
-    if (c->taping && c->tape_every > 0 && (c->steps_done - c->tape_step0) % c->tape_every == 0) {
-        RCCHK(flush_adv(c));
-        RCCHK(tape_push(c));
-    }
-    return AMPS_OK;
-}
-
-// Whether amps_step may advance several steps a launch: nothing then looks at
-// the state, or times a sweep, between them.
-bool use_multi(const amps_ctx* c) { return c->bm.k > 1 && !c->taping && !c->ktiming; }
-
-// One launch of bm.k steps (PURE_FP64).
-int enqueue_multi(amps_ctx* c) {
-    StepArgs a = step_args(c, c->cur);
-    a.step_add = c->pending_adv;
-    RCCHK(c->model == AMPS_SNOWFLAKE     ? launch_sf_multi(a, c->bm, c->stream)
-          : c->model == AMPS_GRAINGROWTH ? launch_gg_multi(a, c->bm, c->stream)
-                                         : launch_sn_multi(a, c->bm, c->stream));
-    c->pending_adv += c->bm.k;
-    c->cur ^= 1;
-    c->steps_done += c->bm.k;
-    return AMPS_OK;
+    return tape_due(c);
 }
 
 // Capture `period` steps (monitor pass included) starting from buffer parity p.
@@ -895,11 +907,11 @@ int amps_step(amps_ctx* c, int nsteps) {
     const bool graphs = c->use_graph && !c->taping && !c->ktiming;
     while (left > 0) {
         const long long s = c->steps_done;
-        if (use_multi(c) && left >= c->bm.k) {
+        if (const int k = multi_steps(c, left)) {
             // not captured: a launch runs longer than its enqueue takes, and a
             // graph of these adds a gap of its own per replay
             RCCHK(enqueue_multi(c));
-            left -= c->bm.k;
+            left -= k;
         } else if (graphs && left >= c->graph_period && s % c->graph_period == 0) {
             RCCHK(flush_adv(c));
             if (!c->gexec[c->cur]) RCCHK(build_graph(c, c->cur));
@@ -1207,13 +1219,20 @@ extern "C" int amps_adjoint(amps_ctx* c, const double* dJ_du, const int32_t* par
         };
         // recompute the segment's inner states from its checkpoint
         RCCHK(launch_fill_u64((unsigned long long*)dstep, 1, (unsigned long long)S0, c->stream));
-        for (int j = 0; j + 1 < m; ++j) {
+        for (int j = 0; j + 1 < m;) {
             StepArgs a = step_args(c, 0);
             a.in.f64 = at(j);
             a.out.f64 = at(j + 1);
             a.step_ctr = dstep;
             a.step_add = j;
-            RCCHK(launch_step_kernel(c, a));
+            if (c->bm.k > 1 && j + c->bm.k < m) {  // bm.k states in a row of `mid`
+                a.step_stride = state;
+                RCCHK(launch_multi(c, a));
+                j += c->bm.k;
+            } else {
+                RCCHK(launch_step_kernel(c, a));
+                ++j;
+            }
         }
         for (int j = m - 1; j >= 0; --j) {
             AdjArgs a{};

@@ -483,12 +483,13 @@ __device__ __forceinline__ void sn_multi_step(SnMultiLds<BS, K, CONS, INPLACE>& 
         },
         [&](int e, const New& n) {
             const int y = e / W, x = e - y * W;
-            if constexpr (S == K - 1) {  // the region is the block itself
-                double* o = a.out.f64 + d.cell_base + (size_t)(oy + y) * d.nx + ox + x;
+            if (S == K - 1 || (a.step_stride && (unsigned)(y - HS) < (unsigned)BS && (unsigned)(x - HS) < (unsigned)BS)) {
+                double* o = a.out.f64 + S * a.step_stride + d.cell_base + (size_t)(oy - HS + y) * d.nx + ox - HS + x;
                 o[0] = n.c;
                 o[a.total_cells] = n.e1;
                 o[2 * a.total_cells] = n.e2;
-            } else {
+            }
+            if constexpr (S < K - 1) {
                 const int o = (B0 + y) * W0 + B0 + x;
                 L.f[GN][0][o] = n.c;
                 L.f[GN][1][o] = n.e1;

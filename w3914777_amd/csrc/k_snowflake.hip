@@ -1639,8 +1639,8 @@ __device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepAr
     const bool ref = d.stencil == AMPS_STENCIL_REF;
     const double inv = d.k[SFK_INV_DXDY], dtt = d.k[SFK_DT_OVER_TAU], dt = d.k[SFK_DT], kap = d.k[SFK_KAPPA];
     const double aop = d.k[SFK_ALPHA_OVER_PI], gam = d.k[SFK_GAMMA], teq = d.k[SFK_TEQ], noise = d.k[SFK_NOISE];
-    double* ophi = a.out.f64 + d.cell_base;
-    double* oT = a.out.f64 + a.total_cells + d.cell_base;
+    double* ophi = a.out.f64 + S * a.step_stride + d.cell_base;
+    double* oT = ophi + a.total_cells;
     // the update's long part without a branch, then the noise and the stores
     struct Part { double ph, t, lt, br; };
     for_cells<W * W, NT, false, Part>(
@@ -1691,11 +1691,12 @@ __device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepAr
             }
             const double phn = ph + dtt * br;
             const double tn = sf_t_update<double>(v.t, v.lt, dt, kap, phn - ph);
-            if constexpr (S == K - 1) {  // the region is the block itself
-                const int g = (oy + y) * d.nx + ox + x;
+            if (S == K - 1 || (a.step_stride && (unsigned)(y - HS) < (unsigned)BS && (unsigned)(x - HS) < (unsigned)BS)) {
+                const int g = (oy - HS + y) * d.nx + ox - HS + x;
                 ophi[g] = phn;
                 oT[g] = tn;
-            } else {
+            }
+            if constexpr (S < K - 1) {
                 L.f[(S + 1) & 1][0][(B0 + y) * W0 + B0 + x] = phn;
                 L.f[(S + 1) & 1][1][(B0 + y) * W0 + B0 + x] = tn;
             }
