@@ -87,7 +87,9 @@ struct amps_ctx {
                                             // [2], [3], [4] snowflake sweep tile counts (summed)
     long long* d_step = nullptr;
     double* d_aux[2] = {nullptr, nullptr};
-    double* d_scratch = nullptr;           // max instance cells (get/set)
+    double* d_scratch = nullptr;           // max instance cells (decoded field of amps_get_field)
+    int* bad = nullptr;                    // host word the read-back kernels set on a non-finite value
+    int* d_bad = nullptr;                  // its device address
     int* d_wl = nullptr;                   // [2][total_tiles]: FP64 and low tile work-lists
     int* d_wl_count = nullptr;             // [2]
     int* d_same_flags = nullptr;           // snowflake [total_tiles], grain growth [q][total_tiles]:
@@ -799,7 +801,7 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     if (c->mode == AMPS_ADAPTIVE && c->monitor == AMPS_MON_TEMPORAL) mem.ask(&c->d_last, gt * 16 * sizeof(double));
     mem.ask(&c->d_stats, 8 * sizeof(unsigned long long));
     mem.ask(&c->d_step, sizeof(long long));
-    mem.ask(&c->d_scratch, (size_t)c->max_inst_cells * sizeof(double));
+    if (has_low(c)) mem.ask(&c->d_scratch, (size_t)c->max_inst_cells * sizeof(double));
     mem.ask(&c->d_wl, 2 * (size_t)tiles * sizeof(int));
     mem.ask(&c->d_wl_count, 2 * sizeof(int));
     c->same_flags_n = (size_t)(c->model == AMPS_GRAINGROWTH ? c->q : 1) * tiles;
@@ -849,6 +851,7 @@ void amps_destroy(amps_ctx* c) {
     for (int p = 0; p < 2; ++p)
         if (c->gexec[p]) (void)hipGraphExecDestroy(c->gexec[p]);
     if (c->memory) (void)hipFree(c->memory);
+    if (c->bad) (void)hipHostFree(c->bad);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -957,13 +960,23 @@ int amps_get_field(amps_ctx* c, int inst, int field, double* dst, size_t n) {
     if (inst < 0 || inst >= c->ninst || field < 0 || field >= c->nfields) return fail(AMPS_E_ARG, "instance or field out of range");
     const InstDesc& d = c->desc[inst];
     if (n != (size_t)d.nx * d.ny) return fail(AMPS_E_ARG, "n must equal nx*ny of the instance");
+    if (!c->bad) {
+        HIPCHK(hipHostMalloc((void**)&c->bad, sizeof(int), hipHostMallocMapped));
+        HIPCHK(hipHostGetDevicePointer((void**)&c->d_bad, c->bad, 0));
+    }
+    *c->bad = 0;  // set by the device if a value is not finite
     const int group = has_low(c) ? c->gm.fg[field] : -1;
-    RCCHK(launch_gather(c->d_desc, c->buf[c->cur], c->total_cells, c->total_tiles, has_low(c) ? c->d_type : nullptr,
-                        group, inst, d.tx * d.ty, field, c->d_scratch, c->tile, c->stream));
-    HIPCHK(hipMemcpyAsync(dst, c->d_scratch, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    const double* src = c->d_scratch;
+    if (group >= 0) {
+        RCCHK(launch_gather(c->d_desc, c->buf[c->cur], c->total_cells, c->total_tiles, c->d_type, group, inst,
+                            d.tx * d.ty, field, c->d_scratch, c->d_bad, c->tile, c->stream));
+    } else {
+        src = c->buf[c->cur].f64 + (size_t)field * c->total_cells + d.cell_base;
+        RCCHK(launch_nonfinite(src, (long long)n, c->d_bad, c->stream));
+    }
+    HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    for (size_t i = 0; i < n; ++i)
-        if (!std::isfinite(dst[i])) return fail(AMPS_E_NONFINITE, "field " + std::to_string(field) + " holds non-finite values");
+    if (*(volatile int*)c->bad) return fail(AMPS_E_NONFINITE, "field " + std::to_string(field) + " holds non-finite values");
     return AMPS_OK;
 }
 

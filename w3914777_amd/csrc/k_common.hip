@@ -697,36 +697,43 @@ __global__ __launch_bounds__(1024) void worklist_kernel(const int* __restrict__ 
 }
 
 // Decode every low tile of field f into a dense FP64 array (instance order),
-// for amps_get_field.  FP64 tiles are copied.
+// for amps_get_field.  FP64 tiles are copied.  *bad (host memory the device
+// can write) becomes 1 if a value is not finite: the host then need not read
+// the field once more after the copy.
 template <int TS>
 __global__ __launch_bounds__(256) void gather_kernel(const InstDesc* inst, Buf b, long long total_cells,
                                                      int total_tiles, const int* type, int group, int instid,
-                                                     int field, double* dst) {
+                                                     int field, double* dst, int* bad) {
+    constexpr int PER = TS * TS / WG;
     const InstDesc& d = inst[instid];
     const int ntile = d.tx * d.ty;
+    bool ok = true;
     for (int lt = blockIdx.x; lt < ntile; lt += gridDim.x) {
         const int gtile = d.tile_base + lt;
-        const int ty = (type && group >= 0) ? type[(size_t)group * total_tiles + gtile] : 2;
+        const int ty = type[(size_t)group * total_tiles + gtile];
         const int tyi = lt / d.tx, txi = lt - tyi * d.tx;
-        if (ty == 1) {
-            decode_tile<TS>(b, total_cells, total_tiles, d, gtile, field, dst);
-        } else {
-            const double* src = b.f64 + (size_t)field * total_cells + d.cell_base;
-            for (int e = threadIdx.x; e < TS * TS; e += WG) {
-                int ly = e / TS, lx = e - ly * TS;
-                size_t c = (size_t)(tyi * TS + ly) * d.nx + txi * TS + lx;
-                dst[c] = src[c];
-            }
+        const double* src = b.f64 + (size_t)field * total_cells + d.cell_base;
+        const __half* f16 = b.f16 + (size_t)field * total_cells + d.cell_base;
+        const double off = b.off[(size_t)field * total_tiles + gtile];
+        const double scl = b.scl[(size_t)field * total_tiles + gtile];
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int e = threadIdx.x + i * WG, ly = e / TS, lx = e - ly * TS;
+            const size_t c = (size_t)(tyi * TS + ly) * d.nx + txi * TS + lx;
+            const double v = ty == 1 ? off + (double)__half2float(f16[c]) * scl : src[c];
+            ok = ok && isfinite(v);
+            dst[c] = v;
         }
     }
+    if (!ok) *bad = 1;
 }
 
-// Count non-finite values of a dense array (amps_get_field check).
-__global__ void nonfinite_kernel(const double* v, long long n, unsigned long long* cnt) {
-    unsigned long long local = 0;
+// The check alone, of a field that needs no decoding (n is a multiple of 256).
+__global__ __launch_bounds__(256) void nonfinite_kernel(const double* v, long long n, int* bad) {
+    bool ok = true;
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-        local += isfinite(v[i]) ? 0 : 1;
-    if (local) atomicAdd(cnt, local);
+        ok = ok && isfinite(v[i]);
+    if (!ok) *bad = 1;
 }
 
 __global__ void fill_u64_kernel(unsigned long long* p, int n, unsigned long long v) {
@@ -989,11 +996,10 @@ int launch_classify(const InstDesc* inst, const int* tile_inst, int total_tiles,
 }
 
 int launch_gather(const InstDesc* inst, const Buf& b, long long total_cells, int total_tiles, const int* type,
-                  int group, int instid, int ntiles_inst, int field, double* dst, int tile, hipStream_t s) {
+                  int group, int instid, int ntiles_inst, int field, double* dst, int* bad, int tile, hipStream_t s) {
     int grid = ntiles_inst > 65536 ? 65536 : ntiles_inst;
-    if (tile == 16) hipLaunchKernelGGL((gather_kernel<16>), dim3(grid), dim3(256), 0, s, inst, b, total_cells, total_tiles, type, group, instid, field, dst);
-    else if (tile == 32) hipLaunchKernelGGL((gather_kernel<32>), dim3(grid), dim3(256), 0, s, inst, b, total_cells, total_tiles, type, group, instid, field, dst);
-    else if (tile == 64) hipLaunchKernelGGL((gather_kernel<64>), dim3(grid), dim3(256), 0, s, inst, b, total_cells, total_tiles, type, group, instid, field, dst);
+    if (tile == 16) hipLaunchKernelGGL((gather_kernel<16>), dim3(grid), dim3(256), 0, s, inst, b, total_cells, total_tiles, type, group, instid, field, dst, bad);
+    else if (tile == 32) hipLaunchKernelGGL((gather_kernel<32>), dim3(grid), dim3(256), 0, s, inst, b, total_cells, total_tiles, type, group, instid, field, dst, bad);
     else return AMPS_E_UNSUPPORTED;
     return hip_ok();
 }
@@ -1015,10 +1021,10 @@ int launch_worklist(const int* type, const int* type_old, int total_tiles, int* 
     return hip_ok();
 }
 
-int launch_nonfinite(const double* v, long long n, unsigned long long* cnt, hipStream_t s) {
+int launch_nonfinite(const double* v, long long n, int* bad, hipStream_t s) {
     long long g = (n + 255) / 256;
     if (g > 4096) g = 4096;
-    hipLaunchKernelGGL(nonfinite_kernel, dim3((int)g), dim3(256), 0, s, v, n, cnt);
+    hipLaunchKernelGGL(nonfinite_kernel, dim3((int)g), dim3(256), 0, s, v, n, bad);
     return hip_ok();
 }
 

@@ -35,8 +35,8 @@ int launch_classify(const InstDesc* inst, const int* tile_inst, int total_tiles,
                     int single, const double* md, double thr, int dilate, int* type_old, int* type,
                     unsigned long long* stats, hipStream_t s);
 int launch_gather(const InstDesc* inst, const Buf& b, long long total_cells, int total_tiles, const int* type,
-                  int group, int instid, int ntiles_inst, int field, double* dst, int tile, hipStream_t s);
-int launch_nonfinite(const double* v, long long n, unsigned long long* cnt, hipStream_t s);
+                  int group, int instid, int ntiles_inst, int field, double* dst, int* bad, int tile, hipStream_t s);
+int launch_nonfinite(const double* v, long long n, int* bad, hipStream_t s);
 int launch_fill_u64(unsigned long long* p, int n, unsigned long long v, hipStream_t s);
 int launch_advance_step(long long* step_ctr, int n, hipStream_t s);
 
