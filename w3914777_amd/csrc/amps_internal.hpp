@@ -141,8 +141,6 @@ struct StepArgs {
     int grid_cap;               // sweep workgroups at most (0: no cap)
     int t_halo;                 // snowflake: halo depth of the T Laplacian (2: reference stencil in some instance)
     int flags;                  // AMPS_FLAG_* of the run (NO_SKIP: no hold, flush or skip on low tiles)
-    size_t step_stride;         // multi-step launch: 0, or the result of step s goes to out.f64 + s * step_stride
-                                // (doubles); otherwise only the last one, to out.f64
     Buf in, out;
     double* aux_in;             // model auxiliary per-cell array (grain growth: sum of squares)
     double* aux_out;
@@ -158,6 +156,8 @@ struct BlockMap {
     int nblocks;
     const int* inst;
     const int* base;
+    size_t step_stride;  // of one launch: 0, or the result of step s goes to out.f64 + s * step_stride
+                         // (doubles); otherwise only the last one, to out.f64
 };
 
 // NO_SKIP list of the snowflake's flat sweep: NSK_SEGS segments (list

@@ -452,10 +452,12 @@ int multi_steps(const amps_ctx* c, int left) {
     return left >= c->bm.k ? c->bm.k : 0;
 }
 
-int launch_multi(const amps_ctx* c, const StepArgs& a) {
-    if (c->model == AMPS_SNOWFLAKE) return launch_sf_multi(a, c->bm, c->stream);
-    if (c->model == AMPS_GRAINGROWTH) return launch_gg_multi(a, c->bm, c->stream);
-    return launch_sn_multi(a, c->bm, c->stream);
+int launch_multi(const amps_ctx* c, const StepArgs& a, size_t step_stride) {
+    BlockMap bm = c->bm;
+    bm.step_stride = step_stride;
+    if (c->model == AMPS_SNOWFLAKE) return launch_sf_multi(a, bm, c->stream);
+    if (c->model == AMPS_GRAINGROWTH) return launch_gg_multi(a, bm, c->stream);
+    return launch_sn_multi(a, bm, c->stream);
 }
 
 // Push a checkpoint of the tape if the step count has reached one.
@@ -469,7 +471,7 @@ int tape_due(amps_ctx* c) {
 int enqueue_multi(amps_ctx* c) {
     StepArgs a = step_args(c, c->cur);
     a.step_add = c->pending_adv;
-    RCCHK(launch_multi(c, a));
+    RCCHK(launch_multi(c, a, 0));
     c->pending_adv += c->bm.k;
     c->cur ^= 1;
     c->steps_done += c->bm.k;
@@ -603,7 +605,7 @@ void plan_multi(amps_ctx* c, std::vector<int>& inst, std::vector<int>& base) {
         base.push_back((int)inst.size());
         inst.insert(inst.end(), (size_t)(c->desc[i].nx / edge) * (c->desc[i].ny / edge), i);
     }
-    c->bm = BlockMap{k, edge, (int)inst.size(), nullptr, nullptr};
+    c->bm = BlockMap{k, edge, (int)inst.size(), nullptr, nullptr, 0};
 }
 }  // namespace
 
@@ -1239,8 +1241,7 @@ extern "C" int amps_adjoint(amps_ctx* c, const double* dJ_du, const int32_t* par
             a.step_ctr = dstep;
             a.step_add = j;
             if (c->bm.k > 1 && j + c->bm.k < m) {  // bm.k states in a row of `mid`
-                a.step_stride = state;
-                RCCHK(launch_multi(c, a));
+                RCCHK(launch_multi(c, a, state));
                 j += c->bm.k;
             } else {
                 RCCHK(launch_step_kernel(c, a));

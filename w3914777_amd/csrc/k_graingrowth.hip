@@ -837,13 +837,13 @@ __device__ __forceinline__ void gg_multi_step(GgMultiLds<BS, K, Q>& L, const Ste
 
 template <int BS, int K, int Q, int NT>
 __global__ __launch_bounds__(NT) void gg_multi_kernel(StepArgs a, const InstDesc* __restrict__ inst,
-                                                      const int* __restrict__ binst, const int* __restrict__ bbase) {
+                                                      BlockMap bm) {
     constexpr int W0 = BS + 2 * K, NL = (W0 * W0 + NT - 1) / NT;
     __shared__ GgMultiLds<BS, K, Q> L;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const int in = a.ninst > 1 ? binst[b] : 0;
+    const int in = a.ninst > 1 ? bm.inst[b] : 0;
     const InstDesc& d = inst[in];
-    const int lb = a.ninst > 1 ? b - bbase[in] : b, nbx = d.nx / BS;
+    const int lb = a.ninst > 1 ? b - bm.base[in] : b, nbx = d.nx / BS;
     const int ty = lb / nbx, oy = ty * BS, ox = (lb - ty * nbx) * BS;
     const bool per = d.bc == AMPS_BC_PERIODIC;
     const double* f0 = a.in.f64 + d.cell_base;
@@ -922,7 +922,7 @@ int launch_gg_aux(const StepArgs& a, int tile, const int* type_old, hipStream_t 
 int launch_gg_multi(const StepArgs& a, const BlockMap& bm, hipStream_t s) {
 #define GG_MULTI(E, K, Q, NT)                                                                               \
     if (bm.edge == E && bm.k == K && a.q == Q) {                                                            \
-        hipLaunchKernelGGL((gg_multi_kernel<E, K, Q, NT>), dim3(bm.nblocks), dim3(NT), 0, s, a, a.inst, bm.inst, bm.base); \
+        hipLaunchKernelGGL((gg_multi_kernel<E, K, Q, NT>), dim3(bm.nblocks), dim3(NT), 0, s, a, a.inst, bm); \
         return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;                                      \
     }
     GG_MULTI(16, 8, 2, 1024)

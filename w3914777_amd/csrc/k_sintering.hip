@@ -431,7 +431,7 @@ struct SnMultiLds {
 
 template <int BS, int K, bool CONS, bool INPLACE, int S, int NT>
 __device__ __forceinline__ void sn_multi_step(SnMultiLds<BS, K, CONS, INPLACE>& L, const StepArgs& a,
-                                              const InstDesc& d, int ox, int oy, bool edge) {
+                                              const BlockMap& bm, const InstDesc& d, int ox, int oy, bool edge) {
     constexpr int H = 2 * K, W0 = BS + 4 * K, WR = W0 - 2;
     constexpr int HS = 2 * (K - 1 - S), W = BS + 2 * HS, B0 = H - HS, G = INPLACE ? 0 : S & 1, GN = INPLACE ? 0 : (S + 1) & 1;
     const double* C = L.f[G][0];
@@ -483,8 +483,8 @@ __device__ __forceinline__ void sn_multi_step(SnMultiLds<BS, K, CONS, INPLACE>& 
         },
         [&](int e, const New& n) {
             const int y = e / W, x = e - y * W;
-            if (S == K - 1 || (a.step_stride && (unsigned)(y - HS) < (unsigned)BS && (unsigned)(x - HS) < (unsigned)BS)) {
-                double* o = a.out.f64 + S * a.step_stride + d.cell_base + (size_t)(oy - HS + y) * d.nx + ox - HS + x;
+            if (S == K - 1 || (bm.step_stride && (unsigned)(y - HS) < (unsigned)BS && (unsigned)(x - HS) < (unsigned)BS)) {
+                double* o = a.out.f64 + S * bm.step_stride + d.cell_base + (size_t)(oy - HS + y) * d.nx + ox - HS + x;
                 o[0] = n.c;
                 o[a.total_cells] = n.e1;
                 o[2 * a.total_cells] = n.e2;
@@ -498,19 +498,19 @@ __device__ __forceinline__ void sn_multi_step(SnMultiLds<BS, K, CONS, INPLACE>& 
         });
     if constexpr (S + 1 < K) {
         __syncthreads();
-        sn_multi_step<BS, K, CONS, INPLACE, S + 1, NT>(L, a, d, ox, oy, edge);
+        sn_multi_step<BS, K, CONS, INPLACE, S + 1, NT>(L, a, bm, d, ox, oy, edge);
     }
 }
 
 template <int BS, int K, bool CONS, bool INPLACE, int NT>
 __global__ __launch_bounds__(NT) void sn_multi_kernel(StepArgs a, const InstDesc* __restrict__ inst,
-                                                      const int* __restrict__ binst, const int* __restrict__ bbase) {
+                                                      BlockMap bm) {
     constexpr int H = 2 * K, W0 = BS + 4 * K, NL = (W0 * W0 + NT - 1) / NT;
     __shared__ SnMultiLds<BS, K, CONS, INPLACE> L;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const int in = a.ninst > 1 ? binst[b] : 0;
+    const int in = a.ninst > 1 ? bm.inst[b] : 0;
     const InstDesc& d = inst[in];
-    const int lb = a.ninst > 1 ? b - bbase[in] : b, nbx = d.nx / BS;
+    const int lb = a.ninst > 1 ? b - bm.base[in] : b, nbx = d.nx / BS;
     const int ty = lb / nbx, oy = ty * BS, ox = (lb - ty * nbx) * BS;
     const bool per = d.bc == AMPS_BC_PERIODIC;
     const double* f0 = a.in.f64 + d.cell_base;
@@ -533,7 +533,7 @@ __global__ __launch_bounds__(NT) void sn_multi_kernel(StepArgs a, const InstDesc
     }
     __syncthreads();
     const bool edge = !per && (ox == 0 || oy == 0 || ox + BS == d.nx || oy + BS == d.ny);
-    sn_multi_step<BS, K, CONS, INPLACE, 0, NT>(L, a, d, ox, oy, edge);
+    sn_multi_step<BS, K, CONS, INPLACE, 0, NT>(L, a, bm, d, ox, oy, edge);
 }
 
 template <int TS, bool ADAPT, bool CONS>
@@ -575,9 +575,9 @@ template <int BS, int K, bool INPLACE, int NT>
 static int sn_multi_launch(const StepArgs& a, const BlockMap& bm, hipStream_t s) {
     const dim3 g(bm.nblocks), b(NT);
     if (a.flags & AMPS_FLAG_CH_CONSERVATIVE)
-        hipLaunchKernelGGL((sn_multi_kernel<BS, K, true, INPLACE, NT>), g, b, 0, s, a, a.inst, bm.inst, bm.base);
+        hipLaunchKernelGGL((sn_multi_kernel<BS, K, true, INPLACE, NT>), g, b, 0, s, a, a.inst, bm);
     else
-        hipLaunchKernelGGL((sn_multi_kernel<BS, K, false, INPLACE, NT>), g, b, 0, s, a, a.inst, bm.inst, bm.base);
+        hipLaunchKernelGGL((sn_multi_kernel<BS, K, false, INPLACE, NT>), g, b, 0, s, a, a.inst, bm);
     return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;
 }
 

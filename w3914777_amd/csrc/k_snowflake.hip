@@ -1596,8 +1596,8 @@ struct SfMultiLds {
 // Step S of K: ring intermediates on the region and one cell around it, then
 // the new phi and T of the region.
 template <int BS, int K, int S, int NT, bool EDGE>
-__device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepArgs& a, const InstDesc& d, int ox, int oy,
-                                     uint32_t key) {
+__device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepArgs& a, const BlockMap& bm,
+                                              const InstDesc& d, int ox, int oy, uint32_t key) {
     using M = SfMultiLds<BS, K>;
     constexpr int H = 2 * K, W0 = M::W0, WR = M::WR;
     constexpr int HS = 2 * (K - 1 - S), W = BS + 2 * HS, B0 = H - HS;  // region: box coordinates B0 .. B0 + W - 1
@@ -1639,7 +1639,7 @@ __device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepAr
     const bool ref = d.stencil == AMPS_STENCIL_REF;
     const double inv = d.k[SFK_INV_DXDY], dtt = d.k[SFK_DT_OVER_TAU], dt = d.k[SFK_DT], kap = d.k[SFK_KAPPA];
     const double aop = d.k[SFK_ALPHA_OVER_PI], gam = d.k[SFK_GAMMA], teq = d.k[SFK_TEQ], noise = d.k[SFK_NOISE];
-    double* ophi = a.out.f64 + S * a.step_stride + d.cell_base;
+    double* ophi = a.out.f64 + S * bm.step_stride + d.cell_base;
     double* oT = ophi + a.total_cells;
     // the update's long part without a branch, then the noise and the stores
     struct Part { double ph, t, lt, br; };
@@ -1691,7 +1691,7 @@ __device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepAr
             }
             const double phn = ph + dtt * br;
             const double tn = sf_t_update<double>(v.t, v.lt, dt, kap, phn - ph);
-            if (S == K - 1 || (a.step_stride && (unsigned)(y - HS) < (unsigned)BS && (unsigned)(x - HS) < (unsigned)BS)) {
+            if (S == K - 1 || (bm.step_stride && (unsigned)(y - HS) < (unsigned)BS && (unsigned)(x - HS) < (unsigned)BS)) {
                 const int g = (oy - HS + y) * d.nx + ox - HS + x;
                 ophi[g] = phn;
                 oT[g] = tn;
@@ -1705,25 +1705,25 @@ __device__ __forceinline__ void sf_multi_step(SfMultiLds<BS, K>& L, const StepAr
 }
 
 template <int BS, int K, int NT, bool EDGE>
-__device__ __forceinline__ void sf_multi_steps(SfMultiLds<BS, K>& L, const StepArgs& a, const InstDesc& d, int ox,
-                                               int oy, long long step) {
-    sf_multi_step<BS, K, 0, NT, EDGE>(L, a, d, ox, oy, noise_key(d.seed, (uint64_t)step));
-    if constexpr (K > 1) sf_multi_step<BS, K, 1, NT, EDGE>(L, a, d, ox, oy, noise_key(d.seed, (uint64_t)(step + 1)));
-    if constexpr (K > 2) sf_multi_step<BS, K, 2, NT, EDGE>(L, a, d, ox, oy, noise_key(d.seed, (uint64_t)(step + 2)));
-    if constexpr (K > 3) sf_multi_step<BS, K, 3, NT, EDGE>(L, a, d, ox, oy, noise_key(d.seed, (uint64_t)(step + 3)));
+__device__ __forceinline__ void sf_multi_steps(SfMultiLds<BS, K>& L, const StepArgs& a, const BlockMap& bm,
+                                               const InstDesc& d, int ox, int oy, long long step) {
+    sf_multi_step<BS, K, 0, NT, EDGE>(L, a, bm, d, ox, oy, noise_key(d.seed, (uint64_t)step));
+    if constexpr (K > 1) sf_multi_step<BS, K, 1, NT, EDGE>(L, a, bm, d, ox, oy, noise_key(d.seed, (uint64_t)(step + 1)));
+    if constexpr (K > 2) sf_multi_step<BS, K, 2, NT, EDGE>(L, a, bm, d, ox, oy, noise_key(d.seed, (uint64_t)(step + 2)));
+    if constexpr (K > 3) sf_multi_step<BS, K, 3, NT, EDGE>(L, a, bm, d, ox, oy, noise_key(d.seed, (uint64_t)(step + 3)));
 }
 
 template <int BS, int K, int NT>
 __global__ __launch_bounds__(NT) void sf_multi_kernel(StepArgs a, const InstDesc* __restrict__ inst,
-                                                      const int* __restrict__ binst, const int* __restrict__ bbase) {
+                                                      BlockMap bm) {
     using M = SfMultiLds<BS, K>;
     constexpr int H = 2 * K, W0 = M::W0, NL = (W0 * W0 + NT - 1) / NT;
     __shared__ __align__(16) M L;
     const long long step = *a.step_ctr + a.step_add;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const int in = a.ninst > 1 ? binst[b] : 0;
+    const int in = a.ninst > 1 ? bm.inst[b] : 0;
     const InstDesc& d = inst[in];
-    const int lb = a.ninst > 1 ? b - bbase[in] : b, nbx = d.nx / BS;
+    const int lb = a.ninst > 1 ? b - bm.base[in] : b, nbx = d.nx / BS;
     const int ty = lb / nbx, oy = ty * BS, ox = (lb - ty * nbx) * BS;
     const bool per = d.bc == AMPS_BC_PERIODIC;
     const double* fphi = a.in.f64 + d.cell_base;
@@ -1747,8 +1747,8 @@ __global__ __launch_bounds__(NT) void sf_multi_kernel(StepArgs a, const InstDesc
     }
     __syncthreads();
     const bool edge = !per && (ox == 0 || oy == 0 || ox + BS == d.nx || oy + BS == d.ny);
-    if (edge) sf_multi_steps<BS, K, NT, true>(L, a, d, ox, oy, step);
-    else sf_multi_steps<BS, K, NT, false>(L, a, d, ox, oy, step);
+    if (edge) sf_multi_steps<BS, K, NT, true>(L, a, bm, d, ox, oy, step);
+    else sf_multi_steps<BS, K, NT, false>(L, a, bm, d, ox, oy, step);
 }
 
 // ------------------------------------------------------------ host launch
@@ -1833,7 +1833,7 @@ int launch_sf_step(const StepArgs& a, int tile, bool adaptive, hipStream_t s, co
 int launch_sf_multi(const StepArgs& a, const BlockMap& bm, hipStream_t s) {
 #define SF_MULTI(E, K, NT)                                                                                  \
     if (bm.edge == E && bm.k == K) {                                                                        \
-        hipLaunchKernelGGL((sf_multi_kernel<E, K, NT>), dim3(bm.nblocks), dim3(NT), 0, s, a, a.inst, bm.inst, bm.base); \
+        hipLaunchKernelGGL((sf_multi_kernel<E, K, NT>), dim3(bm.nblocks), dim3(NT), 0, s, a, a.inst, bm); \
         return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;                                      \
     }
     SF_MULTI(16, 4, 768)
