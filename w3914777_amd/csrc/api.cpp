@@ -70,7 +70,8 @@ struct amps_ctx {
     std::vector<amps_config> cfg;
     std::vector<InstDesc> desc;
     std::vector<int> tile_inst;
-    long long total_cells = 0;
+    long long cells = 0;                   // grid points of all instances
+    long long total_cells = 0;             // cells from one field to the next
     int total_tiles = 0;
     long long max_inst_cells = 0;
     GroupMap gm{};
@@ -146,6 +147,16 @@ namespace {
 // Device memory of a context: the buffers are asked for one by one and come
 // from one zeroed allocation (an allocation costs 30 us to make and 250 us to
 // free, whatever its size).
+//
+// Grids of power-of-two sides would put the same cell of every buffer, and of
+// every field of a buffer, on the same memory channels: the buffers are
+// STAGGER bytes further apart than they need to be, the fields FIELD_PAD
+// cells (a multiple of 32: the vector loads' alignment).  Measured on Q = 36
+// grain growth: adaptive 1024^2 137 us a step with neither (the buffers'
+// stagger alone gives 134), 129 with both; FP64 2048^2 567 -> 530.
+constexpr size_t STAGGER = 4352;
+constexpr long long FIELD_PAD = 1056;
+
 struct DeviceArena {
     struct Ask {
         void** p;
@@ -154,7 +165,7 @@ struct DeviceArena {
     std::vector<Ask> asks;
     template <typename T>
     void ask(T** p, size_t bytes) {
-        asks.push_back({reinterpret_cast<void**>(p), (std::max<size_t>(bytes, 8) + 255) & ~(size_t)255});
+asks.push_back({reinterpret_cast<void**>(p), ((std::max<size_t>(bytes, 8) + 255) & ~(size_t)255) + STAGGER});
     }
     int get(amps_ctx* c) {
         size_t total = 0;
@@ -772,7 +783,8 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
         c->max_inst_cells = std::max(c->max_inst_cells, (long long)d.nx * d.ny);
         for (int t = 0; t < d.tx * d.ty; ++t) c->tile_inst.push_back(i);
     }
-    c->total_cells = cells;
+    c->cells = cells;
+    c->total_cells = cells + FIELD_PAD;
     c->total_tiles = tiles;
 
     int rc = AMPS_OK;
@@ -787,9 +799,9 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     mem.ask(&c->d_tile_inst, sizeof(int) * tiles);
     const size_t nf = (size_t)c->nfields;
     for (int b = 0; b < 2; ++b) {
-        mem.ask(&c->buf[b].f64, nf * cells * sizeof(double));
+        mem.ask(&c->buf[b].f64, nf * c->total_cells * sizeof(double));
         if (has_low(c)) {
-            mem.ask(&c->buf[b].f16, nf * cells * sizeof(__half));
+            mem.ask(&c->buf[b].f16, nf * c->total_cells * sizeof(__half));
             mem.ask(&c->buf[b].off, nf * tiles * sizeof(double));
             mem.ask(&c->buf[b].scl, nf * tiles * sizeof(float));
             if (c->model == AMPS_GRAINGROWTH) mem.ask(&c->buf[b].zmask, tiles * sizeof(unsigned long long));
@@ -1097,7 +1109,7 @@ int amps_get_info(amps_ctx* c, amps_info* info) {
         for (int v : t) hi += (v == 2) || !has_low(c);
         info->hi_frac_last = info->hi_frac_mean = has_low(c) ? hi / denom : 1.0;
     }
-    info->cells = (double)c->total_cells;
+    info->cells = (double)c->cells;
     return AMPS_OK;
 }
 

@@ -99,6 +99,9 @@ __device__ inline void sf_phase1(const Rt* phi, Rt* P, Rt* Q, Rt* E2, const Inst
                                  Rt inv2dx, Rt inv2dy, Rt cth0, Rt sth0, Rt epsb, Rt epsbd, Rt mend,
                                  bool fast = false) {
     using G = SfGeo<TS>;
+    // the 32^2 mixed sweep (NT = WG) is at its register limit: the path for
+    // n == 4 costs it 3% whether it is taken or not
+    constexpr bool FOUR = TS == 16 || NT != WG;
     const int n = (int)d.k[SFK_ANISO_N];
     const bool edge = d.bc != AMPS_BC_PERIODIC &&
                       (ox == 0 || oy == 0 || ox + TS == d.nx || oy + TS == d.ny);
@@ -112,7 +115,7 @@ __device__ inline void sf_phase1(const Rt* phi, Rt* P, Rt* Q, Rt* E2, const Inst
             Rt gx = (phi[c + 1] - phi[c - 1]) * inv2dx;
             Rt gy = (phi[c + G::LW] - phi[c - G::LW]) * inv2dy;
             Rt eps, epsd;
-            sf_aniso<Rt>(gx, gy, n, cth0, sth0, epsb, epsbd, mend, eps, epsd);
+            sf_aniso<Rt, FOUR>(gx, gy, n, cth0, sth0, epsb, epsbd, mend, eps, epsd);
             Rt A = eps * epsd;
             P[o] = A * gx;
             Q[o] = A * gy;
@@ -131,7 +134,7 @@ __device__ inline void sf_phase1(const Rt* phi, Rt* P, Rt* Q, Rt* E2, const Inst
         Rt gx = (phi[c + 1] - phi[c - 1]) * inv2dx;
         Rt gy = (phi[c + G::LW] - phi[c - G::LW]) * inv2dy;
         Rt eps, epsd;
-        sf_aniso<Rt>(gx, gy, n, cth0, sth0, epsb, epsbd, mend, eps, epsd);
+        sf_aniso<Rt, FOUR>(gx, gy, n, cth0, sth0, epsb, epsbd, mend, eps, epsd);
         Rt A = eps * epsd;
         const int o = G::RB + ry0 * G::PW + rx0 - 1;
         P[o] = A * gx;

@@ -93,12 +93,13 @@ __device__ inline void sf_unit_power4(R gx, R gy, R& c, R& s) {
     s = nz ? s : R(0);
 }
 
-template <typename R>
+// FOUR: with a path of its own for n == 4 (the results are the same).
+template <typename R, bool FOUR = true>
 __device__ inline void sf_aniso(R gx, R gy, int n, R cth0, R sth0, R epsb, R epsb_delta, R m_epsb_n_delta,
                                 R& eps, R& epsd) {
     R c, s;
     if (n == 6) sf_unit_power6<R>(gx, gy, c, s);  // the snowflake's six-fold case
-    else if (n == 4) sf_unit_power4<R>(gx, gy, c, s);  // the reference's
+    else if (FOUR && n == 4) sf_unit_power4<R>(gx, gy, c, s);  // the reference's
     else sf_unit_power<R>(gx, gy, n, c, s);
     R ca = c * cth0 + s * sth0;  // cos(n (theta - theta0))
     R sa = s * cth0 - c * sth0;  // sin(n (theta - theta0))
