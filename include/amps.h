@@ -306,10 +306,9 @@ int amps_get_sweep_time(amps_ctx* ctx, int which, int64_t* launches, double* tot
  * hipStream_t; NULL: the null stream) and the call returns without waiting.
  * No reference counterpart: it is for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops).  It allocates
- * nothing: the descriptor and step counter the step kernels read go to a
- * fixed 4 KiB device array of the library, one per GPU, written by a kernel
- * at each call; grids are limited only as in amps_create.  Calls that
- * overlap on one GPU (other streams or host threads) race on that array.
+ * nothing and is one kernel launch: the descriptor and the step index travel
+ * as its arguments, so calls on other streams or host threads share nothing.
+ * Grids are limited only as in amps_create.
  * The result equals amps_step on a PURE_FP64 context of the same config. */
 int amps_sf_step_fp64_noalloc(const amps_config* cfg, const double* d_in, double* d_out, int64_t step,
                               void* stream);

@@ -1320,6 +1320,16 @@ __global__ __launch_bounds__(NT) void sf_f64_tile_kernel(StepArgs a, const InstD
     sf_tile_f64<TS, false, NT>(L, a, d, tile_x, tile_y, 0x1FFu, step);
 }
 
+// The same sweep of one grid whose descriptor and step index are kernel
+// arguments (the no-allocation step: no device copy of them to write first).
+template <int TS, int NT>
+__global__ __launch_bounds__(NT) void sf_f64_arg_kernel(StepArgs a, InstDesc d, long long step) {
+    __shared__ __align__(16) SfLds<TS, double> L;
+    const int w = xcd_remap(blockIdx.x, a.nwork);
+    const int tile_y = w / d.tx, tile_x = w - tile_y * d.tx;
+    sf_tile_f64<TS, false, NT>(L, a, d, tile_x, tile_y, 0x1FFu, step);
+}
+
 // Mixed sweep of the adaptive step: the FP64 tiles (FP64 work-list) and the
 // low tiles that failed the hold sweep's bulk-hold test (its 8 segments of
 // this step's parity) are the items of one persistent launch, so the two
@@ -1830,6 +1840,14 @@ int launch_sf_step(const StepArgs& a, int tile, bool adaptive, hipStream_t s, co
     } else {
         return AMPS_E_UNSUPPORTED;
     }
+    return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;
+}
+
+int launch_sf_step_arg(const StepArgs& a, const InstDesc& d, long long step, int tile, hipStream_t s) {
+    // thread counts as in sf_launch
+    if (tile == 16) hipLaunchKernelGGL((sf_f64_arg_kernel<16, WG>), dim3(a.nwork), dim3(WG), 0, s, a, d, step);
+    else if (tile == 32) hipLaunchKernelGGL((sf_f64_arg_kernel<32, 512>), dim3(a.nwork), dim3(512), 0, s, a, d, step);
+    else return AMPS_E_UNSUPPORTED;
     return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;
 }
 
