@@ -160,6 +160,10 @@ struct BlockMap {
                          // (doubles); otherwise only the last one, to out.f64
 };
 
+// Device counters spread over cache lines of their own (atomics on one line
+// serialise): STATS_STRIDE words apart.
+constexpr int STATS_STRIDE = 8, CLASSIFY_SLOTS = 64;
+
 // NO_SKIP list of the snowflake's flat sweep: NSK_SEGS segments (list
 // position mod NSK_SEGS) of nsk_cap(total_tiles) entries, their counters
 // NSK_CNT_STRIDE ints (256 B) apart so that the appends of one launch spread

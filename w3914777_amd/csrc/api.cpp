@@ -59,6 +59,8 @@ void set_error_text(const char* msg) { g_last_error = msg ? msg : ""; }
 // ints of the list counters: the larger of the two layouts (bulk-hold [2][8],
 // NO_SKIP [2][NSK_SEGS] at a stride of NSK_CNT_STRIDE)
 constexpr size_t FULL_CNT_INTS = 2 * (size_t)NSK_SEGS * NSK_CNT_STRIDE;
+// words of the classification's counters (all passes, the last pass)
+constexpr size_t CLS_WORDS = 2 * (size_t)CLASSIFY_SLOTS * STATS_STRIDE;
 
 struct amps_ctx {
     int model = 0, mode = 0, monitor = 0, tile = 16, every = 10, mfield = 0;
@@ -84,8 +86,9 @@ struct amps_ctx {
     int* d_type_old = nullptr;
     double* d_md = nullptr;
     double* d_last = nullptr;
-    unsigned long long* d_stats = nullptr;  // [0] sum of FP64 tiles over passes, [1] last pass,
-                                            // [2], [3], [4] snowflake sweep tile counts (summed)
+    unsigned long long* d_stats = nullptr;  // [2], [3], [4] snowflake sweep tile counts (summed)
+    unsigned long long* d_cls = nullptr;    // FP64 tiles over monitor passes and of the last pass
+                                            // (launch_classify_convert)
     long long* d_step = nullptr;
     double* d_aux[2] = {nullptr, nullptr};
     double* d_scratch = nullptr;           // max instance cells (decoded field of amps_get_field)
@@ -423,20 +426,14 @@ int enqueue_monitor(amps_ctx* c, int b) {
     }
     // the monitored field's own precision decides how it is read
     if (c->gm.fg[field0] < 0) a.type = nullptr;
-    // the monitor kernel also clears the classification's per-pass FP64 count
+    // the monitor kernel also clears the classification's per-pass FP64 counts
     RCCHK(launch_monitor(a, c->monitor, c->tile, ngroups_eval, field0, stride, c->ngroups, c->d_md, c->d_last,
-                         c->d_stats + 1, c->stream));
-    RCCHK(launch_classify(c->d_desc, c->d_tile_inst, c->total_tiles, c->ngroups, broadcast, c->ninst == 1 ? 1 : 0,
-                          c->d_md, c->thr_eff, c->dilate,
-                          c->d_type_old, c->d_type, c->d_stats, c->stream));
-    RCCHK(launch_convert(c->d_desc, c->d_tile_inst, c->buf[b], c->total_cells, c->total_tiles, c->d_type_old,
-                         c->d_type, c->gm, CONVERT_CHANGED, c->tile, c->stream));
-    if (c->model == AMPS_GRAINGROWTH) {
-        RCCHK(refresh_aux(c, b, true));
-        if (has_low(c))  // converted field-tiles: the buffers no longer agree
-            RCCHK(launch_clear_changed(c->d_type_old, c->d_type, c->gm, c->nfields, c->total_tiles, c->d_same_flags,
-                                       c->buf[b].zmask, c->stream));
-    }
+                         c->d_cls + CLASSIFY_SLOTS * STATS_STRIDE, c->stream));
+    RCCHK(launch_classify_convert(c->d_desc, c->d_tile_inst, c->buf[b], c->total_cells, c->total_tiles, broadcast,
+                                  c->ninst == 1 ? 1 : 0, c->d_md, c->thr_eff, c->dilate, c->d_type_old, c->d_type,
+                                  c->gm, c->model == AMPS_SINTERING ? nullptr : c->d_same_flags, c->d_cls, c->tile,
+                                  c->stream));
+    RCCHK(refresh_aux(c, b, true));
     RCCHK(refresh_worklists(c, true));
     return AMPS_OK;
 }
@@ -814,6 +811,7 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     mem.ask(&c->d_md, gt * sizeof(double));
     if (c->mode == AMPS_ADAPTIVE && c->monitor == AMPS_MON_TEMPORAL) mem.ask(&c->d_last, gt * 16 * sizeof(double));
     mem.ask(&c->d_stats, 8 * sizeof(unsigned long long));
+    mem.ask(&c->d_cls, CLS_WORDS * sizeof(unsigned long long));
     mem.ask(&c->d_step, sizeof(long long));
     if (has_low(c)) mem.ask(&c->d_scratch, (size_t)c->max_inst_cells * sizeof(double));
     mem.ask(&c->d_wl, 2 * (size_t)tiles * sizeof(int));
@@ -887,6 +885,7 @@ int amps_init(amps_ctx* c) {
     HIPCHK(hipMemcpyAsync(c->d_step, &zero, sizeof(zero), hipMemcpyHostToDevice, c->stream));
     static const unsigned long long z8[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     HIPCHK(hipMemcpyAsync(c->d_stats, z8, sizeof(z8), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemsetAsync(c->d_cls, 0, CLS_WORDS * sizeof(unsigned long long), c->stream));
     // step 0 appends to parity 0
     if (c->d_full_cnt) HIPCHK(hipMemsetAsync(c->d_full_cnt, 0, FULL_CNT_INTS * sizeof(int), c->stream));
     HIPCHK(hipMemsetAsync(c->d_same_flags, 0, c->same_flags_n * sizeof(int), c->stream));
@@ -1100,8 +1099,15 @@ int amps_get_info(amps_ctx* c, amps_info* info) {
     info->ninstances = c->ninst;
     const double denom = (double)c->ngroups * c->total_tiles;
     if (c->mode == AMPS_ADAPTIVE && c->monitor_passes > 0) {
-        info->hi_frac_last = st[1] / denom;
-        info->hi_frac_mean = st[0] / (denom * c->monitor_passes);
+        std::vector<unsigned long long> cls(CLS_WORDS);
+        HIPCHK(hipMemcpy(cls.data(), c->d_cls, CLS_WORDS * sizeof(unsigned long long), hipMemcpyDeviceToHost));
+        double all = 0.0, last = 0.0;
+        for (int k = 0; k < CLASSIFY_SLOTS; ++k) {
+            all += (double)cls[(size_t)k * STATS_STRIDE];
+            last += (double)cls[(size_t)(CLASSIFY_SLOTS + k) * STATS_STRIDE];
+        }
+        info->hi_frac_last = last / denom;
+        info->hi_frac_mean = all / (denom * c->monitor_passes);
     } else {
         std::vector<int> t((size_t)c->ngroups * c->total_tiles);
         if (has_low(c)) HIPCHK(hipMemcpy(t.data(), c->d_type, t.size() * sizeof(int), hipMemcpyDeviceToHost));

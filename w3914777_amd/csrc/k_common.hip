@@ -226,46 +226,50 @@ __device__ inline double read_decoded(const Buf& b, long long total_cells, int t
                                                          (double)b.scl[(size_t)field * total_tiles + gtile];
 }
 
-// Monitor1 / Monitor2 on the 4x4 sample lattice, one thread per (group,
-// tile).  Monitor1: get_max_diff1 (snowflake/tools.h:177-193), min starts
-// at 1 and max at 0.  Monitor2: get_max_diff2 (tools.h:194-211) against the
-// samples kept from the previous pass, which are then refreshed (the
-// reference refreshes phi_last right after the monitor, function.h:106-113).
-__global__ void monitor_samples_kernel(const InstDesc* inst, const int* tile_inst, Buf b, long long total_cells,
-                                       int total_tiles, const int* type, int ngroups_eval, int field0,
-                                       int field_stride, int type_groups, int tile, int kind, double* md,
-                                       double* last, unsigned long long* __restrict__ reset) {
-    if (reset && blockIdx.x == 0 && threadIdx.x == 0) *reset = 0ull;  // counter the classification adds to
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= ngroups_eval * total_tiles) return;
+// Monitor1 / Monitor2 on the 4x4 sample lattice, 16 lanes per (group, tile),
+// one sample each (one thread per tile walked its 16 dependent reads: 10.2 us
+// a pass at 1024 tiles against 3.3).  Monitor1: get_max_diff1
+// (snowflake/tools.h:177-193), min starts at 1 and max at 0.  Monitor2:
+// get_max_diff2 (tools.h:194-211) against the samples kept from the previous
+// pass, which are then refreshed (the reference refreshes phi_last right after
+// the monitor, function.h:106-113).  A NaN sample is below and above nothing.
+__global__ __launch_bounds__(256) void monitor_samples_kernel(const InstDesc* __restrict__ inst,
+                                                              const int* __restrict__ tile_inst, Buf b,
+                                                              long long total_cells, int total_tiles,
+                                                              const int* __restrict__ type, int ngroups_eval,
+                                                              int field0, int field_stride, int type_groups, int tile,
+                                                              int kind, double* __restrict__ md,
+                                                              double* __restrict__ last,
+                                                              unsigned long long* __restrict__ reset) {
+    if (blockIdx.x == 0 && threadIdx.x < CLASSIFY_SLOTS) reset[threadIdx.x * STATS_STRIDE] = 0ull;  // the classification's counters
+    const int n = ngroups_eval * total_tiles;
+    const int item = blockIdx.x * 16 + (threadIdx.x >> 4), k = threadIdx.x & 15, j = k >> 2, i = k & 3;
+    const int w = item < n ? item : n - 1;  // lanes past the end repeat the last item
     const int g = w / total_tiles, gtile = w - g * total_tiles;
     const int field = field0 + g * field_stride;
     const InstDesc& d = inst[tile_inst[gtile]];
     const int lt = gtile - d.tile_base, tyi = lt / d.tx, txi = lt - tyi * d.tx;
     const int tgroup = type_groups > 1 ? (g < type_groups ? g : 0) : 0;
     const int ty = type ? type[(size_t)tgroup * total_tiles + gtile] : 2;
+    const double v = read_decoded(b, total_cells, total_tiles, d, field, gtile, ty,
+                                  tyi * tile + sample_off(tile, kind, j), txi * tile + sample_off(tile, kind, i));
     if (kind == AMPS_MON_SPATIAL) {
-        double mn = 1.0, mx = 0.0;
-        for (int j = 0; j < 4; ++j)
-            for (int i = 0; i < 4; ++i) {
-                double v = read_decoded(b, total_cells, total_tiles, d, field, gtile, ty,
-                                        tyi * tile + sample_off(tile, kind, j), txi * tile + sample_off(tile, kind, i));
-                if (v < mn) mn = v;
-                if (v > mx) mx = v;
-            }
-        md[w] = mx - mn;
+        double mn = v < 1.0 ? v : 1.0, mx = v > 0.0 ? v : 0.0;
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) {
+            mn = fmin(mn, __shfl_xor(mn, o, 16));
+            mx = fmax(mx, __shfl_xor(mx, o, 16));
+        }
+        if (k == 0 && item < n) md[w] = mx - mn;
     } else {
-        double m = 0.0;
-        double* lw = last + (size_t)w * 16;
-        for (int j = 0; j < 4; ++j)
-            for (int i = 0; i < 4; ++i) {
-                double v = read_decoded(b, total_cells, total_tiles, d, field, gtile, ty,
-                                        tyi * tile + sample_off(tile, kind, j), txi * tile + sample_off(tile, kind, i));
-                double df = fabs(lw[j * 4 + i] - v);
-                if (df > m) m = df;
-                lw[j * 4 + i] = v;
-            }
-        md[w] = m;
+        const double df = fabs(last[(size_t)w * 16 + k] - v);
+        double m = df > 0.0 ? df : 0.0;
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 16));
+        if (item < n) {
+            last[(size_t)w * 16 + k] = v;
+            if (k == 0) md[w] = m;
+        }
     }
 }
 
@@ -296,7 +300,7 @@ __global__ void monitor_last_init_kernel(const InstDesc* inst, const int* tile_i
 template <int TS>
 __global__ __launch_bounds__(256) void monitor_grad_kernel(StepArgs a, int ngroups_eval, int field0,
                                                            int field_stride, int type_groups, double* md, unsigned long long* __restrict__ reset) {
-    if (reset && blockIdx.x == 0 && threadIdx.x == 0) *reset = 0ull;  // counter the classification adds to
+    if (blockIdx.x == 0 && threadIdx.x < CLASSIFY_SLOTS) reset[threadIdx.x * STATS_STRIDE] = 0ull;  // the classification's counters
     constexpr int H = 1, LW = TS + 2;
     __shared__ double box[LW * LW];
     __shared__ NbField nbf;
@@ -356,7 +360,7 @@ __global__ __launch_bounds__(64) void monitor_grad_wave16(StepArgs a, const Inst
                                                           const int* __restrict__ tinst,
                                                           const int* __restrict__ types, int ngroups_eval, int field0,
                                                           int field_stride, int type_groups, double* __restrict__ md, unsigned long long* __restrict__ reset) {
-    if (reset && blockIdx.x == 0 && threadIdx.x == 0) *reset = 0ull;  // counter the classification adds to
+    if (blockIdx.x == 0 && threadIdx.x < CLASSIFY_SLOTS) reset[threadIdx.x * STATS_STRIDE] = 0ull;  // the classification's counters
     constexpr int TS = 16, LWD = MonWaveLds::LWD, C0 = MonWaveLds::C0;
     static_assert(LWD % 2 == 0 && LWD >= C0 + TS + 2, "16-byte reads of columns x0-2 .. x0+5");
     __shared__ __align__(16) MonWaveLds L;
@@ -545,77 +549,107 @@ __global__ __launch_bounds__(64) void monitor_grad_wave16(StepArgs a, const Inst
     }
 }
 
-// get_type (snowflake/tools.h:212-230): type_old <- type; neighbour max over
-// self and the 4 non-periodic von-Neumann neighbours with fmax (CUDA's max);
-// < thr -> 1, >= thr -> 2, unordered keeps the old type.  One thread per
-// (group, tile); with broadcast every group takes group 0's monitor value.
-constexpr int CL_PT = 1;  // (group, tile) items per thread: one dependent load chain each
+// get_type (snowflake/tools.h:212-230) and the conversion of the tiles whose
+// type it changes, in one launch: type_old <- type; neighbour max over self
+// and the 4 non-periodic von-Neumann neighbours with fmax (CUDA's max), and
+// over the tiles within Chebyshev distance `dilate` (non-periodic, inside the
+// instance); < thr -> 1, >= thr -> 2, unordered keeps the old type.  With
+// broadcast every group takes group 0's monitor value.
+//
+// A workgroup takes `items` consecutive (group, tile) items (at most 64, so
+// that a pass has up to CLASSIFY_GRID workgroups): four threads an item share
+// the neighbour reads, wave 0 decides, then the workgroup converts the changed
+// items one by one (a conversion reads and writes its own tile only, so no
+// other workgroup's decision matters to it).  A changed item loses its "both
+// buffers hold the same" flag and (grain growth) its zero-mask bit.  The pass's
+// FP64 count goes to CLASSIFY_SLOTS counters of their own cache lines.
+//
+// Against a classification of one thread an item and a conversion launch
+// after it, a pass is one launch shorter; dilation by 2 alone took 6.4 us in
+// a chain of 25 reads a thread at 16384 tiles.
+constexpr int CLASSIFY_GRID = 2048;
 
-__global__ __launch_bounds__(1024) void classify_kernel(const InstDesc* __restrict__ inst,
-                                                        const int* __restrict__ tile_inst, int total_tiles,
-                                                        int ngroups, int broadcast, int single, const double* md,
-                                                        double thr, int dilate, int* type_old, int* type,
-                                                        unsigned long long* stats) {
-    __shared__ unsigned cnt[16];
+template <int TS>
+__global__ __launch_bounds__(256) void classify_convert_kernel(const InstDesc* __restrict__ inst,
+                                                               const int* __restrict__ tile_inst, Buf b,
+                                                               long long total_cells, int total_tiles, int broadcast,
+                                                               int single, const double* __restrict__ md, double thr,
+                                                               int dilate, int* __restrict__ type_old,
+                                                               int* __restrict__ type, GroupMap gm, int items,
+                                                               int* __restrict__ same_flags,
+                                                               unsigned long long* __restrict__ stats) {
+    __shared__ double red[2 * WG / 64];
+    __shared__ double part[WG / 64][64];
+    __shared__ int todo[64];
+    __shared__ int ntodo;
+    const int n = gm.ngroups * total_tiles;
+    const int lane = threadIdx.x & 63, quarter = threadIdx.x >> 6;
     unsigned nhi = 0;
-    const int n = ngroups * total_tiles;
-#pragma unroll
-    for (int k = 0; k < CL_PT; ++k) {
-        const int w = (blockIdx.x * CL_PT + k) * blockDim.x + threadIdx.x;
-        if (w >= n) continue;
-        const int g = w / total_tiles, gtile = w - g * total_tiles;
+    for (long long c0 = (long long)blockIdx.x * items; c0 < n; c0 += (long long)gridDim.x * items) {
+        const long long w = c0 + lane;
+        const bool mine = lane < items && w < n;
+        const int g = mine ? (int)w / total_tiles : 0, gtile = mine ? (int)w - g * total_tiles : 0;
         const InstDesc& d = inst[single ? 0 : tile_inst[gtile]];  // one instance: no tile -> instance load
         const int lt = gtile - d.tile_base, uy = lt / d.tx, ux = lt - uy * d.tx;
         const double* m0 = md + (size_t)(broadcast ? 0 : g) * total_tiles;
         double m = m0[gtile];
-        if (uy < d.ty - 1) m = fmax(m, m0[gtile + d.tx]);
-        if (uy > 0) m = fmax(m, m0[gtile - d.tx]);
-        if (ux < d.tx - 1) m = fmax(m, m0[gtile + 1]);
-        if (ux > 0) m = fmax(m, m0[gtile - 1]);
-        // dilation of the FP64 set: the maximum over the tiles within
-        // Chebyshev distance `dilate` (non-periodic, inside the instance)
+        if (quarter == 0) {
+            if (uy < d.ty - 1) m = fmax(m, m0[gtile + d.tx]);
+            if (uy > 0) m = fmax(m, m0[gtile - d.tx]);
+            if (ux < d.tx - 1) m = fmax(m, m0[gtile + 1]);
+            if (ux > 0) m = fmax(m, m0[gtile - 1]);
+        }
         if (dilate > 0) {
-            const int y0 = max(uy - dilate, 0), y1 = min(uy + dilate, d.ty - 1);
+            const int y1 = min(uy + dilate, d.ty - 1);
             const int x0 = max(ux - dilate, 0), x1 = min(ux + dilate, d.tx - 1);
-            for (int yy = y0; yy <= y1; ++yy)
+            for (int yy = max(uy - dilate, 0) + quarter; yy <= y1; yy += WG / 64)
                 for (int xx = x0; xx <= x1; ++xx) m = fmax(m, m0[d.tile_base + yy * d.tx + xx]);
         }
-        int t = type[w];
-        type_old[w] = t;
-        if (m < thr) t = 1;
-        else if (m >= thr) t = 2;
-        type[w] = t;
-        nhi += t == 2 ? 1u : 0u;
-    }
-    // FP64 count of the block: wave sums, then one atomic per counter per
-    // block (per-wave atomics on one address serialise)
-    const unsigned ws = (unsigned)__ockl_wfred_add_i32((int)nhi);
-    if ((threadIdx.x & 63) == 0) cnt[threadIdx.x >> 6] = ws;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long tot = 0;
-        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) tot += cnt[i];
-        if (tot) {
-            atomicAdd(&stats[0], tot);
-            atomicAdd(&stats[1], tot);
+        part[quarter][lane] = m;
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            int op = 0;  // 1 encode, 2 decode
+            bool hi = false;
+            if (mine) {
+#pragma unroll
+                for (int q = 1; q < WG / 64; ++q) m = fmax(m, part[q][lane]);
+                const int to = type[w];
+                int tn = to;
+                type_old[w] = to;
+                if (m < thr) tn = 1;
+                else if (m >= thr) tn = 2;
+                type[w] = tn;
+                hi = tn == 2;
+                op = (to == 2 && tn == 1) ? 1 : ((to == 1 && tn == 2) ? 2 : 0);
+                if (op) {
+                    if (same_flags) same_flags[w] = 0;
+                    if (b.zmask) atomicAnd(b.zmask + gtile, ~(1ull << g));
+                }
+            }
+            nhi += (unsigned)__popcll(__ballot(hi));
+            const unsigned long long mo = __ballot(op != 0);
+            if (op) todo[__popcll(mo & ((1ull << lane) - 1ull))] = (int)w * 2 + (op - 1);
+            if (lane == 0) ntodo = __popcll(mo);
         }
+        __syncthreads();
+        const int nt = ntodo;
+        for (int i = 0; i < nt; ++i) {
+            const int it = todo[i], wi = it >> 1;
+            const int gi = wi / total_tiles, ti = wi - gi * total_tiles;
+            const InstDesc& di = inst[single ? 0 : tile_inst[ti]];
+            for (int f = 0; f < gm.nfields; ++f) {
+                if (gm.fg[f] != gi) continue;
+                if ((it & 1) == 0) encode_tile<TS>(b, total_cells, total_tiles, di, ti, f, red);
+                else decode_tile<TS>(b, total_cells, total_tiles, di, ti, f, b.f64 + (size_t)f * total_cells + di.cell_base);
+                __syncthreads();
+            }
+        }
+        __syncthreads();  // part, todo and ntodo are rewritten by the next round
     }
-}
-
-// Clears same_flags[f][tile] where the type group of field f changed type on
-// the tile (the monitor pass converted it: its two buffers no longer agree).
-__global__ void clear_changed_kernel(const int* __restrict__ type_old, const int* __restrict__ type, GroupMap gm,
-                                     int nfields, int total_tiles, int* __restrict__ same_flags,
-                                     unsigned long long* __restrict__ zmask) {
-    const long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if (e >= (long long)nfields * total_tiles) return;
-    const int f = (int)(e / total_tiles), t = (int)(e - (long long)f * total_tiles);
-    const int g = gm.fg[f];
-    if (g < 0) return;
-    const size_t k = (size_t)g * total_tiles + t;
-    if (type_old[k] != type[k]) {
-        same_flags[e] = 0;
-        if (zmask) atomicAnd(zmask + t, ~(1ull << f));
+    if (threadIdx.x == 0 && nhi) {
+        const int slot = blockIdx.x & (CLASSIFY_SLOTS - 1);
+        atomicAdd(stats + slot * STATS_STRIDE, (unsigned long long)nhi);
+        atomicAdd(stats + (CLASSIFY_SLOTS + slot) * STATS_STRIDE, (unsigned long long)nhi);
     }
 }
 
@@ -814,7 +848,7 @@ __global__ __launch_bounds__(64) void monitor_grad_wave32(StepArgs a, const Inst
                                                           const int* __restrict__ tinst,
                                                           const int* __restrict__ types, int field0,
                                                           double* __restrict__ md, unsigned long long* __restrict__ reset) {
-    if (reset && blockIdx.x == 0 && threadIdx.x == 0) *reset = 0ull;  // counter the classification adds to
+    if (blockIdx.x == 0 && threadIdx.x < CLASSIFY_SLOTS) reset[threadIdx.x * STATS_STRIDE] = 0ull;  // the classification's counters
     constexpr int TS = 32, LWD = 38, C0 = 2;
     __shared__ __align__(16) double box[(TS + 2) * LWD];
     const int lane = threadIdx.x;
@@ -970,7 +1004,7 @@ int launch_monitor(const StepArgs& a, int kind, int tile, int ngroups_eval, int 
         else if (tile == 64) hipLaunchKernelGGL((monitor_grad_kernel<64>), dim3(grid), dim3(256), 0, s, a, ngroups_eval, field0, field_stride, type_groups, md, reset);
         else return AMPS_E_UNSUPPORTED;
     } else {
-        hipLaunchKernelGGL(monitor_samples_kernel, dim3((n + 255) / 256), dim3(256), 0, s, a.inst, a.tile_inst, a.in,
+        hipLaunchKernelGGL(monitor_samples_kernel, dim3((n + 15) / 16), dim3(256), 0, s, a.inst, a.tile_inst, a.in,
                            a.total_cells, a.total_tiles, a.type, ngroups_eval, field0, field_stride, type_groups, tile,
                            kind, md, last, reset);
     }
@@ -985,13 +1019,19 @@ int launch_monitor_last_init(const StepArgs& a, int tile, int ngroups_eval, int 
     return hip_ok();
 }
 
-int launch_classify(const InstDesc* inst, const int* tile_inst, int total_tiles, int ngroups, int broadcast,
-                    int single, const double* md, double thr, int dilate, int* type_old, int* type,
-                    unsigned long long* stats, hipStream_t s) {
-    const int n = ngroups * total_tiles;
-    const int per = 1024 * CL_PT;
-    hipLaunchKernelGGL(classify_kernel, dim3(n > 0 ? (n + per - 1) / per : 1), dim3(1024), 0, s, inst, tile_inst,
-                       total_tiles, ngroups, broadcast, single, md, thr, dilate, type_old, type, stats);
+int launch_classify_convert(const InstDesc* inst, const int* tile_inst, const Buf& b, long long total_cells,
+                            int total_tiles, int broadcast, int single, const double* md, double thr, int dilate,
+                            int* type_old, int* type, const GroupMap& gm, int* same_flags, unsigned long long* stats,
+                            int tile, hipStream_t s) {
+    const int n = gm.ngroups * total_tiles;
+    int items = (n + CLASSIFY_GRID - 1) / CLASSIFY_GRID;
+    items = items < 8 ? 8 : (items > 64 ? 64 : items);
+    int grid = (n + items - 1) / items;
+    if (grid > CLASSIFY_GRID) grid = CLASSIFY_GRID;
+    if (grid < 1) grid = 1;
+    if (tile == 16) hipLaunchKernelGGL((classify_convert_kernel<16>), dim3(grid), dim3(WG), 0, s, inst, tile_inst, b, total_cells, total_tiles, broadcast, single, md, thr, dilate, type_old, type, gm, items, same_flags, stats);
+    else if (tile == 32) hipLaunchKernelGGL((classify_convert_kernel<32>), dim3(grid), dim3(WG), 0, s, inst, tile_inst, b, total_cells, total_tiles, broadcast, single, md, thr, dilate, type_old, type, gm, items, same_flags, stats);
+    else return AMPS_E_UNSUPPORTED;
     return hip_ok();
 }
 
@@ -1001,15 +1041,6 @@ int launch_gather(const InstDesc* inst, const Buf& b, long long total_cells, int
     if (tile == 16) hipLaunchKernelGGL((gather_kernel<16>), dim3(grid), dim3(256), 0, s, inst, b, total_cells, total_tiles, type, group, instid, field, dst, bad);
     else if (tile == 32) hipLaunchKernelGGL((gather_kernel<32>), dim3(grid), dim3(256), 0, s, inst, b, total_cells, total_tiles, type, group, instid, field, dst, bad);
     else return AMPS_E_UNSUPPORTED;
-    return hip_ok();
-}
-
-int launch_clear_changed(const int* type_old, const int* type, const GroupMap& gm, int nfields, int total_tiles,
-                         int* same_flags, unsigned long long* zmask, hipStream_t s) {
-    const long long n = (long long)nfields * total_tiles;
-    if (n <= 0) return AMPS_OK;
-    hipLaunchKernelGGL(clear_changed_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, type_old, type, gm,
-                       nfields, total_tiles, same_flags, zmask);
     return hip_ok();
 }
 

@@ -24,16 +24,20 @@ int launch_init(const InstDesc* inst_dev, int inst, long long ncells, int model,
                 long long total_cells, hipStream_t s);
 int launch_convert(const InstDesc* inst, const int* tile_inst, const Buf& b, long long total_cells, int total_tiles,
                    const int* type_old, const int* type, const GroupMap& gm, int mode, int tile, hipStream_t s);
-// reset (may be null) is set to 0 by the monitor kernel (the counter the
-// classification that follows adds to).
+// reset: the counters of the classification that follows (CLASSIFY_SLOTS, at
+// a stride of STATS_STRIDE), set to 0 by the monitor kernel.
 int launch_monitor(const StepArgs& a, int kind, int tile, int ngroups_eval, int field0, int field_stride,
                    int type_groups, double* md, double* last, unsigned long long* reset, hipStream_t s);
 int launch_monitor_last_init(const StepArgs& a, int tile, int ngroups_eval, int field0, int field_stride,
                              double* last, hipStream_t s);
-// single: one instance (descriptor 0 for every tile).
-int launch_classify(const InstDesc* inst, const int* tile_inst, int total_tiles, int ngroups, int broadcast,
-                    int single, const double* md, double thr, int dilate, int* type_old, int* type,
-                    unsigned long long* stats, hipStream_t s);
+// Classification and conversion of a monitor pass.  single: one instance
+// (descriptor 0 for every tile).  same_flags (may be null): one per (group,
+// tile), cleared where the type changes.  stats: the FP64 counts of all passes
+// and of the last one, CLASSIFY_SLOTS each at a stride of STATS_STRIDE.
+int launch_classify_convert(const InstDesc* inst, const int* tile_inst, const Buf& b, long long total_cells,
+                            int total_tiles, int broadcast, int single, const double* md, double thr, int dilate,
+                            int* type_old, int* type, const GroupMap& gm, int* same_flags, unsigned long long* stats,
+                            int tile, hipStream_t s);
 int launch_gather(const InstDesc* inst, const Buf& b, long long total_cells, int total_tiles, const int* type,
                   int group, int instid, int ntiles_inst, int field, double* dst, int* bad, int tile, hipStream_t s);
 int launch_nonfinite(const double* v, long long n, int* bad, hipStream_t s);
@@ -51,10 +55,6 @@ int launch_sf_step_arg(const StepArgs& a, const InstDesc& d, long long step, int
 int launch_sf_multi(const StepArgs& a, const BlockMap& bm, hipStream_t s);
 int launch_gg_multi(const StepArgs& a, const BlockMap& bm, hipStream_t s);
 int launch_sn_multi(const StepArgs& a, const BlockMap& bm, hipStream_t s);
-// same_flags[f][tile] = 0 and bit f of zmask[tile] cleared for every field f whose
-// type group changed type on the tile.
-int launch_clear_changed(const int* type_old, const int* type, const GroupMap& gm, int nfields, int total_tiles,
-                         int* same_flags, unsigned long long* zmask, hipStream_t s);
 int launch_worklist(const int* type, const int* type_old, int total_tiles, int* wl_hi, int* wl_lo, int* counts,
                     int* same_flags, hipStream_t s);
 int launch_gg_step(const StepArgs& a, int tile, bool adaptive, int grid, hipStream_t s, const hipEvent_t* ev = nullptr);
