@@ -129,6 +129,8 @@ struct StepArgs {
     int full_cap;
     unsigned long long* stats;  // [2] FP64 tiles, [3] low tiles given the full update, [4] NO_SKIP: low
                                 // tiles the flat sweep listed (summed over steps)
+    unsigned long long* spread; // one-launch step: the counters of stats [2], [3], [4], CLASSIFY_SLOTS each at
+                                // a stride of STATS_STRIDE
     const int* type;            // [group][total_tiles] (nullptr: all FP64)
     long long total_cells;
     int total_tiles;

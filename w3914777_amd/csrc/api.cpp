@@ -59,8 +59,9 @@ void set_error_text(const char* msg) { g_last_error = msg ? msg : ""; }
 // ints of the list counters: the larger of the two layouts (bulk-hold [2][8],
 // NO_SKIP [2][NSK_SEGS] at a stride of NSK_CNT_STRIDE)
 constexpr size_t FULL_CNT_INTS = 2 * (size_t)NSK_SEGS * NSK_CNT_STRIDE;
-// words of the classification's counters (all passes, the last pass)
-constexpr size_t CLS_WORDS = 2 * (size_t)CLASSIFY_SLOTS * STATS_STRIDE;
+// words of the spread counters: the classification's (all passes, the last
+// pass) and the one-launch step's three
+constexpr size_t CLS_WORDS = 5 * (size_t)CLASSIFY_SLOTS * STATS_STRIDE;
 
 struct amps_ctx {
     int model = 0, mode = 0, monitor = 0, tile = 16, every = 10, mfield = 0;
@@ -112,6 +113,7 @@ struct amps_ctx {
     int pending_adv = 0;
     bool initialised = false;
 
+    bool one_launch = false;               // snowflake low-precision step of a small grid: one launch
     BlockMap bm{};                         // PURE_FP64: several steps a launch where that is faster
     int* d_blk_inst = nullptr;
     int* d_blk_base = nullptr;
@@ -311,6 +313,22 @@ bool has_low(const amps_ctx* c) { return c->mode != AMPS_PURE_FP64; }
 bool two_sweeps(const amps_ctx* c) { return c->model == AMPS_SNOWFLAKE && has_low(c); }
 bool low_sweep_first(const amps_ctx* c) { return two_sweeps(c); }
 
+// The snowflake's low-precision step takes one launch (launch_sf_one) up to
+// this many tiles.  Measured, us per step, two launches against one (seed
+// crystal, the least and the most gain of adaptive, fixed-type and NO_SKIP
+// runs of two parameter sets):
+//   tile 16: 1024 tiles 14.6 : 8.2 and 12.4 : 7.9, 4096 11.0 : 8.6 and
+//            16.4 : 14.4, 9216 14.8 : 14.3 and 19.2 : 22.8
+//   tile 32:  256 tiles 17.1 : 8.7 and 14.2 : 9.8, 1024 15.9 : 9.8 and
+//            14.0 : 11.3, 2304 16.9 : 13.5 and 15.0 : 14.5, 4096 26.9 : 31.5
+// One launch gives every low tile four waves and the mixed sweep's LDS; two
+// finish most of them by one wave with less.  Where no tile holds (phi between
+// 0 and 1 everywhere) one launch gains more: 4096 tiles of 16^2 75.6 : 20.6.
+int one_launch_max(int tile) { return tile == 16 ? 4096 : 2048; }
+
+// Sweep timing keeps the two launches it names.
+bool one_launch(const amps_ctx* c) { return c->one_launch && !c->ktiming; }
+
 StepArgs step_args(amps_ctx* c, int from) {
     StepArgs a{};
     a.inst = c->d_desc;
@@ -329,6 +347,7 @@ StepArgs step_args(amps_ctx* c, int from) {
         a.full_cnt = c->d_full_cnt;
         a.full_cap = c->full_cap;
         a.stats = c->d_stats;
+        a.spread = c->d_cls + 2 * CLASSIFY_SLOTS * STATS_STRIDE;
     }
     if (c->model == AMPS_GRAINGROWTH && has_low(c)) a.same_flags = c->d_same_flags;
     a.type = has_low(c) ? c->d_type : nullptr;
@@ -371,7 +390,9 @@ int kev_flush(amps_ctx* c) {
 int launch_step_kernel(amps_ctx* c, const StepArgs& a, const hipEvent_t* ev = nullptr) {
     const bool adaptive = has_low(c);
     const int grid = a.grid_cap > 0 && a.grid_cap < a.nwork ? a.grid_cap : a.nwork;
-    if (c->model == AMPS_SNOWFLAKE) return launch_sf_step(a, c->tile, adaptive, c->stream, ev);
+    if (c->model == AMPS_SNOWFLAKE)
+        return adaptive && one_launch(c) ? launch_sf_one(a, c->tile, c->stream)
+                                         : launch_sf_step(a, c->tile, adaptive, c->stream, ev);
     return c->model == AMPS_GRAINGROWTH ? launch_gg_step(a, c->tile, adaptive, grid, c->stream, ev)
                                         : launch_sn_step(a, c->tile, adaptive, grid, c->stream, ev);
 }
@@ -411,7 +432,7 @@ int clear_zmasks(amps_ctx* c) {
 // type) lose their same_flags; otherwise (fields or types set from the host)
 // every tile does.
 int refresh_worklists(amps_ctx* c, bool after_monitor = false) {
-    if (c->model != AMPS_SNOWFLAKE || !has_low(c)) return AMPS_OK;
+    if (c->model != AMPS_SNOWFLAKE || !has_low(c) || one_launch(c)) return AMPS_OK;
     return launch_worklist(c->d_type, after_monitor ? c->d_type_old : nullptr, c->total_tiles, c->d_wl,
                            c->d_wl + c->total_tiles, c->d_wl_count, c->d_same_flags, c->stream);
 }
@@ -839,6 +860,9 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
         c->bm.base = c->d_blk_base;
     }
     if (e != hipSuccess) { amps_destroy(c); return fail(AMPS_E_HIP, std::string("upload: ") + hipGetErrorString(e)); }
+    // HALF2 has kernels of its own; wg_per_cu sizes the grid of the two launches
+    c->one_launch = c->model == AMPS_SNOWFLAKE && has_low(c) && !(c->flags & AMPS_FLAG_HALF2) &&
+                    cfgs[0].wg_per_cu <= 0 && c->total_tiles <= one_launch_max(c->tile);
     const char* ng = std::getenv("AMPS_NO_GRAPH");
     c->use_graph = !(ng && ng[0] == '1');
     if (cfgs[0].wg_per_cu > 0) {
@@ -1087,9 +1111,16 @@ int amps_get_info(amps_ctx* c, amps_info* info) {
     HIPCHK(hipMemcpy(st, c->d_stats, sizeof(st), hipMemcpyDeviceToHost));
     std::memset(info, 0, sizeof(*info));
     info->steps_done = c->steps_done;
-    info->fp64_tile_updates = (int64_t)st[2];
-    info->low_full_tile_updates = (int64_t)st[3];
-    info->low_listed_tile_updates = (int64_t)st[4];
+    std::vector<unsigned long long> cls(CLS_WORDS);
+    HIPCHK(hipMemcpy(cls.data(), c->d_cls, CLS_WORDS * sizeof(unsigned long long), hipMemcpyDeviceToHost));
+    const auto counted = [&](int kind) {
+        unsigned long long n = 0;
+        for (int k = 0; k < CLASSIFY_SLOTS; ++k) n += cls[(size_t)(kind * CLASSIFY_SLOTS + k) * STATS_STRIDE];
+        return n;
+    };
+    info->fp64_tile_updates = (int64_t)(st[2] + counted(2));
+    info->low_full_tile_updates = (int64_t)(st[3] + counted(3));
+    info->low_listed_tile_updates = (int64_t)(st[4] + counted(4));
     info->monitor_passes = c->monitor_passes;
     int maxt = 0;
     for (auto& d : c->desc) maxt = std::max(maxt, d.tx * d.ty);
@@ -1099,15 +1130,8 @@ int amps_get_info(amps_ctx* c, amps_info* info) {
     info->ninstances = c->ninst;
     const double denom = (double)c->ngroups * c->total_tiles;
     if (c->mode == AMPS_ADAPTIVE && c->monitor_passes > 0) {
-        std::vector<unsigned long long> cls(CLS_WORDS);
-        HIPCHK(hipMemcpy(cls.data(), c->d_cls, CLS_WORDS * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-        double all = 0.0, last = 0.0;
-        for (int k = 0; k < CLASSIFY_SLOTS; ++k) {
-            all += (double)cls[(size_t)k * STATS_STRIDE];
-            last += (double)cls[(size_t)(CLASSIFY_SLOTS + k) * STATS_STRIDE];
-        }
-        info->hi_frac_last = last / denom;
-        info->hi_frac_mean = all / (denom * c->monitor_passes);
+        info->hi_frac_last = counted(1) / denom;
+        info->hi_frac_mean = counted(0) / (denom * c->monitor_passes);
     } else {
         std::vector<int> t((size_t)c->ngroups * c->total_tiles);
         if (has_low(c)) HIPCHK(hipMemcpy(t.data(), c->d_type, t.size() * sizeof(int), hipMemcpyDeviceToHost));
@@ -1130,7 +1154,13 @@ extern "C" int amps_set_kernel_timing(amps_ctx* c, int enable) {
         c->kev_pairs.assign(512, 1);
         for (auto& e : c->kev) HIPCHK(hipEventCreate(&e));
     }
+    const bool was_one = one_launch(c);
     c->ktiming = enable != 0;
+    if (was_one && c->ktiming && c->initialised) {  // the two-launch step's lists and counters
+        HIPCHK(hipMemsetAsync(c->d_full_cnt, 0, FULL_CNT_INTS * sizeof(int), c->stream));
+        RCCHK(launch_worklist(c->d_type, nullptr, c->total_tiles, c->d_wl, c->d_wl + c->total_tiles, c->d_wl_count,
+                              nullptr, c->stream));
+    }
     c->klaunches = 0;
     c->kms = 0.0;
     c->kms_part[0] = c->kms_part[1] = 0.0;

@@ -589,6 +589,13 @@ __device__ void sf_tile_f64(SfLds<TS, double>& L, const StepArgs& a, const InstD
 // |phi(1-phi)| <= SF_NOISE_SKIP_LOW (its per-step contribution is then below
 // 2e-9).
 constexpr float SF_BULK_EPS = 1.0e-8f;
+// Orders one wave's LDS writes before its reads, without a barrier: the other
+// waves of the workgroup, if any, have left.
+__device__ __forceinline__ void one_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+}
+
 constexpr int SAME_PHI = 1, SAME_T = 2;  // same_flags bits: both buffers hold the same phi / T
 constexpr float SF_NOISE_SKIP_LOW = 1.0e-6f;
 
@@ -1137,7 +1144,7 @@ __device__ void sf_hold_tile(float* Tb, const StepArgs& a, const InstDesc& d, in
         const float sc = bd == 0 ? s1 : (bd == 1 ? s7 : (bd == 2 ? s3 : s5));
         Tb[hbox[k]] = o + __half2float(__ushort_as_half(hw[k])) * sc;
     }
-    __syncthreads();  // one wave: orders the LDS writes before the reads
+    one_wave_sync();  // the box is written
     // T' = T + dt lap T, same operand order as the full sweep's Laplacian;
     // every box read is an aligned 16-byte read: the own row as columns
     // x0-4 .. x0+R+3, the rows above and below as columns x0 .. x0+R-1
@@ -1199,7 +1206,7 @@ __device__ void sf_hold_tile(float* Tb, const StepArgs& a, const InstDesc& d, in
         }
         a.same_flags[w] = SAME_PHI;  // phi is now in both buffers
     }
-    __syncthreads();  // the box is rewritten by the next tile
+    one_wave_sync();  // the box is rewritten by the next tile
 }
 
 // Each wave takes a group of HOLD_GT list positions g, g + ngr, g + 2 ngr,
@@ -1462,48 +1469,14 @@ __global__ __launch_bounds__(256, 3) void sf_mixed_kernel(StepArgs a, const Inst
 // reads, and the tile's min/max is a wave reduction.
 constexpr int FLAT_NT = 64;
 
-template <int TS, bool MULTI>
-__global__ __launch_bounds__(FLAT_NT) void sf_flat_kernel(StepArgs a, const InstDesc* __restrict__ inst,
-                                                          const int* __restrict__ tinst, const int* __restrict__ wl,
-                                                          const int* __restrict__ wlc) {
+// A level-2 tile by one wave: T' from the T box (Tb), phi' = +0.
+template <int TS>
+__device__ void sf_flat_tile(float* Tb, const StepArgs& a, const InstDesc& d, int w, const NbCode& c, double offp,
+                             double offT) {
     using G = SfGeo<TS>;
     using GF = SfGeo<TS, FLAT_NT>;
     constexpr int H = G::H, LW = G::LW, R = G::R, NP = WG / FLAT_NT;
-    __shared__ __align__(16) float Tb[LW * LW];
-    const int b = blockIdx.x;
-    const int w = wl[b];
-    const int n = *wlc;
-    const long long step = *a.step_ctr + a.step_add;
-    if (b == 0) {
-        if (threadIdx.x == 0) a.stats[3] += (unsigned long long)n;  // low tiles of the step (one writer)
-        // the next step's counters (lane k: segment k): their last reader, the
-        // previous step's mixed sweep, has finished
-        static_assert(FLAT_NT == NSK_SEGS, "one lane per segment");
-        a.full_cnt[((int)((step + 1) & 1) * NSK_SEGS + (int)threadIdx.x) * NSK_CNT_STRIDE] = 0;
-    }
-    if (b >= n) return;
-    const InstDesc& d = inst[MULTI ? tinst[w] : 0];
-    const int tt = nb_type_lane<TS>(a, d, w);
-    NbCode c;
-    nb_code_fetch<TS>(c, a, d, w);
-    const unsigned hm = hmask_of(tt);
-    const int flat = low_flat_level(c, hm);
-    const double offp = __shfl(c.o0, 4), offT = __shfl(c.o1, 4);  // lane 4: the tile itself
-    if (flat == 3) {
-        sf_tile_zero<TS, FLAT_NT>(a, d, w, offp, offT);
-        return;
-    }
-    if (flat < 2) {
-        // segment = list position mod NSK_SEGS: at most nsk_cap entries each,
-        // and the appends spread over NSK_SEGS counters on their own lines
-        if (threadIdx.x == 0) {
-            const int seg = b & (NSK_SEGS - 1);
-            const int j = atomicAdd(a.full_cnt + ((int)(step & 1) * NSK_SEGS + seg) * NSK_CNT_STRIDE, 1);
-            a.full_seg[seg * nsk_cap(a.total_tiles) + j] = w;
-        }
-        return;
-    }
-    // level 2: the T words of the tile and of its halo (no FP64 neighbour:
+    // the T words of the tile and of its halo (no FP64 neighbour:
     // every element from the fp16 storage)
     const int lt = w - d.tile_base;
     const int tile_y = lt / d.tx, tile_x = lt - tile_y * d.tx;
@@ -1544,7 +1517,7 @@ __global__ __launch_bounds__(FLAT_NT) void sf_flat_kernel(StepArgs a, const Inst
         const unsigned short wt = (unsigned short)raw_word4(ht[k], hmap.off[k]);
         Tb[hmap.box[k]] = sf_decode_rel(o1 - offT, wt, s1);
     }
-    __syncthreads();  // the T box is in LDS
+    one_wave_sync();  // the T box is in LDS
     const float dt = d.kf[SFK_DT], kap = d.kf[SFK_KAPPA];
     float rt[NP][R];
     float mnt = INFINITY, mxt = -INFINITY;
@@ -1586,6 +1559,136 @@ __global__ __launch_bounds__(FLAT_NT) void sf_flat_kernel(StepArgs a, const Inst
         a.out.scl[a.total_tiles + w] = ct.scl;
         a.same_flags[w] = 0;
     }
+}
+
+template <int TS, bool MULTI>
+__global__ __launch_bounds__(FLAT_NT) void sf_flat_kernel(StepArgs a, const InstDesc* __restrict__ inst,
+                                                          const int* __restrict__ tinst, const int* __restrict__ wl,
+                                                          const int* __restrict__ wlc) {
+    constexpr int LW = SfGeo<TS>::LW;
+    __shared__ __align__(16) float Tb[LW * LW];
+    const int b = blockIdx.x;
+    const int w = wl[b];
+    const int n = *wlc;
+    const long long step = *a.step_ctr + a.step_add;
+    if (b == 0) {
+        if (threadIdx.x == 0) a.stats[3] += (unsigned long long)n;  // low tiles of the step (one writer)
+        // the next step's counters (lane k: segment k): their last reader, the
+        // previous step's mixed sweep, has finished
+        static_assert(FLAT_NT == NSK_SEGS, "one lane per segment");
+        a.full_cnt[((int)((step + 1) & 1) * NSK_SEGS + (int)threadIdx.x) * NSK_CNT_STRIDE] = 0;
+    }
+    if (b >= n) return;
+    const InstDesc& d = inst[MULTI ? tinst[w] : 0];
+    const int tt = nb_type_lane<TS>(a, d, w);
+    NbCode c;
+    nb_code_fetch<TS>(c, a, d, w);
+    const unsigned hm = hmask_of(tt);
+    const int flat = low_flat_level(c, hm);
+    const double offp = __shfl(c.o0, 4), offT = __shfl(c.o1, 4);  // lane 4: the tile itself
+    if (flat == 3) {
+        sf_tile_zero<TS, FLAT_NT>(a, d, w, offp, offT);
+        return;
+    }
+    if (flat < 2) {
+        // segment = list position mod NSK_SEGS: at most nsk_cap entries each,
+        // and the appends spread over NSK_SEGS counters on their own lines
+        if (threadIdx.x == 0) {
+            const int seg = b & (NSK_SEGS - 1);
+            const int j = atomicAdd(a.full_cnt + ((int)(step & 1) * NSK_SEGS + seg) * NSK_CNT_STRIDE, 1);
+            a.full_seg[seg * nsk_cap(a.total_tiles) + j] = w;
+        }
+        return;
+    }
+    sf_flat_tile<TS>(Tb, a, d, w, c, offp, offT);
+}
+
+// --------------------------------------------------- one-launch adaptive step
+// The low-precision step of a grid with few tiles in one launch, a workgroup
+// per tile: an FP64 tile by sf_tile_f64; a low tile that the first sweep of the
+// two-launch step would finish (NO_SKIP: flat levels 2 and 3; otherwise the
+// bulk hold) by wave 0 with that sweep's code, the other waves leaving; every
+// other low tile by the mixed sweep's low path.  Each tile's update reads the
+// input buffer only and runs the same code as in the two-launch step, so the
+// result is the same, bit for bit, and no work-lists are needed.
+//
+// Bound by the latency of a tile's loads, not by their number: with few tiles
+// the two launches each wait for theirs with most of the chip idle.  512^2 at
+// tile 16: the step's kernels 12.7 -> 6.4 us, 500 adaptive steps with their
+// monitor passes 7.09 -> 4.47 ms.  The lists pay again once the tiles fill the chip several times over (one_launch_max).
+template <int TS, int HH>
+union SfOneLds {
+    SfMixLds<TS> m;
+    float flat[SfGeo<TS>::LW * SfGeo<TS>::LW];
+    float hold[HoldGeo<TS, HH>::ROWS * HoldGeo<TS, HH>::LW];
+};
+
+template <int TS, int HH, bool MULTI, bool NOSKIP>
+__global__ __launch_bounds__(256, TS == 16 ? 4 : 3) void sf_one_kernel(StepArgs a, const InstDesc* __restrict__ inst,
+                                                                      const int* __restrict__ tinst) {
+    __shared__ __align__(16) SfOneLds<TS, HH> U;
+    const long long step = *a.step_ctr + a.step_add;
+    const int w = xcd_remap(blockIdx.x, a.nwork);
+    const InstDesc& d = inst[MULTI ? tinst[w] : 0];
+    const int t = nb_type_lane<TS>(a, d, w);
+    NbCode c;
+    nb_code_fetch<TS>(c, a, d, w);
+    const unsigned hmask = hmask_of(t);
+    unsigned long long* cnt = a.spread + (blockIdx.x & (CLASSIFY_SLOTS - 1)) * STATS_STRIDE;
+    constexpr int KIND = CLASSIFY_SLOTS * STATS_STRIDE;  // counters of FP64, low and listed tiles
+    if ((hmask >> 4) & 1u) {
+        if (threadIdx.x == 0) atomicAdd(cnt, 1ull);
+        const int lt = w - d.tile_base;
+        const int tile_y = lt / d.tx, tile_x = lt - tile_y * d.tx;
+        sf_tile_f64<TS, true>(U.m.h, a, d, tile_x, tile_y, hmask, step);
+        return;
+    }
+    int flat = 0;
+    if constexpr (NOSKIP) {
+        if (threadIdx.x == 0) atomicAdd(cnt + KIND, 1ull);
+        flat = low_flat_level(c, hmask);
+        if (flat >= 2) {
+            if (threadIdx.x >= FLAT_NT) return;
+            const double offp = __shfl(c.o0, 4), offT = __shfl(c.o1, 4);  // lane 4: the tile itself
+            if (flat == 3) sf_tile_zero<TS, FLAT_NT>(a, d, w, offp, offT);
+            else sf_flat_tile<TS>(U.flat, a, d, w, c, offp, offT);
+            return;
+        }
+        if (threadIdx.x == 0) atomicAdd(cnt + 2 * KIND, 1ull);
+    } else {
+        const int lane = threadIdx.x & 63;
+        HoldMeta m;
+        m.type = t;
+        m.op = c.o0;
+        m.ot = c.o1;
+        m.sp = c.s0;
+        m.st = c.s1;
+        const unsigned hb = lane < 9 ? hold_bits(m.type, m.op, m.sp) : 0u;
+        if ((__ballot(hb & 1u) & 0x1FFull) == 0x1FFull || (__ballot(hb & 2u) & 0x1FFull) == 0x1FFull) {
+            if (threadIdx.x >= 64) return;
+            const int same = a.same_flags[w];
+            // T-flat: the tile and its edge neighbours (see sf_hold_kernel)
+            const double own = __shfl(m.ot, 4, 64);
+            const unsigned long long fl = __ballot(fabs(m.ot - own) + SF_H_BOUND * (double)m.st <= SF_T_FLAT);
+            if ((fl & 0xBAull) != 0xBAull) sf_hold_tile<TS, HH>(U.hold, a, d, w, m, 0, (same & SAME_PHI) != 0);
+            else if (same != (SAME_PHI | SAME_T)) sf_flat_copy<TS, HoldGeo<TS, HH>::R>(a, d, w, same);
+            return;
+        }
+        if (threadIdx.x == 0) atomicAdd(cnt + KIND, 1ull);
+    }
+    LowFetch<TS> f;
+    low_fetch<TS>(f, a, d, w, hmask);
+    nb_code_store<TS>(U.m.l, 0, c);
+    __syncthreads();  // neighbour table visible
+    sf_tile_low<TS, NOSKIP>(U.m.l, 0, c, a, d, w, f, hmask, step, nullptr, flat);
+}
+
+template <int TS, bool MULTI, bool NOSKIP>
+static void sf_one_launch(const StepArgs& a, hipStream_t s) {
+    const dim3 g(a.nwork), b(WG);
+    // the hold reads T with the widest Laplacian's halo
+    if (a.t_halo == 2 || NOSKIP) hipLaunchKernelGGL((sf_one_kernel<TS, 2, MULTI, NOSKIP>), g, b, 0, s, a, a.inst, a.tile_inst);
+    else hipLaunchKernelGGL((sf_one_kernel<TS, 1, MULTI, NOSKIP>), g, b, 0, s, a, a.inst, a.tile_inst);
 }
 
 // ------------------------------------------------------ several FP64 steps
@@ -1840,6 +1943,21 @@ int launch_sf_step(const StepArgs& a, int tile, bool adaptive, hipStream_t s, co
     } else {
         return AMPS_E_UNSUPPORTED;
     }
+    return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;
+}
+
+int launch_sf_one(const StepArgs& a, int tile, hipStream_t s) {
+    const bool noskip = (a.flags & AMPS_FLAG_NO_SKIP) != 0, multi = a.ninst > 1;
+#define SF_ONE(TS, M, N) if (tile == TS && multi == M && noskip == N) sf_one_launch<TS, M, N>(a, s)
+    SF_ONE(16, false, false);
+    SF_ONE(16, false, true);
+    SF_ONE(16, true, false);
+    SF_ONE(16, true, true);
+    SF_ONE(32, false, false);
+    SF_ONE(32, false, true);
+    SF_ONE(32, true, false);
+    SF_ONE(32, true, true);
+#undef SF_ONE
     return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;
 }
 

@@ -48,6 +48,9 @@ int launch_advance_step(long long* step_ctr, int n, hipStream_t s);
 // start and end of the first (snowflake adaptive: the bulk-hold sweep) and,
 // for the snowflake's adaptive step only, of the second (the mixed sweep).
 int launch_sf_step(const StepArgs& a, int tile, bool adaptive, hipStream_t s, const hipEvent_t* ev = nullptr);
+// The snowflake's low-precision step in one launch (grids with few tiles; not
+// HALF2); counts its tiles in a.spread.
+int launch_sf_one(const StepArgs& a, int tile, hipStream_t s);
 // PURE_FP64 step `step` of one grid from a.in to a.out, its descriptor passed
 // by value (a.inst and a.step_ctr unused).
 int launch_sf_step_arg(const StepArgs& a, const InstDesc& d, long long step, int tile, hipStream_t s);
