@@ -122,11 +122,10 @@ struct StepArgs {
     const int* wl_low_count;
     int* same_flags;            // [total_tiles] snowflake low tiles: bit 0 both buffers hold the same phi,
                                 // bit 1 the same T (words, offset and scale)
-    int* full_seg;              // snowflake low tiles listed for the mixed sweep this step: [8][full_cap]
-                                // (bulk-hold sweep) or [NSK_SEGS][nsk_cap] (NO_SKIP flat sweep)
-    int* full_cnt;              // entries per segment by step parity: [2][8], or NO_SKIP
-                                // [2][NSK_SEGS] at a stride of NSK_CNT_STRIDE ints
-    int full_cap;
+    int* full_seg;              // snowflake low tiles listed for the mixed sweep this step:
+                                // [NSK_SEGS][nsk_cap]
+    int* full_cnt;              // entries per segment by step parity: [2][NSK_SEGS] at a stride of
+                                // NSK_CNT_STRIDE ints
     unsigned long long* stats;  // [2] FP64 tiles, [3] low tiles given the full update, [4] NO_SKIP: low
                                 // tiles the flat sweep listed (summed over steps)
     unsigned long long* spread; // one-launch step: the counters of stats [2], [3], [4], CLASSIFY_SLOTS each at
@@ -166,7 +165,7 @@ struct BlockMap {
 // serialise): STATS_STRIDE words apart.
 constexpr int STATS_STRIDE = 8, CLASSIFY_SLOTS = 64;
 
-// NO_SKIP list of the snowflake's flat sweep: NSK_SEGS segments (list
+// List of the snowflake's first sweep (hold or flat): NSK_SEGS segments (list
 // position mod NSK_SEGS) of nsk_cap(total_tiles) entries, their counters
 // NSK_CNT_STRIDE ints (256 B) apart so that the appends of one launch spread
 // over as many cache lines (one line's atomics serialise).

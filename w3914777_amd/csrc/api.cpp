@@ -56,8 +56,7 @@ namespace amps {
 void set_error_text(const char* msg) { g_last_error = msg ? msg : ""; }
 }  // namespace amps
 
-// ints of the list counters: the larger of the two layouts (bulk-hold [2][8],
-// NO_SKIP [2][NSK_SEGS] at a stride of NSK_CNT_STRIDE)
+// ints of the list counters: [2][NSK_SEGS] at a stride of NSK_CNT_STRIDE
 constexpr size_t FULL_CNT_INTS = 2 * (size_t)NSK_SEGS * NSK_CNT_STRIDE;
 // words of the spread counters: the classification's (all passes, the last
 // pass) and the one-launch step's three
@@ -102,7 +101,6 @@ struct amps_ctx {
     size_t same_flags_n = 0;
     int* d_full_seg = nullptr;             // snowflake: low tiles listed for the mixed sweep (StepArgs::full_seg)
     int* d_full_cnt = nullptr;             // their counts (StepArgs::full_cnt)
-    int full_cap = 0;
 
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -323,7 +321,8 @@ bool low_sweep_first(const amps_ctx* c) { return two_sweeps(c); }
 //            14.0 : 11.3, 2304 16.9 : 13.5 and 15.0 : 14.5, 4096 26.9 : 31.5
 // One launch gives every low tile four waves and the mixed sweep's LDS; two
 // finish most of them by one wave with less.  Where no tile holds (phi between
-// 0 and 1 everywhere) one launch gains more: 4096 tiles of 16^2 75.6 : 20.6.
+// 0 and 1 everywhere) one launch wins too: 4096 tiles of 16^2 31.2 : 20.5,
+// 2025 of 32^2 34.0 : 28.1.
 int one_launch_max(int tile) { return tile == 16 ? 4096 : 2048; }
 
 // Sweep timing keeps the two launches it names.
@@ -345,7 +344,6 @@ StepArgs step_args(amps_ctx* c, int from) {
         a.same_flags = c->d_same_flags;
         a.full_seg = c->d_full_seg;
         a.full_cnt = c->d_full_cnt;
-        a.full_cap = c->full_cap;
         a.stats = c->d_stats;
         a.spread = c->d_cls + 2 * CLASSIFY_SLOTS * STATS_STRIDE;
     }
@@ -839,8 +837,7 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     mem.ask(&c->d_wl_count, 2 * sizeof(int));
     c->same_flags_n = (size_t)(c->model == AMPS_GRAINGROWTH ? c->q : 1) * tiles;
     mem.ask(&c->d_same_flags, c->same_flags_n * sizeof(int));
-    c->full_cap = (tiles + 7) / 8;
-    mem.ask(&c->d_full_seg, std::max(8 * (size_t)c->full_cap, (size_t)NSK_SEGS * nsk_cap(tiles)) * sizeof(int));
+    mem.ask(&c->d_full_seg, (size_t)NSK_SEGS * nsk_cap(tiles) * sizeof(int));
     mem.ask(&c->d_full_cnt, FULL_CNT_INTS * sizeof(int));
     std::vector<int> blk_inst, blk_base;
     plan_multi(c, blk_inst, blk_base);

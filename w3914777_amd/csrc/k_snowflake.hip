@@ -1229,8 +1229,9 @@ __global__ __launch_bounds__(64) void sf_hold_kernel(StepArgs a, const InstDesc*
     const long long step = *a.step_ctr + a.step_add;
     // the next step appends to the other parity's segments: clear them (the
     // kernel that read them, the previous step's mixed sweep, has finished)
-    if (blockIdx.x == 0 && threadIdx.x < 8) a.full_cnt[(int)((step + 1) & 1) * 8 + threadIdx.x] = 0;
-    int* fcnt = a.full_cnt + (int)(step & 1) * 8;
+    static_assert(NSK_SEGS == 64, "one lane per segment");
+    if (blockIdx.x == 0) a.full_cnt[((int)((step + 1) & 1) * NSK_SEGS + (int)threadIdx.x) * NSK_CNT_STRIDE] = 0;
+    int* fcnt = a.full_cnt + (int)(step & 1) * NSK_SEGS * NSK_CNT_STRIDE;
     const int n = *wlc;
     const int ngr = (n + HOLD_GT - 1) / HOLD_GT;
     const int lane = threadIdx.x & 63, tj = lane / 9, tk = lane - 9 * tj;
@@ -1272,10 +1273,13 @@ __global__ __launch_bounds__(64) void sf_hold_kernel(StepArgs a, const InstDesc*
                 if ((fl & fmsk) != fmsk) sf_hold_tile<TS, H>(Tb, a, d, wt, m, 9 * j, (same & SAME_PHI) != 0);
                 else if (same != (SAME_PHI | SAME_T)) sf_flat_copy<TS, G::R>(a, d, wt, same);
             } else if (lane == 0) {
-                // for the mixed sweep; segment = list position mod 8 (at most
-                // ceil(n / 8) entries each; 8 counters spread the atomics)
-                const int seg = p & 7;
-                a.full_seg[seg * a.full_cap + atomicAdd(fcnt + seg, 1)] = wt;
+                // for the mixed sweep; segment = list position mod NSK_SEGS:
+                // at most nsk_cap entries each, and counters on their own
+                // lines, as on one line the appends of a state in which few
+                // tiles hold take turns (4096^2 at tile 16, no tile
+                // holding, 1048 -> 307 us per step; tile 32 358 -> 174)
+                const int seg = p & (NSK_SEGS - 1);
+                a.full_seg[seg * nsk_cap(a.total_tiles) + atomicAdd(fcnt + seg * NSK_CNT_STRIDE, 1)] = wt;
             }
         }
     }
@@ -1337,9 +1341,23 @@ __global__ __launch_bounds__(NT) void sf_f64_arg_kernel(StepArgs a, InstDesc d, 
     sf_tile_f64<TS, false, NT>(L, a, d, tile_x, tile_y, 0x1FFu, step);
 }
 
+// Inclusive prefix sum over the wave's lanes, by lane moves within the vector
+// unit: rows of 16 lanes by shifts, then a row's last lane added to the rows
+// after it.  (Six cross-lane permutes through the LDS unit: 0.3 us at the head
+// of every workgroup of a launch of 10 us.)
+__device__ __forceinline__ int wave_prefix(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1, zero shifted in
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // Mixed sweep of the adaptive step: the FP64 tiles (FP64 work-list) and the
-// low tiles that failed the hold sweep's bulk-hold test (its 8 segments of
-// this step's parity) are the items of one persistent launch, so the two
+// low tiles that failed the hold sweep's bulk-hold test (its NSK_SEGS segments
+// of this step's parity) are the items of one persistent launch, so the two
 // latency-bound tile chains run side by side.  Items [0, nh) are FP64 tiles
 // (work-list entry i, stored XCD-remapped by the work-list kernel), the rest
 // low tiles; the LDS is a union of the two layouts, with a barrier after
@@ -1366,35 +1384,17 @@ __global__ __launch_bounds__(256, 3) void sf_mixed_kernel(StepArgs a, const Inst
     // the index and value are clamped in case there is no such FP64 item).
     const int G = gridDim.x, T = a.total_tiles;
     const int wfirst = wl[blockIdx.x < (unsigned)T ? (int)blockIdx.x : T - 1];
-    int c0[8], c1[8];
     const int lane = threadIdx.x & 63;
-    if (NOSKIP) {
-        // lane k: segment k's count of either parity
-        c0[0] = fcnt2[lane * NSK_CNT_STRIDE];
-        c1[0] = fcnt2[(NSK_SEGS + lane) * NSK_CNT_STRIDE];
-    } else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) { c0[k] = fcnt2[k]; c1[k] = fcnt2[8 + k]; }
-    }
+    // lane k: segment k's count of either parity
+    const int ceven = fcnt2[lane * NSK_CNT_STRIDE], codd = fcnt2[(NSK_SEGS + lane) * NSK_CNT_STRIDE];
     const int nh = *wlc;
     const long long step = *a.step_ctr + a.step_add;
     const bool odd = (step & 1) != 0;
-    int cnt[8], nf = 0, sincl = 0;
-    if (NOSKIP) {
-        // inclusive prefix of the segment counts over the lanes: item j of
-        // the concatenated segments lies in the first segment whose prefix
-        // exceeds j
-        sincl = odd ? c1[0] : c0[0];
-#pragma unroll
-        for (int dlt = 1; dlt < 64; dlt <<= 1) {
-            const int t = __shfl_up(sincl, dlt);
-            if (lane >= dlt) sincl += t;
-        }
-        nf = __shfl(sincl, 63);
-    } else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) { cnt[k] = odd ? c1[k] : c0[k]; nf += cnt[k]; }
-    }
+    // inclusive prefix of the segment counts over the lanes: item j of the
+    // concatenated segments lies in the first segment whose prefix exceeds j
+    const int cnt = odd ? codd : ceven;
+    const int sincl = wave_prefix(cnt);
+    const int nf = __builtin_amdgcn_readlane(sincl, 63);
     const int n = nh + nf;
     asm volatile("" ::"s"(wfirst));  // the entry's load stays in the counts' round (not sunk into the loop)
     if (blockIdx.x == 0 && threadIdx.x == 0) {  // tile counts of the step (one writer per launch)
@@ -1411,20 +1411,10 @@ __global__ __launch_bounds__(256, 3) void sf_mixed_kernel(StepArgs a, const Inst
             const int tile_y = lt / d.tx, tile_x = lt - tile_y * d.tx;
             sf_tile_f64<TS, true>(U.h, a, d, tile_x, tile_y, hmask_of(t), step);
         } else {
-            int w;
-            if (NOSKIP) {
-                const int j = i - nh;
-                const int seg = __ffsll((long long)__ballot(sincl > j)) - 1;
-                const int excl = __shfl(sincl, seg) - __shfl(odd ? c1[0] : c0[0], seg);
-                w = fseg[seg * nsk_cap(a.total_tiles) + (j - excl)];
-            } else {
-                // entry j of the concatenated segments
-                int j = i - nh, seg = 0;
-#pragma unroll
-                for (int k = 0; k < 7; ++k)
-                    if (seg == k && j >= cnt[k]) { j -= cnt[k]; seg = k + 1; }
-                w = fseg[seg * a.full_cap + j];
-            }
+            const int j = i - nh;
+            const int seg = __ffsll((long long)__ballot(sincl > j)) - 1;
+            const int excl = __builtin_amdgcn_readlane(sincl, seg) - __builtin_amdgcn_readlane(cnt, seg);
+            const int w = fseg[seg * nsk_cap(a.total_tiles) + (j - excl)];
             const InstDesc& d = inst[MULTI ? tinst[w] : 0];
             const int t = nb_type_lane<TS>(a, d, w);
             NbCode c0;
