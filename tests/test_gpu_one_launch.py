@@ -9,13 +9,14 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 SIDES = {16: [(16, 16), (80, 48), (1024, 1024), (1024, 1040)],   # 1, 15, 4096 and 4160 tiles
-         32: [(32, 32), (96, 64), (1024, 2048), (1024, 2080)]}   # 1, 6, 2048 and 2080
+         32: [(32, 32), (96, 64), (512, 1024), (1024, 544), (1024, 2048), (1024, 2080)]}  # 1, 6, 512, 544, 2048, 2080
 
 
 def config(amps, nx, ny, tile, mode, flags, stencil):
     c = amps.Config.default(amps.SNOWFLAKE)
     c.nx, c.ny, c.tile, c.mode, c.flags, c.stencil = nx, ny, tile, mode, flags, stencil
     c.params[amps.SF["CX"]], c.params[amps.SF["CY"]], c.params[amps.SF["R2"]] = nx // 2, ny // 2, 36
+    c.params[amps.SF["ANISO"]] = 6 if stencil == amps.STENCIL_REF else 4
     return c
 
 

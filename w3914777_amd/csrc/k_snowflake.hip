@@ -91,13 +91,9 @@ __device__ inline int ring_src(int r, int o, int n, int bc) {
 
 // Phase 1 on a box of R-typed values: P = eps eps' gx, Q = eps eps' gy, E2 = eps^2
 // over the (TS+2)^2 ring box (stored as described at SfGeo::PW).
-//
-// fast: index the ring directly where no ring cell needs the zero-flux
-// mirror (a tile off the domain edge, or periodic boundaries).
 template <int TS, typename Rt, int NT = WG>
 __device__ inline void sf_phase1(const Rt* phi, Rt* P, Rt* Q, Rt* E2, const InstDesc& d, int ox, int oy,
-                                 Rt inv2dx, Rt inv2dy, Rt cth0, Rt sth0, Rt epsb, Rt epsbd, Rt mend,
-                                 bool fast = false) {
+                                 Rt inv2dx, Rt inv2dy, Rt cth0, Rt sth0, Rt epsb, Rt epsbd, Rt mend) {
     using G = SfGeo<TS>;
     // the 32^2 mixed sweep (NT = WG) is at its register limit: the path for
     // n == 4 costs it 3% whether it is taken or not
@@ -105,24 +101,6 @@ __device__ inline void sf_phase1(const Rt* phi, Rt* P, Rt* Q, Rt* E2, const Inst
     const int n = (int)d.k[SFK_ANISO_N];
     const bool edge = d.bc != AMPS_BC_PERIODIC &&
                       (ox == 0 || oy == 0 || ox + TS == d.nx || oy + TS == d.ny);
-    if (fast && !edge) {
-        // box index (ry0 + 1) LW + rx0 + 1 = e + 2 ry0 + LW + 1, ring index
-        // RB + ry0 PW + rx0 - 1 = e + 2 ry0 + RB - 1 (LW = PW = RW + 2)
-        static_assert(G::LW == G::RW + 2 && G::PW == G::RW + 2, "ring and box rows differ by 2");
-        for (int e = threadIdx.x; e < G::RW * G::RW; e += NT) {
-            const int ry0 = e / G::RW;
-            const int c = e + 2 * ry0 + G::LW + 1, o = e + 2 * ry0 + G::RB - 1;
-            Rt gx = (phi[c + 1] - phi[c - 1]) * inv2dx;
-            Rt gy = (phi[c + G::LW] - phi[c - G::LW]) * inv2dy;
-            Rt eps, epsd;
-            sf_aniso<Rt, FOUR>(gx, gy, n, cth0, sth0, epsb, epsbd, mend, eps, epsd);
-            Rt A = eps * epsd;
-            P[o] = A * gx;
-            Q[o] = A * gy;
-            E2[o] = eps * eps;
-        }
-        return;
-    }
     for (int e = threadIdx.x; e < G::RW * G::RW; e += NT) {
         const int ry0 = e / G::RW, rx0 = e - ry0 * G::RW;
         int ry = ry0, rx = rx0;
@@ -287,7 +265,7 @@ __device__ inline void sf_phase1_h2(const float* phi, float* P, float* Q, float*
     constexpr int HALF = G::RW * G::RW / 2;
     static_assert(G::LW == G::RW + 2 && G::PW == G::RW + 2, "ring and box rows differ by 2");
     if ((int)d.k[SFK_ANISO_N] != 6) {
-        sf_phase1<TS, float>(phi, P, Q, E2, d, ox, oy, inv2dx, inv2dy, cth0, sth0, epsb, epsbd, mend, false);
+        sf_phase1<TS, float>(phi, P, Q, E2, d, ox, oy, inv2dx, inv2dy, cth0, sth0, epsb, epsbd, mend);
         return;
     }
     const bool edge = d.bc != AMPS_BC_PERIODIC &&
@@ -425,59 +403,6 @@ __device__ inline void sf_halo_map(SfHalo<TS, NT>& hm, const InstDesc& d, int ox
 // group lies inside its row).  The loads go straight into the registers
 // they are decoded from, so the branch around a thread's missing element
 // needs no wait at its join.
-// Per-launch constants of a thread for the tiles of a one-instance grid that
-// need no boundary map: its halo elements relative to the tile's first cell
-// (box index, region; region -1: no element), its ring cells for phase 1
-// and, for lanes 0..8, the offset of tile neighbour k = lane in the tile
-// index.  Computing these per tile costs divisions and boundary maps that
-// an interior tile does not need.
-template <int TS>
-struct SfTileConst {
-    using G = SfGeo<TS>;
-    static constexpr int NR = (G::RW * G::RW + WG - 1) / WG;
-    int hrel[G::NHT], hbox[G::NHT], hreg[G::NHT];
-    int nbrel;
-};
-
-template <int TS>
-__device__ inline void sf_tile_const(SfTileConst<TS>& t, const InstDesc& d) {
-    using G = SfGeo<TS>;
-    constexpr int H = G::H;
-#pragma unroll
-    for (int k = 0; k < G::NHT; ++k) {
-        const int h = threadIdx.x + k * WG;
-        int bly = 0, blx = 0;
-        if (h < G::NH) halo_coord<TS>(h, bly, blx);
-        t.hrel[k] = (bly - H) * d.nx + (blx - H);
-        t.hbox[k] = bly * G::LW + blx;
-        t.hreg[k] = h < G::NH ? box_region<TS, H>(bly, blx) : -1;
-    }
-    const int kk = (threadIdx.x & 63) < 9 ? (int)(threadIdx.x & 63) : 8;
-    t.nbrel = (kk / 3 - 1) * d.tx + (kk % 3 - 1);
-}
-
-// The halo map of tile (tile_x, tile_y): from the launch constants when the
-// tile's halo needs no boundary map, else computed.
-template <int TS>
-__device__ inline void sf_halo_of(SfHalo<TS>& hm, const InstDesc& d, int tile_x, int tile_y,
-                                  const SfTileConst<TS>* tc) {
-    using G = SfGeo<TS>;
-    constexpr int H = G::H;
-    const int ox = tile_x * TS, oy = tile_y * TS;
-    const bool interior = ox >= H && oy >= H && ox + TS + H <= d.nx && oy + TS + H <= d.ny;
-    if (tc && interior) {
-        const int org = oy * d.nx + ox;
-#pragma unroll
-        for (int k = 0; k < G::NHT; ++k) {
-            hm.off[k] = tc->hreg[k] >= 0 ? org + tc->hrel[k] : -1;
-            hm.box[k] = tc->hbox[k];
-            hm.reg[k] = tc->hreg[k] >= 0 ? tc->hreg[k] : 4;
-        }
-    } else {
-        sf_halo_map<TS>(hm, d, ox, oy);
-    }
-}
-
 // phi = false: the T elements only (hp untouched).
 template <int TS, bool ADAPT, int NT = WG>
 __device__ inline void sf_halo_load(uint2* hp, uint2* ht, const StepArgs& a, const InstDesc& d,
@@ -617,6 +542,8 @@ __device__ inline void sf_store_low(__half* dst16, int gcell0, const unsigned sh
     if (R == 4) {
         *reinterpret_cast<uint2*>(dst16 + gcell0) =
             make_uint2((unsigned)w[0] | ((unsigned)w[1] << 16), (unsigned)w[2] | ((unsigned)w[3] << 16));
+    } else if (R == 2) {
+        *reinterpret_cast<unsigned*>(dst16 + gcell0) = (unsigned)w[0] | ((unsigned)w[1] << 16);
     } else {
 #pragma unroll
         for (int i = 0; i < R; ++i) dst16[gcell0 + i] = __ushort_as_half(w[i]);
@@ -626,20 +553,18 @@ __device__ inline void sf_store_low(__half* dst16, int gcell0, const unsigned sh
 // Everything a low tile needs from memory, fetched in one round: own fp16
 // words, the halo elements (each from the storage its tile's type in `hmask`
 // says is current) and the offsets/scales of the tile and its neighbours.
-template <int TS>
+template <int TS, int NT = WG>
 struct LowFetch {
-    using G = SfGeo<TS>;
+    using G = SfGeo<TS, NT>;
     unsigned short op[G::R], ot[G::R];              // own fp16 words (phi, T)
     uint2 hp[G::NHT], ht[G::NHT];                   // halo elements: FP64 bits or the fp16 word's 4-word group
     double offp, offT;
     float sclp, sclT;
 };
 
-// tc (may be null): launch constants of a one-instance grid.
-template <int TS>
-__device__ inline void low_fetch(LowFetch<TS>& f, const StepArgs& a, const InstDesc& d, int w, unsigned hmask,
-                                 const SfTileConst<TS>* tc = nullptr) {
-    using G = SfGeo<TS>;
+template <int TS, int NT = WG>
+__device__ inline void low_fetch(LowFetch<TS, NT>& f, const StepArgs& a, const InstDesc& d, int w, unsigned hmask) {
+    using G = SfGeo<TS, NT>;
     constexpr int R = G::R;
     const int lt = w - d.tile_base;
     const int tile_y = lt / d.tx, tile_x = lt - tile_y * d.tx;
@@ -653,13 +578,18 @@ __device__ inline void low_fetch(LowFetch<TS>& f, const StepArgs& a, const InstD
         const uint2 v = *reinterpret_cast<const uint2*>(hT + gcell0);
         f.op[0] = u.x & 0xFFFFu; f.op[1 % R] = u.x >> 16; f.op[2 % R] = u.y & 0xFFFFu; f.op[3 % R] = u.y >> 16;
         f.ot[0] = v.x & 0xFFFFu; f.ot[1 % R] = v.x >> 16; f.ot[2 % R] = v.y & 0xFFFFu; f.ot[3 % R] = v.y >> 16;
+    } else if (R == 2) {
+        const unsigned u = *reinterpret_cast<const unsigned*>(hphi + gcell0);
+        const unsigned v = *reinterpret_cast<const unsigned*>(hT + gcell0);
+        f.op[0] = u & 0xFFFFu; f.op[1 % R] = u >> 16;
+        f.ot[0] = v & 0xFFFFu; f.ot[1 % R] = v >> 16;
     } else {
 #pragma unroll
         for (int j = 0; j < R; ++j) { f.op[j] = hphi[gcell0 + j]; f.ot[j] = hT[gcell0 + j]; }
     }
-    SfHalo<TS> hm;
-    sf_halo_of<TS>(hm, d, tile_x, tile_y, tc);
-    sf_halo_load<TS, true>(f.hp, f.ht, a, d, hm, hmask);
+    SfHalo<TS, NT> hm;
+    sf_halo_map<TS, NT>(hm, d, ox, oy);
+    sf_halo_load<TS, true, NT>(f.hp, f.ht, a, d, hm, hmask);
     f.offp = a.in.off[w];
     f.offT = a.in.off[a.total_tiles + w];
     f.sclp = a.in.scl[w];
@@ -669,15 +599,15 @@ __device__ inline void low_fetch(LowFetch<TS>& f, const StepArgs& a, const InstD
 // LDS of the low sweep: the float boxes, the neighbour offset/scale table
 // (two slots: the next tile's is written while the current tile computes),
 // the per-wave bulk-hold flags and the min/max reduction slots.
-template <int TS>
+template <int TS, int NT = WG>
 struct SfLowLds {
     using G = SfGeo<TS>;
     float phi[G::LW * G::LW], T[G::LW * G::LW];
     float P[G::RSZ], Q[G::RSZ], E2[G::RSZ];
     double nbo[2][2][9];  // [slot][field][neighbour]
     float nbs[2][2][9];
-    unsigned hflag[WG / 64];
-    float red[4 * WG / 64];
+    unsigned hflag[NT / 64];
+    float red[4 * NT / 64];
 };
 
 // Offsets and scales of neighbour tile k = threadIdx.x (threads 0..8) of
@@ -687,13 +617,11 @@ struct NbCode {
     float s0, s1;
 };
 
-// Tile index of neighbour k = min(lane, 8) of tile w: w + the launch
-// constant for a tile off the tile grid's border (tc given), else mapped.
+// Tile index of neighbour k = min(lane, 8) of tile w.
 template <int TS>
-__device__ inline int nb_tile_of(const InstDesc& d, int w, const SfTileConst<TS>* tc) {
+__device__ inline int nb_tile_of(const InstDesc& d, int w) {
     const int lt = w - d.tile_base;
     const int tile_y = lt / d.tx, tile_x = lt - tile_y * d.tx;
-    if (tc && tile_x > 0 && tile_y > 0 && tile_x < d.tx - 1 && tile_y < d.ty - 1) return w + tc->nbrel;
     Nb nb;
     nb_setup(nb, d, tile_x, tile_y, TS);
     const int l = threadIdx.x & 63;
@@ -701,20 +629,19 @@ __device__ inline int nb_tile_of(const InstDesc& d, int w, const SfTileConst<TS>
 }
 
 template <int TS>
-__device__ inline void nb_code_fetch(NbCode& c, const StepArgs& a, const InstDesc& d, int w,
-                                     const SfTileConst<TS>* tc = nullptr) {
+__device__ inline void nb_code_fetch(NbCode& c, const StepArgs& a, const InstDesc& d, int w) {
     // every thread loads (threads 9.. repeat neighbour 8, cache hits): no
     // branch around the loads, so their wait lands where they are used
     // (threads 0..8 are lanes 0..8 of wave 0)
-    const int g = nb_tile_of<TS>(d, w, tc);
+    const int g = nb_tile_of<TS>(d, w);
     c.o0 = a.in.off[g];
     c.o1 = a.in.off[a.total_tiles + g];
     c.s0 = a.in.scl[g];
     c.s1 = a.in.scl[a.total_tiles + g];
 }
 
-template <int TS>
-__device__ inline void nb_code_store(SfLowLds<TS>& L, int slot, const NbCode& c) {
+template <int TS, int NT>
+__device__ inline void nb_code_store(SfLowLds<TS, NT>& L, int slot, const NbCode& c) {
     if (threadIdx.x < 9) {
         L.nbo[slot][0][threadIdx.x] = c.o0;
         L.nbo[slot][1][threadIdx.x] = c.o1;
@@ -790,7 +717,7 @@ __device__ inline float sf_t_flat(float t, float lt, float dt, float kap, float 
 // gradient is exactly +0, so each ring cell takes the zero-gradient values
 // (theta = 0), computed once with the operations of the loop (bitwise the
 // values it would write, signs of zero included).  Exact, not a skip.
-template <int TS, bool H2>
+template <int TS, bool H2, int NT = WG>
 __device__ inline void sf_phase1_flat(float* P, float* Q, float* E2, const InstDesc& d, float cth0, float sth0,
                                       float epsb, float epsbd, float mend) {
     using G = SfGeo<TS>;
@@ -806,7 +733,7 @@ __device__ inline void sf_phase1_flat(float* P, float* Q, float* E2, const InstD
     }
     const float A = eps * epsd;
     const float pq = A * 0.0f, e2 = eps * eps;
-    for (int e = threadIdx.x; e < G::RW * G::RW; e += WG) {
+    for (int e = threadIdx.x; e < G::RW * G::RW; e += NT) {
         const int ry0 = e / G::RW;
         const int o = e + 2 * ry0 + G::RB - 1;  // RB + ry0 PW + rx0 - 1 (PW = RW + 2)
         P[o] = pq;
@@ -826,11 +753,11 @@ __device__ inline void sf_phase1_flat(float* P, float* Q, float* E2, const InstD
 // NOSKIP: no bulk hold and no noise skip (every term of the update is
 // evaluated, as the reference's type-1 branch does); flat: the tile's
 // low_flat_level (0 or 1: level 1 takes sf_phase1_flat).
-template <int TS, bool NOSKIP, bool H2 = false>
-__device__ void sf_tile_low(SfLowLds<TS>& L, int slot, const NbCode& nxt, const StepArgs& a, const InstDesc& d,
-                            int gtile, const LowFetch<TS>& f, unsigned hmask, long long step,
-                            const SfTileConst<TS>* tcon = nullptr, int flat = 0) {
-    using G = SfGeo<TS>;
+template <int TS, bool NOSKIP, bool H2 = false, int NT = WG>
+__device__ void sf_tile_low(SfLowLds<TS, NT>& L, int slot, const NbCode& nxt, const StepArgs& a, const InstDesc& d,
+                            int gtile, const LowFetch<TS, NT>& f, unsigned hmask, long long step,
+                            int flat = 0) {
+    using G = SfGeo<TS, NT>;
     constexpr int H = G::H, LW = G::LW, R = G::R;
     const int lt = gtile - d.tile_base;
     const int tile_y = lt / d.tx, tile_x = lt - tile_y * d.tx;
@@ -845,8 +772,8 @@ __device__ void sf_tile_low(SfLowLds<TS>& L, int slot, const NbCode& nxt, const 
         pc[j] = __half2float(__ushort_as_half(f.op[j])) * sclp;
         tc[j] = __half2float(__ushort_as_half(f.ot[j])) * sclT;
     }
-    SfHalo<TS> hm;
-    sf_halo_of<TS>(hm, d, tile_x, tile_y, tcon);
+    SfHalo<TS, NT> hm;
+    sf_halo_map<TS, NT>(hm, d, ox, oy);
     const float c0 = (float)offp, c1 = (float)(1.0 - offp);
     bool near0 = true, near1 = true;
 #pragma unroll
@@ -888,16 +815,16 @@ __device__ void sf_tile_low(SfLowLds<TS>& L, int slot, const NbCode& nxt, const 
     if (!NOSKIP) {
         unsigned fl = L.hflag[0];
 #pragma unroll
-        for (int i = 1; i < WG / 64; ++i) fl &= L.hflag[i];
+        for (int i = 1; i < NT / 64; ++i) fl &= L.hflag[i];
         hold = fl != 0u;
     }
-    nb_code_store<TS>(L, slot ^ 1, nxt);
+    nb_code_store(L, slot ^ 1, nxt);
     __half* dphi = a.out.f16 + d.cell_base;
     __half* dT = a.out.f16 + a.total_cells + d.cell_base;
     if (hold) {
         // phi held (same fp16 words, offset and scale); T' = T + dt lap T
         float lt[R];
-        sf_lap<TS, float>(L.T, ly, x0, d.stencil == AMPS_STENCIL_REF, d.kf[SFK_INV_DXDY], tc, lt);
+        sf_lap<TS, float, NT>(L.T, ly, x0, d.stencil == AMPS_STENCIL_REF, d.kf[SFK_INV_DXDY], tc, lt);
         float mnt = INFINITY, mxt = -INFINITY, dmn = 0.0f, dmx = 0.0f;
 #pragma unroll
         for (int i = 0; i < R; ++i) {
@@ -905,7 +832,7 @@ __device__ void sf_tile_low(SfLowLds<TS>& L, int slot, const NbCode& nxt, const 
             mnt = fminf(mnt, tc[i]);
             mxt = fmaxf(mxt, tc[i]);
         }
-        block_minmax2(mnt, mxt, dmn, dmx, L.red);  // C
+        block_minmax2<NT>(mnt, mxt, dmn, dmx, L.red);  // C
         const TileCode ct = tile_code(mnt, mxt);
         const double offTn = offT + (double)ct.mid;
         unsigned short w[R];
@@ -924,20 +851,20 @@ __device__ void sf_tile_low(SfLowLds<TS>& L, int slot, const NbCode& nxt, const 
 
     // a phi box of exact zeros needs no ring gradients (sf_phase1_flat)
     if (NOSKIP && flat == 1)
-        sf_phase1_flat<TS, H2>(L.P, L.Q, L.E2, d, d.kf[SFK_COS_N_THETA0], d.kf[SFK_SIN_N_THETA0], d.kf[SFK_EPSB],
+        sf_phase1_flat<TS, H2, NT>(L.P, L.Q, L.E2, d, d.kf[SFK_COS_N_THETA0], d.kf[SFK_SIN_N_THETA0], d.kf[SFK_EPSB],
                                d.kf[SFK_EPSB_DELTA], d.kf[SFK_MEPSB_ANISO_DELTA]);
     else if constexpr (H2)
         sf_phase1_h2<TS>(L.phi, L.P, L.Q, L.E2, d, ox, oy, d.kf[SFK_INV_2DX], d.kf[SFK_INV_2DY],
                          d.kf[SFK_COS_N_THETA0], d.kf[SFK_SIN_N_THETA0], d.kf[SFK_EPSB], d.kf[SFK_EPSB_DELTA],
                          d.kf[SFK_MEPSB_ANISO_DELTA]);
     else
-        sf_phase1<TS, float>(L.phi, L.P, L.Q, L.E2, d, ox, oy, d.kf[SFK_INV_2DX], d.kf[SFK_INV_2DY],
+        sf_phase1<TS, float, NT>(L.phi, L.P, L.Q, L.E2, d, ox, oy, d.kf[SFK_INV_2DX], d.kf[SFK_INV_2DY],
                              d.kf[SFK_COS_N_THETA0], d.kf[SFK_SIN_N_THETA0], d.kf[SFK_EPSB], d.kf[SFK_EPSB_DELTA],
-                             d.kf[SFK_MEPSB_ANISO_DELTA], tcon != nullptr);
+                             d.kf[SFK_MEPSB_ANISO_DELTA]);
     __syncthreads();  // B
 
     float rp[R], rt[R];
-    sf_phase2<TS, float, H2>(L.phi, L.T, L.P, L.Q, L.E2, ly, x0, pc, tc, rp, rt,
+    sf_phase2<TS, float, H2, NT>(L.phi, L.T, L.P, L.Q, L.E2, ly, x0, pc, tc, rp, rt,
                          d.stencil == AMPS_STENCIL_REF, d.kf[SFK_INV_DXDY], d.kf[SFK_INV_2DX], d.kf[SFK_INV_2DY],
                          d.kf[SFK_DT_OVER_TAU], d.kf[SFK_DT], d.kf[SFK_KAPPA], d.kf[SFK_ALPHA_OVER_PI],
                          d.kf[SFK_GAMMA], (float)(d.k[SFK_TEQ] - offT), (float)offp, d.kf[SFK_NOISE],
@@ -948,7 +875,7 @@ __device__ void sf_tile_low(SfLowLds<TS>& L, int slot, const NbCode& nxt, const 
         mnp = fminf(mnp, rp[i]); mxp = fmaxf(mxp, rp[i]);
         mnt = fminf(mnt, rt[i]); mxt = fmaxf(mxt, rt[i]);
     }
-    block_minmax2(mnp, mxp, mnt, mxt, L.red);  // C
+    block_minmax2<NT>(mnp, mxp, mnt, mxt, L.red);  // C
     const TileCode cp = tile_code(mnp, mxp);
     const TileCode ct = tile_code(mnt, mxt);
     const double offpn = offp + (double)cp.mid, offTn = offT + (double)ct.mid;
@@ -1298,12 +1225,12 @@ __global__ __launch_bounds__(64) void sf_hold_kernel(StepArgs a, const InstDesc*
 // (2 elsewhere); hmask_of() turns it into the wave-uniform 9-bit mask of FP64
 // neighbours.
 template <int TS>
-__device__ inline int nb_type_lane(const StepArgs& a, const InstDesc& d, int w, const SfTileConst<TS>* tc = nullptr) {
+__device__ inline int nb_type_lane(const StepArgs& a, const InstDesc& d, int w) {
     const int lane = threadIdx.x & 63;
     if (a.type == nullptr) return 2;
     // every lane loads (lanes 9.. repeat neighbour 8): no branch around the
     // load, so its wait lands where the type is used
-    const int t = a.type[nb_tile_of<TS>(d, w, tc)];
+    const int t = a.type[nb_tile_of<TS>(d, w)];
     return lane < 9 ? t : 2;
 }
 
@@ -1362,11 +1289,12 @@ __device__ __forceinline__ int wave_prefix(int v) {
 // (work-list entry i, stored XCD-remapped by the work-list kernel), the rest
 // low tiles; the LDS is a union of the two layouts, with a barrier after
 // every item.
-template <int TS>
+template <int TS, int NT = WG>
 union SfMixLds {
     SfLds<TS, double> h;
-    SfLowLds<TS> l;
+    SfLowLds<TS, NT> l;
 };
+
 
 //
 // NOSKIP: the low items are the tiles the flat sweep (sf_flat_kernel)
@@ -1422,9 +1350,9 @@ __global__ __launch_bounds__(256, 3) void sf_mixed_kernel(StepArgs a, const Inst
             const unsigned hmask = hmask_of(t);
             LowFetch<TS> f;
             low_fetch<TS>(f, a, d, w, hmask);
-            nb_code_store<TS>(U.l, 0, c0);
+            nb_code_store(U.l, 0, c0);
             __syncthreads();  // neighbour table visible
-            sf_tile_low<TS, NOSKIP, H2>(U.l, 0, c0, a, d, w, f, hmask, step, nullptr,
+            sf_tile_low<TS, NOSKIP, H2>(U.l, 0, c0, a, d, w, f, hmask, step,
                                         NOSKIP ? low_flat_level(c0, hmask) : 0);
         }
         __syncthreads();  // the LDS union is rewritten by the next item
@@ -1606,17 +1534,24 @@ __global__ __launch_bounds__(FLAT_NT) void sf_flat_kernel(StepArgs a, const Inst
 // the two launches each wait for theirs with most of the chip idle.  512^2 at
 // tile 16: the step's kernels 12.7 -> 6.4 us, 500 adaptive steps with their
 // monitor passes 7.09 -> 4.47 ms.  The lists pay again once the tiles fill the chip several times over (one_launch_max).
-template <int TS, int HH>
+template <int TS, int HH, int NT>
 union SfOneLds {
-    SfMixLds<TS> m;
+    SfMixLds<TS, NT> m;
     float flat[SfGeo<TS>::LW * SfGeo<TS>::LW];
     float hold[HoldGeo<TS, HH>::ROWS * HoldGeo<TS, HH>::LW];
 };
 
-template <int TS, int HH, bool MULTI, bool NOSKIP>
-__global__ __launch_bounds__(256, TS == 16 ? 4 : 3) void sf_one_kernel(StepArgs a, const InstDesc* __restrict__ inst,
+// 32^2 tiles that all fit two to a CU (SF_ONE_WIDE) run with NT = 512 threads,
+// 2 cells each: 512^2 9.0 -> 8.1 us (adaptive NO_SKIP), 10.3 -> 8.5 (reference
+// physics), 9.1 -> 7.2 (all low), 704^2 9.4 -> 8.4.  At 1024 tiles, two rounds
+// of them, 256 threads at three to a CU are up to 10% faster (16.6 against
+// 17.8), and 512 threads at three to a CU spill.
+constexpr int SF_ONE_WIDE = 512;
+
+template <int TS, int HH, bool MULTI, bool NOSKIP, int NT>
+__global__ __launch_bounds__(NT, NT != WG || TS == 16 ? 4 : 3) void sf_one_kernel(StepArgs a, const InstDesc* __restrict__ inst,
                                                                       const int* __restrict__ tinst) {
-    __shared__ __align__(16) SfOneLds<TS, HH> U;
+    __shared__ __align__(16) SfOneLds<TS, HH, NT> U;
     const long long step = *a.step_ctr + a.step_add;
     const int w = xcd_remap(blockIdx.x, a.nwork);
     const InstDesc& d = inst[MULTI ? tinst[w] : 0];
@@ -1630,7 +1565,7 @@ __global__ __launch_bounds__(256, TS == 16 ? 4 : 3) void sf_one_kernel(StepArgs 
         if (threadIdx.x == 0) atomicAdd(cnt, 1ull);
         const int lt = w - d.tile_base;
         const int tile_y = lt / d.tx, tile_x = lt - tile_y * d.tx;
-        sf_tile_f64<TS, true>(U.m.h, a, d, tile_x, tile_y, hmask, step);
+        sf_tile_f64<TS, true, NT>(U.m.h, a, d, tile_x, tile_y, hmask, step);
         return;
     }
     int flat = 0;
@@ -1666,19 +1601,30 @@ __global__ __launch_bounds__(256, TS == 16 ? 4 : 3) void sf_one_kernel(StepArgs 
         }
         if (threadIdx.x == 0) atomicAdd(cnt + KIND, 1ull);
     }
-    LowFetch<TS> f;
-    low_fetch<TS>(f, a, d, w, hmask);
-    nb_code_store<TS>(U.m.l, 0, c);
+    LowFetch<TS, NT> f;
+    low_fetch<TS, NT>(f, a, d, w, hmask);
+    nb_code_store(U.m.l, 0, c);
     __syncthreads();  // neighbour table visible
-    sf_tile_low<TS, NOSKIP>(U.m.l, 0, c, a, d, w, f, hmask, step, nullptr, flat);
+    sf_tile_low<TS, NOSKIP, false, NT>(U.m.l, 0, c, a, d, w, f, hmask, step, flat);
 }
 
-template <int TS, bool MULTI, bool NOSKIP>
+template <int TS, bool MULTI, bool NOSKIP, int NT>
 static void sf_one_launch(const StepArgs& a, hipStream_t s) {
-    const dim3 g(a.nwork), b(WG);
+    const dim3 g(a.nwork), b(NT);
     // the hold reads T with the widest Laplacian's halo
-    if (a.t_halo == 2 || NOSKIP) hipLaunchKernelGGL((sf_one_kernel<TS, 2, MULTI, NOSKIP>), g, b, 0, s, a, a.inst, a.tile_inst);
-    else hipLaunchKernelGGL((sf_one_kernel<TS, 1, MULTI, NOSKIP>), g, b, 0, s, a, a.inst, a.tile_inst);
+    if (a.t_halo == 2 || NOSKIP)
+        hipLaunchKernelGGL((sf_one_kernel<TS, 2, MULTI, NOSKIP, NT>), g, b, 0, s, a, a.inst, a.tile_inst);
+    else
+        hipLaunchKernelGGL((sf_one_kernel<TS, 1, MULTI, NOSKIP, NT>), g, b, 0, s, a, a.inst, a.tile_inst);
+}
+
+template <int TS, int NT>
+static void sf_one_select(const StepArgs& a, hipStream_t s) {
+    const bool noskip = (a.flags & AMPS_FLAG_NO_SKIP) != 0, multi = a.ninst > 1;
+    if (multi && noskip) sf_one_launch<TS, true, true, NT>(a, s);
+    else if (multi) sf_one_launch<TS, true, false, NT>(a, s);
+    else if (noskip) sf_one_launch<TS, false, true, NT>(a, s);
+    else sf_one_launch<TS, false, false, NT>(a, s);
 }
 
 // ------------------------------------------------------ several FP64 steps
@@ -1937,17 +1883,9 @@ int launch_sf_step(const StepArgs& a, int tile, bool adaptive, hipStream_t s, co
 }
 
 int launch_sf_one(const StepArgs& a, int tile, hipStream_t s) {
-    const bool noskip = (a.flags & AMPS_FLAG_NO_SKIP) != 0, multi = a.ninst > 1;
-#define SF_ONE(TS, M, N) if (tile == TS && multi == M && noskip == N) sf_one_launch<TS, M, N>(a, s)
-    SF_ONE(16, false, false);
-    SF_ONE(16, false, true);
-    SF_ONE(16, true, false);
-    SF_ONE(16, true, true);
-    SF_ONE(32, false, false);
-    SF_ONE(32, false, true);
-    SF_ONE(32, true, false);
-    SF_ONE(32, true, true);
-#undef SF_ONE
+    if (tile == 16) sf_one_select<16, WG>(a, s);
+    else if (a.nwork <= SF_ONE_WIDE) sf_one_select<32, 512>(a, s);
+    else sf_one_select<32, WG>(a, s);
     return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;
 }
 

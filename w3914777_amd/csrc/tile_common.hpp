@@ -348,21 +348,28 @@ __device__ inline void block_minmax(float& mn, float& mx, float* red) {
 }
 
 // Min and max of two values over the workgroup with a single barrier; red
-// must hold 4*WG/64 floats.  No leading barrier: the caller guarantees that
+// must hold 4*NT/64 floats.  No leading barrier: the caller guarantees that
 // every thread has passed a barrier since it last read red.
+template <int NT = WG>
 __device__ inline void block_minmax2(float& mn0, float& mx0, float& mn1, float& mx1, float* red) {
-    static_assert(WG == 256, "four waves per workgroup");
     wave_minmax(mn0, mx0);
     wave_minmax(mn1, mx1);
     const int w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) *reinterpret_cast<float4*>(red + 4 * w) = make_float4(mn0, mx0, mn1, mx1);
     __syncthreads();
-    const float4 r0 = reinterpret_cast<const float4*>(red)[0], r1 = reinterpret_cast<const float4*>(red)[1];
-    const float4 r2 = reinterpret_cast<const float4*>(red)[2], r3 = reinterpret_cast<const float4*>(red)[3];
-    mn0 = fminf(fminf(r0.x, r1.x), fminf(r2.x, r3.x));
-    mx0 = fmaxf(fmaxf(r0.y, r1.y), fmaxf(r2.y, r3.y));
-    mn1 = fminf(fminf(r0.z, r1.z), fminf(r2.z, r3.z));
-    mx1 = fmaxf(fmaxf(r0.w, r1.w), fmaxf(r2.w, r3.w));
+    float4 m = reinterpret_cast<const float4*>(red)[0];
+#pragma unroll
+    for (int i = 1; i < NT / 64; ++i) {
+        const float4 r = reinterpret_cast<const float4*>(red)[i];
+        m.x = fminf(m.x, r.x);
+        m.y = fmaxf(m.y, r.y);
+        m.z = fminf(m.z, r.z);
+        m.w = fmaxf(m.w, r.w);
+    }
+    mn0 = m.x;
+    mx0 = m.y;
+    mn1 = m.z;
+    mx1 = m.w;
 }
 
 __device__ inline double block_max_d(double v, double* red) {
