@@ -607,7 +607,7 @@ struct SfLowLds {
     double nbo[2][2][9];  // [slot][field][neighbour]
     float nbs[2][2][9];
     unsigned hflag[NT / 64];
-    float red[4 * NT / 64];
+    alignas(16) float red[4 * NT / 64];
 };
 
 // Offsets and scales of neighbour tile k = threadIdx.x (threads 0..8) of

@@ -348,8 +348,8 @@ __device__ inline void block_minmax(float& mn, float& mx, float* red) {
 }
 
 // Min and max of two values over the workgroup with a single barrier; red
-// must hold 4*NT/64 floats.  No leading barrier: the caller guarantees that
-// every thread has passed a barrier since it last read red.
+// must hold 4*NT/64 floats, 16-byte aligned.  No leading barrier: the caller
+// guarantees that every thread has passed a barrier since it last read red.
 template <int NT = WG>
 __device__ inline void block_minmax2(float& mn0, float& mx0, float& mn1, float& mx1, float* red) {
     wave_minmax(mn0, mx0);
