@@ -20,7 +20,7 @@
 
 namespace amps {
 
-template <int TS, bool CONS>
+template <int TS, bool CONS, int NT = WG>
 struct SnLds {
     static constexpr int LWC = TS + 4, LWE = TS + 2, RW = TS + 2;
     double c[LWC * LWC];
@@ -30,7 +30,7 @@ struct SnLds {
     // eta bounds of a low tile (block_minmax2), read 16 bytes at a time: slow
     // where mob leaves them 8 bytes off (adaptive step, 4096^2: 157 us against
     // 141 aligned, tile 16 244 against 204)
-    alignas(16) float redf[4 * WG / 64];
+    alignas(16) float redf[4 * NT / 64];
 };
 
 // mu = B(2c + 4 sum eta^3 - 6 sum eta^2) - 2A c^2 (1-c) + 2A c (1-c)^2 -
@@ -92,12 +92,12 @@ __device__ inline int sn_box_cell(const InstDesc& d, int ox, int oy, int ly, int
 
 // Phase 1: mu (and with CONS the mobility) on the tile and its ring
 // (sintering/function.h:67-72), from the staged c and eta boxes.
-template <int TS, bool CONS>
-__device__ inline void sn_phase1(SnLds<TS, CONS>& L, const InstDesc& d, int ox, int oy) {
+template <int TS, bool CONS, int NT>
+__device__ inline void sn_phase1(SnLds<TS, CONS, NT>& L, const InstDesc& d, int ox, int oy) {
     constexpr int LWC = TS + 4, LWE = TS + 2, RW = TS + 2;
     const double inv = d.k[SNK_INV_DXDY], A2 = d.k[SNK_A2], B = d.k[SNK_B], hkc = d.k[SNK_HALF_KC];
     const bool edge = d.bc != AMPS_BC_PERIODIC && (ox == 0 || oy == 0 || ox + TS == d.nx || oy + TS == d.ny);
-    for (int e = threadIdx.x; e < RW * RW; e += WG) {
+    for (int e = threadIdx.x; e < RW * RW; e += NT) {
         int ry = e / RW, rx = e - ry * RW;
         int sy = edge ? ring_src_sn(ry, oy, d.ny, d.bc) : ry, sx = edge ? ring_src_sn(rx, ox, d.nx, d.bc) : rx;
         int cc = (sy + 1) * LWC + sx + 1;
@@ -141,8 +141,8 @@ __device__ inline void sn_update_cell(const double* U, const double* M, double c
 }
 
 // The same for tile cell (ly, lx) of the single-step sweeps.
-template <int TS, bool CONS>
-__device__ inline void sn_phase2_cell(const SnLds<TS, CONS>& L, const InstDesc& d, int ly, int lx, double& cn,
+template <int TS, bool CONS, int NT>
+__device__ inline void sn_phase2_cell(const SnLds<TS, CONS, NT>& L, const InstDesc& d, int ly, int lx, double& cn,
                                       double& n1, double& n2) {
     constexpr int LWC = TS + 4, LWE = TS + 2, RW = TS + 2;
     const int rc = (ly + 1) * RW + lx + 1, ce = (ly + 1) * LWE + lx + 1;
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(256) void sn_f64_kernel(StepArgs a, const InstDesc*
             for (int k = 0; k < NE; ++k) if (me.off[k] >= 0) { L.e1[threadIdx.x + k * WG] = v1[k]; L.e2[threadIdx.x + k * WG] = v2[k]; }
         }
         __syncthreads();
-        sn_phase1<TS, CONS>(L, d, ox, oy);
+        sn_phase1(L, d, ox, oy);
         __syncthreads();
         double* oc = a.out.f64 + d.cell_base;
         double* o1 = a.out.f64 + a.total_cells + d.cell_base;
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(256) void sn_f64_kernel(StepArgs a, const InstDesc*
             const int ly = e / TS, lx = e - ly * TS;
             const size_t g = (size_t)(oy + ly) * d.nx + ox + lx;
             double cn, n1, n2;
-            sn_phase2_cell<TS, CONS>(L, d, ly, lx, cn, n1, n2);
+            sn_phase2_cell(L, d, ly, lx, cn, n1, n2);
             oc[g] = cn;
             o1[g] = n1;
             o2[g] = n2;
@@ -229,15 +229,15 @@ __global__ __launch_bounds__(256) void sn_f64_kernel(StepArgs a, const InstDesc*
 //   the storage that type selects once it arrives (the own cells and the c
 //   ring are in flight meanwhile), then decoded in registers.
 // One barrier then separates staging from phase 1, as in the FP64 sweep.
-template <int TS, bool MULTI, bool CONS>
-__global__ __launch_bounds__(256) void sn_amp_kernel(StepArgs a, const InstDesc* __restrict__ inst,
+template <int TS, bool MULTI, bool CONS, int NT>
+__global__ __launch_bounds__(NT) void sn_amp_kernel(StepArgs a, const InstDesc* __restrict__ inst,
                                                      const int* __restrict__ tinst, const int* __restrict__ types) {
     constexpr int LWC = TS + 4, LWE = TS + 2;
-    constexpr int R = TS * TS / WG, TPR = TS / R, PER = R;
-    constexpr int RNC = LWC * LWC - TS * TS, RNE = LWE * LWE - TS * TS, KC = (RNC + WG - 1) / WG;
-    static_assert(RNE <= WG, "one eta ring element per thread");
-    static_assert(R == 1 || R == 4, "strips of 1 or 4 cells");
-    __shared__ SnLds<TS, CONS> L;
+    constexpr int R = TS * TS / NT, TPR = TS / R, PER = R;
+    constexpr int RNC = LWC * LWC - TS * TS, RNE = LWE * LWE - TS * TS, KC = (RNC + NT - 1) / NT;
+    static_assert(RNE <= NT, "one eta ring element per thread");
+    static_assert(R == 1 || R == 2 || R == 4, "strips of 1, 2 or 4 cells");
+    __shared__ SnLds<TS, CONS, NT> L;
     const int b = blockIdx.x;
     if (b >= a.nwork) return;
     const int w = xcd_remap(b, a.nwork);
@@ -281,20 +281,23 @@ __global__ __launch_bounds__(256) void sn_amp_kernel(StepArgs a, const InstDesc*
         const double2 u0 = *reinterpret_cast<const double2*>(fc + g0);
         const double2 u1 = *reinterpret_cast<const double2*>(fc + g0 + 2);
         oc[0] = u0.x; oc[1 % R] = u0.y; oc[2 % R] = u1.x; oc[3 % R] = u1.y;
+    } else if (R == 2) {
+        const double2 u0 = *reinterpret_cast<const double2*>(fc + g0);
+        oc[0] = u0.x; oc[1 % R] = u0.y;
     } else {
         oc[0] = fc[g0];
     }
     const bool own64 = ty == 2;
     uint4 p1[2], p2[2];
-    if (R == 4) {
-        // FP64: R doubles in two 16-byte loads; fp16: the aligned 8-word group,
-        // loaded twice
+    if (R >= 2) {
+        // FP64: R doubles in 16-byte loads; fp16: the aligned 8-word group,
+        // loaded as often
         const uint4* a1 = own64 ? reinterpret_cast<const uint4*>(f1 + g0) : reinterpret_cast<const uint4*>(h1 + (g0 & ~7));
         const uint4* a2 = own64 ? reinterpret_cast<const uint4*>(f2 + g0) : reinterpret_cast<const uint4*>(h2 + (g0 & ~7));
         p1[0] = a1[0];
-        p1[1] = a1[own64 ? 1 : 0];
+        p1[1] = R == 4 ? a1[own64 ? 1 : 0] : p1[0];
         p2[0] = a2[0];
-        p2[1] = a2[own64 ? 1 : 0];
+        p2[1] = R == 4 ? a2[own64 ? 1 : 0] : p2[0];
     } else {
         const uint2 u1 = *(own64 ? reinterpret_cast<const uint2*>(f1 + g0) : reinterpret_cast<const uint2*>(h1 + (g0 & ~3)));
         const uint2 u2 = *(own64 ? reinterpret_cast<const uint2*>(f2 + g0) : reinterpret_cast<const uint2*>(h2 + (g0 & ~3)));
@@ -308,7 +311,7 @@ __global__ __launch_bounds__(256) void sn_amp_kernel(StepArgs a, const InstDesc*
     int rcb[KC];
 #pragma unroll
     for (int k = 0; k < KC; ++k) {
-        const int r = threadIdx.x + k * WG;
+        const int r = threadIdx.x + k * NT;
         int bly = 0, blx = 0;
         sn_ring_coord<TS, 2>(r < RNC ? r : 0, bly, blx);
         rcb[k] = r < RNC ? bly * LWC + blx : -1;
@@ -339,8 +342,8 @@ __global__ __launch_bounds__(256) void sn_amp_kernel(StepArgs a, const InstDesc*
                 q2[j] = (j & 1) ? raw_f64(u2.z, u2.w) : raw_f64(u2.x, u2.y);
             }
         } else {
-            const uint2 w1 = R == 4 ? raw_words8(p1[0], g0) : make_uint2(p1[0].x, p1[0].y);
-            const uint2 w2 = R == 4 ? raw_words8(p2[0], g0) : make_uint2(p2[0].x, p2[0].y);
+            const uint2 w1 = R >= 2 ? raw_words8(p1[0], g0) : make_uint2(p1[0].x, p1[0].y);
+            const uint2 w2 = R >= 2 ? raw_words8(p2[0], g0) : make_uint2(p2[0].x, p2[0].y);
 #pragma unroll
             for (int j = 0; j < R; ++j) {
                 q1[j] = oo1 + (double)__half2float(__ushort_as_half((unsigned short)raw_word4(w1, g0 + j))) * (double)os1;
@@ -358,16 +361,16 @@ __global__ __launch_bounds__(256) void sn_amp_kernel(StepArgs a, const InstDesc*
         }
     }
     __syncthreads();
-    sn_phase1<TS, CONS>(L, d, ox, oy);
+    sn_phase1(L, d, ox, oy);
     __syncthreads();
     double nc[PER], n1[PER], n2[PER];
     int gc[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-        const int e = threadIdx.x + i * WG;
+        const int e = threadIdx.x + i * NT;
         const int ly = e / TS, lx = e - ly * TS;
         gc[i] = (oy + ly) * d.nx + ox + lx;
-        sn_phase2_cell<TS, CONS>(L, d, ly, lx, nc[i], n1[i], n2[i]);
+        sn_phase2_cell(L, d, ly, lx, nc[i], n1[i], n2[i]);
     }
     double* oc_ = a.out.f64 + d.cell_base;
 #pragma unroll
@@ -390,7 +393,7 @@ __global__ __launch_bounds__(256) void sn_amp_kernel(StepArgs a, const InstDesc*
         }
         float lo0 = __double2float_rd(m1), hi0 = __double2float_ru(x1);
         float lo1 = __double2float_rd(m2), hi1 = __double2float_ru(x2);
-        block_minmax2(lo0, hi0, lo1, hi1, L.redf);
+        block_minmax2<NT>(lo0, hi0, lo1, hi1, L.redf);
         for (int k = 0; k < 2; ++k) {
             const double* v = k == 0 ? n1 : n2;
             const double mn = k == 0 ? lo0 : lo1, mx = k == 0 ? hi0 : hi1;
@@ -539,14 +542,25 @@ __global__ __launch_bounds__(NT) void sn_multi_kernel(StepArgs a, const InstDesc
     sn_multi_step<BS, K, CONS, INPLACE, 0, NT>(L, a, bm, d, ox, oy, edge);
 }
 
+// One workgroup per tile.  32^2 tiles, at most one to a CU, take 512
+// threads, 2 cells each: the step then waits on a tile's own chain (512^2 8.9
+// -> 8.1 us, 256^2 8.0 -> 7.3).  400 tiles take the same time with either, and 256
+// threads are faster for more (1024^2 15.7 against 16.4 us, 4096^2 141 : 154).
+constexpr int SN_AMP_WIDE = 256;
+
+template <int TS, bool CONS, int NT>
+static void sn_amp_launch(const StepArgs& a, hipStream_t s, const hipEvent_t* ev) {
+    if (a.ninst > 1)
+        launch_sweep(sn_amp_kernel<TS, true, CONS, NT>, dim3(a.nwork), dim3(NT), s, ev, a, a.inst, a.tile_inst, a.type);
+    else
+        launch_sweep(sn_amp_kernel<TS, false, CONS, NT>, dim3(a.nwork), dim3(NT), s, ev, a, a.inst, a.tile_inst, a.type);
+}
+
 template <int TS, bool ADAPT, bool CONS>
 static void sn_launch2(const StepArgs& a, int grid, hipStream_t s, const hipEvent_t* ev) {
     if (ADAPT) {
-        // one workgroup per tile
-        if (a.ninst > 1)
-            launch_sweep(sn_amp_kernel<TS, true, CONS>, dim3(a.nwork), dim3(WG), s, ev, a, a.inst, a.tile_inst, a.type);
-        else
-            launch_sweep(sn_amp_kernel<TS, false, CONS>, dim3(a.nwork), dim3(WG), s, ev, a, a.inst, a.tile_inst, a.type);
+        if (TS == 32 && a.nwork <= SN_AMP_WIDE) sn_amp_launch<TS, CONS, TS == 32 ? 512 : WG>(a, s, ev);
+        else sn_amp_launch<TS, CONS, WG>(a, s, ev);
     } else {
         if (a.ninst > 1)
             launch_sweep(sn_f64_kernel<TS, true, CONS>, dim3(grid), dim3(WG), s, ev, a, a.inst, a.tile_inst);
