@@ -4,8 +4,9 @@
 // uneven grids of one model), all device buffers, one HIP stream and the
 // captured step graphs.  amps_step enqueues work without host
 // synchronisation: the monitor cadence, tile classification, conversion and
-// the explicit-Euler sweeps are all device work, replayed from hipGraphs in
-// blocks of one monitor period.
+// the explicit-Euler sweeps are all device work: steps one by one, several to
+// a launch (PURE_FP64), or, once a context has taken enough, as hipGraphs of
+// whole monitor periods.
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -118,7 +119,8 @@ struct amps_ctx {
 
     // graphs: one per starting buffer parity
     bool use_graph = true;
-    int graph_period = 0;
+    int graph_period = 0;                  // steps of a graph
+    int eager_steps = 0;                   // steps enqueued one by one so far, up to GRAPH_AFTER
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
 
     // adjoint tape
@@ -517,7 +519,18 @@ int enqueue_one(amps_ctx* c) {
     return tape_due(c);
 }
 
-// Capture `period` steps (monitor pass included) starting from buffer parity p.
+// Steps are enqueued one by one (3.4 us of host time each, which the shortest
+// step's 6 us on the device hide), and as graphs of GRAPH_STEPS or more once a
+// context has taken GRAPH_AFTER.  A replay leaves the device idle for 6 us, and
+// a graph of 40 steps takes some 0.2 ms to build: us per step of 500, graphs of
+// 10, 20, 40 and 80 steps, one by one:
+//   snowflake adaptive 512^2, later runs  8.0  7.6  7.4  7.3, 7.4
+//                             first run   8.2  7.9  7.8  7.9, 7.4
+//   sintering adaptive 64^2,  later runs  5.8  5.4  5.2  5.0, 6.0
+//   host time per step                    1.5  0.9  0.6  0.4, 3.4
+constexpr int GRAPH_STEPS = 40, GRAPH_AFTER = 400;
+
+// Capture graph_period steps (monitor passes included) starting from buffer parity p.
 int build_graph(amps_ctx* c, int p) {
     hipGraph_t g = nullptr;
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
@@ -869,7 +882,9 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
             cus = 256;
         c->grid_cap = cfgs[0].wg_per_cu * cus;
     }
-    c->graph_period = c->mode == AMPS_ADAPTIVE ? (c->every % 2 ? 2 * c->every : c->every) : 10;
+    // an even number of whole monitor periods, GRAPH_STEPS at least
+    const int base = c->mode == AMPS_ADAPTIVE ? (c->every % 2 ? 2 * c->every : c->every) : 2;
+    c->graph_period = (GRAPH_STEPS + base - 1) / base * base;
     *out = c;
     return AMPS_OK;
 }
@@ -949,7 +964,8 @@ int amps_step(amps_ctx* c, int nsteps) {
             // graph of these adds a gap of its own per replay
             RCCHK(enqueue_multi(c));
             left -= k;
-        } else if (graphs && left >= c->graph_period && s % c->graph_period == 0) {
+        } else if (graphs && left >= c->graph_period && c->eager_steps >= GRAPH_AFTER &&
+                   (c->mode != AMPS_ADAPTIVE || s % c->every == 0)) {
             RCCHK(flush_adv(c));
             if (!c->gexec[c->cur]) RCCHK(build_graph(c, c->cur));
             HIPCHK(hipGraphLaunch(c->gexec[c->cur], c->stream));
@@ -959,6 +975,7 @@ int amps_step(amps_ctx* c, int nsteps) {
             left -= c->graph_period;
         } else {
             RCCHK(enqueue_one(c));
+            if (c->eager_steps < GRAPH_AFTER) c->eager_steps++;
             left--;
         }
     }
