@@ -319,7 +319,7 @@ bool low_sweep_first(const amps_ctx* c) { return two_sweeps(c); }
 // runs of two parameter sets):
 //   tile 16: 1024 tiles 14.6 : 8.2 and 12.4 : 7.9, 4096 11.0 : 8.6 and
 //            16.4 : 14.4, 9216 14.8 : 14.3 and 19.2 : 22.8
-//   tile 32:  256 tiles 17.1 : 8.7 and 14.2 : 9.8, 1024 15.9 : 9.8 and
+//   tile 32:  256 tiles 17.5 : 8.3 and 14.2 : 8.5, 1024 15.9 : 9.8 and
 //            14.0 : 11.3, 2304 16.9 : 13.5 and 15.0 : 14.5, 4096 26.9 : 31.5
 // One launch gives every low tile four waves and the mixed sweep's LDS; two
 // finish most of them by one wave with less.  Where no tile holds (phi between
