@@ -7,9 +7,75 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
+from tests.launcher import Launcher  # noqa: E402
+
+# The first library that brings a HIP runtime into a process decides which one
+# libamps.so uses: torch carries its own, of another release than the one the
+# library is built against.  These files import torch when they are collected
+# and pass its streams and memory to the library, so they run in a process of
+# their own, on torch's runtime; every other test runs on the library's.
+TORCH_FIRST = {"test_gpu_noalloc_streams.py"}
+
+_launcher = None
+
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs the HIP engine)")
+
+
+def _alone(config):
+    """Only TORCH_FIRST files were asked for: this is their own process."""
+    names = {os.path.basename(str(a).split("::")[0]) for a in config.args}
+    return bool(names) and names <= TORCH_FIRST
+
+
+@pytest.hookimpl(tryfirst=True)
+def pytest_pycollect_makemodule(module_path, parent):
+    if module_path.name in TORCH_FIRST and not _alone(parent.config):
+        return OwnProcessFile.from_parent(parent, path=module_path)
+
+
+class OwnProcessFile(pytest.File):
+    def collect(self):
+        item = OwnProcessItem.from_parent(self, name="own_process")
+        item.add_marker("gpu")
+        yield item
+
+
+class OwnProcessItem(pytest.Item):
+    def runtest(self):
+        r = _launcher.run([sys.executable, "-u", "-m", "pytest", "-x", "-q", "-p", "no:cacheprovider", "-m", "gpu",
+                           str(self.path)], cwd=ROOT, timeout=110)
+        if r.returncode != 0:
+            pytest.fail(r.stdout + r.stderr, pytrace=False)
+
+    def reportinfo(self):
+        return self.path, 0, self.name
+
+
+def pytest_collection_finish(session):
+    """Start the launcher before a test loads the HIP runtime."""
+    global _launcher
+    if session.config.option.collectonly or _launcher is not None:
+        return
+    if any(isinstance(i, OwnProcessItem) or _starts_programs(i) for i in session.items):
+        _launcher = Launcher()
+
+
+def pytest_unconfigure(config):
+    if _launcher is not None:
+        _launcher.close()
+
+
+def _starts_programs(item):
+    return item.get_closest_marker("gpu") is not None and hasattr(getattr(item, "module", None), "subprocess")
+
+
+@pytest.fixture(autouse=True)
+def _programs_by_launcher(request, monkeypatch):
+    """The GPU tests' subprocess.run is the launcher's."""
+    if _launcher is not None and _starts_programs(request.node):
+        monkeypatch.setattr(request.module, "subprocess", _launcher)
 
 
 @pytest.fixture(scope="session")
