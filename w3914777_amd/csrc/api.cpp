@@ -628,9 +628,12 @@ void plan_sn(long long b16, long long b32, int cus, int& k, int& edge) {
 }
 
 // Chooses a PURE_FP64 context's steps per launch and blocks (bm.k = 0: single
-// steps only); inst and base receive the block map's tables.
+// steps only); inst and base receive the block map's tables.  wg_per_cu sizes
+// the single-step sweeps of grain growth and sintering, so a context that asks
+// for one takes those (the snowflake's FP64 sweep ignores it).
 void plan_multi(amps_ctx* c, std::vector<int>& inst, std::vector<int>& base) {
     if (c->mode != AMPS_PURE_FP64) return;
+    if (c->model != AMPS_SNOWFLAKE && c->cfg[0].wg_per_cu > 0) return;
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
