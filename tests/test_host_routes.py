@@ -35,3 +35,34 @@ for name, model, q in (("gg2", amps.GRAINGROWTH, 2), ("gg5", amps.GRAINGROWTH, 5
             assert multi and n < 16, key
         else:
             assert (multi, n) == (0, 16), key
+
+
+@pytest.mark.parametrize("ckpt", [1, 3, 8, 20])
+@pytest.mark.parametrize("model", ["SNOWFLAKE", "SINTERING"])
+def test_adjoint_fits_the_memory_of_its_states(run, model, ckpt):
+    """A taped run and its adjoint fit a device that holds the context, the
+    checkpoints, the states between two of them and two cotangents, whatever
+    the number of checkpoints (blocks of them are allocated ahead)."""
+    out = run(f"""
+cfg = amps.Config.default(amps.{model})
+cfg.nx, cfg.ny, cfg.tile = 64, 64, 16
+ids = [amps.GRAD_SF["DELTA"]] if cfg.model == amps.SNOWFLAKE else [amps.GRAD_SN["KC"]]
+import numpy as np
+F = cfg.nfields()
+for ckpts in (1, 2, 3, 4, 5, 8, 9, 16, 17):
+    with amps.Context(cfg) as c:
+        c.init()
+        base = stub.live()
+        state = F * (64 * 64 + 1056) * 8
+        steps = {ckpt} * (ckpts - 1) + ({ckpt} - 1 if {ckpt} > 1 else 0)
+        stub.limit(base + (ckpts + {ckpt} - 1 + 2) * state + 65536)
+        try:
+            c.tape_begin({ckpt})
+            c.step(steps)
+            c.adjoint([np.zeros((F, 64, 64))], ids, want_du0=True)
+            out[str(ckpts)] = "fits"
+        except amps.AmpsError as e:
+            out[str(ckpts)] = str(e)
+        stub.limit(2 ** 63)
+""")
+    assert set(out.values()) == {"fits"}, out

@@ -1240,8 +1240,8 @@ int grad_slot(int model, int id) {
     return -1;
 }
 
-// Device memory of one adjoint call, one allocation (see DeviceArena),
-// released on every exit path.
+// Device memory of one adjoint call beyond the tape's, one allocation (see
+// DeviceArena), released on every exit path.
 struct AdjMem {
     void* p = nullptr;
     ~AdjMem() {
@@ -1271,12 +1271,17 @@ extern "C" int amps_adjoint(amps_ctx* c, const double* dJ_du, const int32_t* par
     const auto seg_end = [&](int s) { return s + 1 < nseg ? c->tape_steps[s + 1] : c->steps_done; };
     long long mmax = 1;
     for (int s = 0; s < nseg; ++s) mmax = std::max(mmax, seg_end(s) - c->tape_steps[s]);
+    // Memory for the inner states of a segment, then two cotangents: the tape's
+    // checkpoints not yet taken come first, so that a recording that fits (its
+    // blocks are allocated ahead) leaves no more to ask for than its states need.
     AdjMem mem;
-    const size_t words = 2 * state + (size_t)NG * c->total_tiles + 1 + (size_t)(mmax - 1) * state;
+    const size_t need = (size_t)(mmax - 1) + 2, kept = std::min(need, c->tape_free_n);
+    const size_t words = (need - kept) * state + (size_t)NG * c->total_tiles + 1;
     if (hipMalloc(&mem.p, words * 8) != hipSuccess) return fail(AMPS_E_NOMEM, "adjoint work memory");
-    double* lam[2] = {static_cast<double*>(mem.p), static_cast<double*>(mem.p) + state};
-    double* mid = lam[1] + state;  // [mmax - 1] states
-    double* gacc = mid + (size_t)(mmax - 1) * state;
+    double* own = static_cast<double*>(mem.p);
+    const auto room = [&](size_t i) { return i < kept ? c->tape_free + i * state : own + (i - kept) * state; };
+    double* lam[2] = {room(need - 2), room(need - 1)};
+    double* gacc = own + (need - kept) * state;
     long long* dstep = reinterpret_cast<long long*>(gacc + (size_t)NG * c->total_tiles);
     // cotangent of the final state: host [inst][field][ny][nx] -> device [field][cells]
     size_t hoff = 0;
@@ -1295,7 +1300,7 @@ extern "C" int amps_adjoint(amps_ctx* c, const double* dJ_du, const int32_t* par
         if (m <= 0) continue;
         const auto at = [&](int j) -> double* {  // state j of the segment
             return j == 0 ? c->tape[s]
-                          : (j < m ? mid + (size_t)(j - 1) * state : (s + 1 < nseg ? c->tape[s + 1] : c->buf[c->cur].f64));
+                          : (j < m ? room(j - 1) : (s + 1 < nseg ? c->tape[s + 1] : c->buf[c->cur].f64));
         };
         // recompute the segment's inner states from its checkpoint
         RCCHK(launch_fill_u64((unsigned long long*)dstep, 1, (unsigned long long)S0, c->stream));
@@ -1305,7 +1310,8 @@ extern "C" int amps_adjoint(amps_ctx* c, const double* dJ_du, const int32_t* par
             a.out.f64 = at(j + 1);
             a.step_ctr = dstep;
             a.step_add = j;
-            if (c->bm.k > 1 && j + c->bm.k < m) {  // bm.k states in a row of `mid`
+            // bm.k inner states in a row
+            if (c->bm.k > 1 && j + c->bm.k < m && ((size_t)j >= kept || (size_t)(j + c->bm.k) <= kept)) {
                 RCCHK(launch_multi(c, a, state));
                 j += c->bm.k;
             } else {
