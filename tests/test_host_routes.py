@@ -66,3 +66,49 @@ for ckpts in (1, 2, 3, 4, 5, 8, 9, 16, 17):
         stub.limit(2 ** 63)
 """)
     assert set(out.values()) == {"fits"}, out
+
+
+def test_short_calls_replay_graphs_on_an_idle_stream(run):
+    """Calls of 10 to 39 steps replay graphs once the context has taken 100
+    steps, if the host waited for the stream before the call; without a wait
+    their steps are enqueued one by one, and calls of 40 and more replay the
+    long graphs after 400 steps either way."""
+    out = run("""
+def graphs(every, calls, wait):
+    cfg = amps.Config.default(amps.SINTERING)
+    cfg.nx = cfg.ny = 64
+    if every:
+        cfg.mode, cfg.monitor_every = amps.ADAPTIVE, every
+    else:
+        cfg.mode = amps.PURE_HALF2
+    res = []
+    with amps.Context(cfg) as c:
+        c.init()
+        for n in calls:
+            stub.clear()
+            c.step(n)
+            res.append(stub.log().count("graph"))
+            if wait == "sync": c.sync()
+            if wait == "get": c.get_field(0)
+    return res
+calls = [10] * 12 + [25, 39, 9]
+for every in (0, 1, 7, 10, 20, 50):
+    for wait in ("sync", "get", "none"):
+        out[f"{every} {wait}"] = graphs(every, calls, wait)
+out["long"] = graphs(10, [400, 40, 10, 80, 10], "none")
+out["long after short"] = graphs(10, [10] * 40 + [40], "sync")[-1]
+""")
+    for key, got in out.items():
+        if key == "long":
+            assert got == [0, 1, 0, 2, 0]
+        elif key == "long after short":
+            assert got == 1
+        elif key.split()[1] == "none" or key.startswith("50"):
+            assert got == [0] * 15, key
+        else:
+            # graphs hold whole monitor periods and start on a monitor step
+            every = int(key.split()[0])
+            if every in (0, 1, 10):
+                assert got == [0] * 10 + [1, 1, 2, 3, 0], (key, got)
+            else:
+                assert max(got) >= 1 and got[:10] == [0] * 10, (key, got)

@@ -117,11 +117,16 @@ struct amps_ctx {
     int* d_blk_inst = nullptr;
     int* d_blk_base = nullptr;
 
-    // graphs: one per starting buffer parity
+    // graphs: of many steps, and of few for the calls that take fewer; one
+    // per starting buffer parity
+    struct Graphs {
+        int steps = 0;
+        hipGraphExec_t exec[2] = {nullptr, nullptr};
+    };
     bool use_graph = true;
-    int graph_period = 0;                  // steps of a graph
-    int eager_steps = 0;                   // steps enqueued one by one so far, up to GRAPH_AFTER
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
+    Graphs many, few;
+    int steps_taken = 0;                   // steps enqueued outside launches of several, up to GRAPH_AFTER
+    bool idle = false;                     // nothing enqueued since the host last waited for the stream
 
     // adjoint tape
     int tape_every = 0;
@@ -371,9 +376,16 @@ StepArgs step_args(amps_ctx* c, int from) {
     return a;
 }
 
+// Waits for the context's stream.
+int sync_stream(amps_ctx* c) {
+    HIPCHK(hipStreamSynchronize(c->stream));
+    c->idle = true;
+    return AMPS_OK;
+}
+
 int kev_flush(amps_ctx* c) {
     if (c->kev_used == 0) return AMPS_OK;
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     for (int i = 0; i < c->kev_used; ++i) {
         float a = 0.0f, b = 0.0f;
         HIPCHK(hipEventElapsedTime(&a, c->kev[4 * i], c->kev[4 * i + 1]));
@@ -528,24 +540,43 @@ int enqueue_one(amps_ctx* c) {
 //                             first run   8.2  7.9  7.8  7.9, 7.4
 //   sintering adaptive 64^2,  later runs  5.8  5.4  5.2  5.0, 6.0
 //   host time per step                    1.5  0.9  0.6  0.4, 3.4
-constexpr int GRAPH_STEPS = 40, GRAPH_AFTER = 400;
+//
+// A call of fewer steps replays graphs of GRAPH_FEW or more if the host has
+// waited for the stream since the last call: nothing runs that would hide the
+// enqueueing then.  us per step, calls of 10 steps with amps_sync after each,
+// one by one : graphs, and without a wait between calls:
+//   grain growth adaptive 64^2, q = 2  10.3 : 8.4   7.4 : 7.4
+//   sintering adaptive 64^2             8.6 : 7.2   6.0 : 6.1
+//   snowflake adaptive 64^2             9.1 : 8.3   6.9 : 7.3
+//   snowflake adaptive 512^2           10.3 : 9.7   8.1 : 8.6
+//   grain growth FP64 64^2, q = 8       8.6 : 8.1   6.7 : 6.9
+// Without waits a graph would only save host time (2 us a step instead of 4).
+// Its building takes 50 to 120 us and a replay saves 3 to 20.
+constexpr int GRAPH_STEPS = 40, GRAPH_AFTER = 400, GRAPH_FEW = 10, GRAPH_FEW_AFTER = 100;
 
-// Capture graph_period steps (monitor passes included) starting from buffer parity p.
-int build_graph(amps_ctx* c, int p) {
+// The graphs a call of nsteps steps replays (nullptr: none yet).
+amps_ctx::Graphs* call_graphs(amps_ctx* c, int nsteps) {
+    if (!c->use_graph || c->taping || c->ktiming) return nullptr;
+    if (nsteps >= c->many.steps) return &c->many;
+    return c->idle && c->steps_taken >= GRAPH_FEW_AFTER ? &c->few : nullptr;
+}
+
+// Capture g's steps (monitor passes included) starting from buffer parity p.
+int build_graph(amps_ctx* c, amps_ctx::Graphs& gs, int p) {
     hipGraph_t g = nullptr;
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int b = p;
     int rc = AMPS_OK;
-    for (int k = 0; k < c->graph_period && rc == AMPS_OK; ++k) {
+    for (int k = 0; k < gs.steps && rc == AMPS_OK; ++k) {
         if (c->mode == AMPS_ADAPTIVE && k % c->every == 0) rc = enqueue_monitor(c, b);
         if (rc == AMPS_OK) rc = enqueue_step(c, b, k, true);
         b ^= 1;
     }
-    if (rc == AMPS_OK) rc = launch_advance_step(c->d_step, c->graph_period, c->stream);
+    if (rc == AMPS_OK) rc = launch_advance_step(c->d_step, gs.steps, c->stream);
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (rc != AMPS_OK) { if (g) (void)hipGraphDestroy(g); return rc; }
     if (e != hipSuccess) return fail(AMPS_E_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-    e = hipGraphInstantiate(&c->gexec[p], g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(&gs.exec[p], g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     if (e != hipSuccess) return fail(AMPS_E_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
     return AMPS_OK;
@@ -885,9 +916,10 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
             cus = 256;
         c->grid_cap = cfgs[0].wg_per_cu * cus;
     }
-    // an even number of whole monitor periods, GRAPH_STEPS at least
+    // even numbers of whole monitor periods
     const int base = c->mode == AMPS_ADAPTIVE ? (c->every % 2 ? 2 * c->every : c->every) : 2;
-    c->graph_period = (GRAPH_STEPS + base - 1) / base * base;
+    c->many.steps = (GRAPH_STEPS + base - 1) / base * base;
+    c->few.steps = (GRAPH_FEW + base - 1) / base * base;
     *out = c;
     return AMPS_OK;
 }
@@ -899,8 +931,8 @@ void amps_destroy(amps_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     tape_clear(c);
     for (hipEvent_t e : c->kev) (void)hipEventDestroy(e);
-    for (int p = 0; p < 2; ++p)
-        if (c->gexec[p]) (void)hipGraphExecDestroy(c->gexec[p]);
+    for (hipGraphExec_t g : {c->many.exec[0], c->many.exec[1], c->few.exec[0], c->few.exec[1]})
+        if (g) (void)hipGraphExecDestroy(g);
     if (c->memory) (void)hipFree(c->memory);
     if (c->bad) (void)hipHostFree(c->bad);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -911,7 +943,7 @@ void amps_destroy(amps_ctx* c) {
 
 int amps_init(amps_ctx* c) {
     if (!c) return fail(AMPS_E_ARG, "ctx is NULL");
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     tape_clear(c);
     c->cur = 0;
     for (int i = 0; i < c->ninst; ++i)
@@ -940,7 +972,7 @@ int amps_init(amps_ctx* c) {
     }
     RCCHK(refresh_aux(c, 0));
     RCCHK(refresh_worklists(c));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     c->steps_done = 0;
     c->monitor_passes = 0;
     c->pending_adv = 0;
@@ -959,7 +991,8 @@ int amps_step(amps_ctx* c, int nsteps) {
         c->timing_open = true;
     }
     int left = nsteps;
-    const bool graphs = c->use_graph && !c->taping && !c->ktiming;
+    amps_ctx::Graphs* g = call_graphs(c, nsteps);
+    c->idle = false;
     while (left > 0) {
         const long long s = c->steps_done;
         if (const int k = multi_steps(c, left)) {
@@ -967,18 +1000,19 @@ int amps_step(amps_ctx* c, int nsteps) {
             // graph of these adds a gap of its own per replay
             RCCHK(enqueue_multi(c));
             left -= k;
-        } else if (graphs && left >= c->graph_period && c->eager_steps >= GRAPH_AFTER &&
+        } else if (g && left >= g->steps && (g == &c->few || c->steps_taken >= GRAPH_AFTER) &&
                    (c->mode != AMPS_ADAPTIVE || s % c->every == 0)) {
             RCCHK(flush_adv(c));
-            if (!c->gexec[c->cur]) RCCHK(build_graph(c, c->cur));
-            HIPCHK(hipGraphLaunch(c->gexec[c->cur], c->stream));
-            // graph_period is even: the buffer parity is unchanged
-            c->steps_done += c->graph_period;
-            if (c->mode == AMPS_ADAPTIVE) c->monitor_passes += c->graph_period / c->every;
-            left -= c->graph_period;
+            if (!g->exec[c->cur]) RCCHK(build_graph(c, *g, c->cur));
+            HIPCHK(hipGraphLaunch(g->exec[c->cur], c->stream));
+            // an even number of steps: the buffer parity is unchanged
+            c->steps_done += g->steps;
+            if (c->mode == AMPS_ADAPTIVE) c->monitor_passes += g->steps / c->every;
+            left -= g->steps;
+            c->steps_taken = std::min(c->steps_taken + g->steps, GRAPH_AFTER);
         } else {
             RCCHK(enqueue_one(c));
-            if (c->eager_steps < GRAPH_AFTER) c->eager_steps++;
+            if (c->steps_taken < GRAPH_AFTER) c->steps_taken++;
             left--;
         }
     }
@@ -989,7 +1023,7 @@ int amps_step(amps_ctx* c, int nsteps) {
 
 int amps_sync(amps_ctx* c, double* elapsed_ms) {
     if (!c) return fail(AMPS_E_ARG, "ctx is NULL");
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     if (elapsed_ms) *elapsed_ms = 0.0;
     if (c->timing_open) {
         float ms = 0.0f;
@@ -1005,7 +1039,7 @@ int amps_monitor_now(amps_ctx* c) {
     if (c->mode != AMPS_ADAPTIVE) return fail(AMPS_E_STATE, "monitor passes need ADAPTIVE mode");
     RCCHK(enqueue_monitor(c, c->cur));
     c->monitor_passes++;
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     return AMPS_OK;
 }
 
@@ -1029,7 +1063,7 @@ int amps_get_field(amps_ctx* c, int inst, int field, double* dst, size_t n) {
         RCCHK(launch_nonfinite(src, (long long)n, c->d_bad, c->stream));
     }
     HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     if (*(volatile int*)c->bad) return fail(AMPS_E_NONFINITE, "field " + std::to_string(field) + " holds non-finite values");
     return AMPS_OK;
 }
@@ -1052,7 +1086,7 @@ int amps_set_field(amps_ctx* c, int inst, int field, const double* src, size_t n
     RCCHK(refresh_worklists(c));  // the other buffer no longer holds the same fields
     HIPCHK(hipMemsetAsync(c->d_same_flags, 0, c->same_flags_n * sizeof(int), c->stream));
     RCCHK(clear_zmasks(c));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     return AMPS_OK;
 }
 
@@ -1062,7 +1096,7 @@ int amps_get_tile_types(amps_ctx* c, int inst, int32_t* dst, size_t n) {
     const InstDesc& d = c->desc[inst];
     const size_t nt = (size_t)d.tx * d.ty;
     if (n != nt * c->ngroups) return fail(AMPS_E_ARG, "n must equal tiles * type_groups");
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     for (int g = 0; g < c->ngroups; ++g)
         HIPCHK(hipMemcpy(dst + g * nt, c->d_type + (size_t)g * c->total_tiles + d.tile_base, nt * sizeof(int),
                          hipMemcpyDeviceToHost));
@@ -1078,7 +1112,7 @@ int amps_set_tile_types(amps_ctx* c, int inst, const int32_t* src, size_t n) {
     if (n != nt * c->ngroups) return fail(AMPS_E_ARG, "n must equal tiles * type_groups");
     for (size_t i = 0; i < n; ++i)
         if (src[i] != 1 && src[i] != 2) return fail(AMPS_E_ARG, "tile types must be 1 or 2");
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     HIPCHK(hipMemcpy(c->d_type_old, c->d_type, (size_t)c->ngroups * c->total_tiles * sizeof(int), hipMemcpyDeviceToDevice));
     for (int g = 0; g < c->ngroups; ++g)
         HIPCHK(hipMemcpy(c->d_type + (size_t)g * c->total_tiles + d.tile_base, src + g * nt, nt * sizeof(int),
@@ -1089,7 +1123,7 @@ int amps_set_tile_types(amps_ctx* c, int inst, const int32_t* src, size_t n) {
     RCCHK(refresh_worklists(c));
     HIPCHK(hipMemsetAsync(c->d_same_flags, 0, c->same_flags_n * sizeof(int), c->stream));
     RCCHK(clear_zmasks(c));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     return AMPS_OK;
 }
 
@@ -1099,7 +1133,7 @@ int amps_get_monitor_values(amps_ctx* c, int inst, double* dst, size_t n) {
     const InstDesc& d = c->desc[inst];
     const size_t nt = (size_t)d.tx * d.ty;
     if (n != nt * c->ngroups) return fail(AMPS_E_ARG, "n must equal tiles * type_groups");
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     for (int g = 0; g < c->ngroups; ++g)
         HIPCHK(hipMemcpy(dst + g * nt, c->d_md + (size_t)g * c->total_tiles + d.tile_base, nt * sizeof(double),
                          hipMemcpyDeviceToHost));
@@ -1113,7 +1147,7 @@ int amps_get_raw_field(amps_ctx* c, int inst, int field, uint16_t* words, size_t
     if (!has_low(c) || c->gm.fg[field] < 0) return fail(AMPS_E_STATE, "the field has no low-precision storage");
     const InstDesc& d = c->desc[inst];
     if (n != (size_t)d.nx * d.ny || ntiles != (size_t)d.tx * d.ty) return fail(AMPS_E_ARG, "n or ntiles does not match the instance");
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     const Buf& b = c->buf[c->cur];
     HIPCHK(hipMemcpy(words, b.f16 + (size_t)field * c->total_cells + d.cell_base, n * sizeof(uint16_t), hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(off, b.off + (size_t)field * c->total_tiles + d.tile_base, ntiles * sizeof(double), hipMemcpyDeviceToHost));
@@ -1123,7 +1157,7 @@ int amps_get_raw_field(amps_ctx* c, int inst, int field, uint16_t* words, size_t
 
 int amps_get_info(amps_ctx* c, amps_info* info) {
     if (!c || !info) return fail(AMPS_E_ARG, "NULL argument");
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     unsigned long long st[8];
     HIPCHK(hipMemcpy(st, c->d_stats, sizeof(st), hipMemcpyDeviceToHost));
     std::memset(info, 0, sizeof(*info));
@@ -1349,7 +1383,7 @@ extern "C" int amps_adjoint(amps_ctx* c, const double* dJ_du, const int32_t* par
                                       c->stream));
         }
     }
-    HIPCHK(hipStreamSynchronize(c->stream));
+    RCCHK(sync_stream(c));
     for (int i = 0; i < c->ninst; ++i) {
         const InstDesc& d = c->desc[i];
         const int nt = d.tx * d.ty;
