@@ -112,3 +112,27 @@ out["long after short"] = graphs(10, [10] * 40 + [40], "sync")[-1]
                 assert got == [0] * 10 + [1, 1, 2, 3, 0], (key, got)
             else:
                 assert max(got) >= 1 and got[:10] == [0] * 10, (key, got)
+
+
+def test_block_tables_only_for_batches(run):
+    """The map from blocks to instances of the launches of several steps exists
+    for batches only: one grid takes the same memory without such launches."""
+    out = run("""
+def live(model, n, wg):
+    cfgs = []
+    for k in range(n):
+        cfg = amps.Config.default(model)
+        cfg.nx, cfg.ny, cfg.wg_per_cu = 512, 512 + 32 * k, wg
+        cfgs.append(cfg)
+    with amps.Context(cfgs) as c:
+        c.init()
+        stub.clear()
+        c.step(12)
+        return stub.live(), any("multi" in k for k in stub.log())
+for name, model in (("gg", amps.GRAINGROWTH), ("sn", amps.SINTERING)):
+    for n in (1, 3):
+        out[f"{name} {n}"] = [live(model, n, 0), live(model, n, 1)]
+""")
+    for key, ((with_multi, used), (without, unused)) in out.items():
+        assert used and not unused, key
+        assert (with_multi > without) == (key[-1] == "3"), key

@@ -149,8 +149,8 @@ struct StepArgs {
 
 // Plan of a PURE_FP64 context's multi-step launches: k steps (0: single steps
 // only) on square blocks whose edge (16 or 32) divides every instance's
-// sides; block b of the launch belongs to instance inst[b], whose blocks
-// start at base[instance].
+// sides; block b of a batch's launch belongs to instance inst[b], whose blocks
+// start at base[instance] (both null for one instance).
 struct BlockMap {
     int k;
     int edge;

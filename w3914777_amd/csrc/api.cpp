@@ -659,7 +659,7 @@ void plan_sn(long long b16, long long b32, int cus, int& k, int& edge) {
 }
 
 // Chooses a PURE_FP64 context's steps per launch and blocks (bm.k = 0: single
-// steps only); inst and base receive the block map's tables.  wg_per_cu sizes
+// steps only); inst and base receive a batch's block tables.  wg_per_cu sizes
 // the single-step sweeps of grain growth and sintering, so a context that asks
 // for one takes those (the snowflake's FP64 sweep ignores it).
 void plan_multi(amps_ctx* c, std::vector<int>& inst, std::vector<int>& base) {
@@ -675,11 +675,12 @@ void plan_multi(amps_ctx* c, std::vector<int>& inst, std::vector<int>& base) {
     else if (c->model == AMPS_GRAINGROWTH) plan_gg(c->q, b16, b32, cus, k, edge);
     else plan_sn(b16, b32, cus, k, edge);
     if (k == 0) return;
+    c->bm = BlockMap{k, edge, (int)(edge == 16 ? b16 : b32), nullptr, nullptr, 0};
+    if (c->ninst == 1) return;  // every block is instance 0's
     for (int i = 0; i < c->ninst; ++i) {
         base.push_back((int)inst.size());
         inst.insert(inst.end(), (size_t)(c->desc[i].nx / edge) * (c->desc[i].ny / edge), i);
     }
-    c->bm = BlockMap{k, edge, (int)inst.size(), nullptr, nullptr, 0};
 }
 }  // namespace
 
@@ -888,7 +889,7 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     mem.ask(&c->d_full_cnt, FULL_CNT_INTS * sizeof(int));
     std::vector<int> blk_inst, blk_base;
     plan_multi(c, blk_inst, blk_base);
-    if (c->bm.k > 0) {
+    if (!blk_inst.empty()) {
         mem.ask(&c->d_blk_inst, blk_inst.size() * sizeof(int));
         mem.ask(&c->d_blk_base, blk_base.size() * sizeof(int));
     }
@@ -896,7 +897,7 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     if (rc != AMPS_OK) { std::string m = g_last_error; amps_destroy(c); return fail(rc, m); }
     e = hipMemcpy(c->d_desc, c->desc.data(), sizeof(InstDesc) * n, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->d_tile_inst, c->tile_inst.data(), sizeof(int) * tiles, hipMemcpyHostToDevice);
-    if (e == hipSuccess && c->bm.k > 0) {
+    if (e == hipSuccess && !blk_inst.empty()) {
         e = hipMemcpy(c->d_blk_inst, blk_inst.data(), blk_inst.size() * sizeof(int), hipMemcpyHostToDevice);
         if (e == hipSuccess)
             e = hipMemcpy(c->d_blk_base, blk_base.data(), blk_base.size() * sizeof(int), hipMemcpyHostToDevice);
