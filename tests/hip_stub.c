@@ -1,7 +1,7 @@
 /* A HIP runtime without a GPU, for CPU tests of the host code of libamps.so:
  * device memory is host memory, counted and limited; kernels are not run but
- * named, in the order of their launches, in a log; streams, events and graphs
- * are empty shells.  Loaded before libamps.so it takes libamdhip64.so.7's place
+ * named in a log, with the copies, memsets and frees, in the order of the
+ * calls; streams, events and graphs are empty shells.  Loaded before libamps.so it takes libamdhip64.so.7's place
  * (same SONAME and symbol versions). */
 #include <stdint.h>
 #include <stdio.h>
@@ -53,6 +53,7 @@ int hipMalloc(void** p, size_t bytes) {
 }
 int hipFree(void* p) {
     if (!p) return OK;
+    note("free");
     Head* h = (Head*)((char*)p - 256);
     live -= h->bytes;
     free(h);
@@ -61,9 +62,9 @@ int hipFree(void* p) {
 int hipHostMalloc(void** p, size_t bytes, unsigned flags) { (void)flags; *p = calloc(1, bytes); return OK; }
 int hipHostFree(void* p) { free(p); return OK; }
 int hipHostGetDevicePointer(void** d, void* h, unsigned flags) { (void)flags; *d = h; return OK; }
-int hipMemcpy(void* d, const void* s, size_t n, int kind) { (void)kind; memcpy(d, s, n); return OK; }
+int hipMemcpy(void* d, const void* s, size_t n, int kind) { (void)kind; note("copy"); memcpy(d, s, n); return OK; }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void* st) { (void)st; return hipMemcpy(d, s, n, kind); }
-int hipMemset(void* d, int v, size_t n) { memset(d, v, n); return OK; }
+int hipMemset(void* d, int v, size_t n) { note("memset"); memset(d, v, n); return OK; }
 int hipMemsetAsync(void* d, int v, size_t n, void* st) { (void)st; return hipMemset(d, v, n); }
 
 /* ---- kernels */

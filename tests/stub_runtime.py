@@ -1,8 +1,8 @@
 """Runs a script in a process whose libamps.so is bound to tests/hip_stub.c in
 place of the HIP runtime: kernels are logged, not run.  The script finds
 `amps` (the package), `stub` (live(), peak(), limit(bytes), clear() and
-log(): the kernels launched, "graph" for a replayed graph, a leading + while a
-graph is captured) and `out`, a dict that comes back."""
+log(): the kernels launched, "graph" for a replayed graph, "copy", "memset" and
+"free", a leading + while a graph is captured) and `out`, a dict that comes back."""
 import json
 import os
 import re

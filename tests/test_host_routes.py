@@ -136,3 +136,25 @@ for name, model in (("gg", amps.GRAINGROWTH), ("sn", amps.SINTERING)):
     for key, ((with_multi, used), (without, unused)) in out.items():
         assert used and not unused, key
         assert (with_multi > without) == (key[-1] == "3"), key
+
+
+def test_info_and_init_take_few_runtime_calls(run):
+    """amps_get_info of an adaptive context is one kernel that writes the sums
+    to host memory (a copy of the spread counters took twice as long); amps_init
+    clears all counters with one memset."""
+    out = run("""
+for name, model in (("sf", amps.SNOWFLAKE), ("gg", amps.GRAINGROWTH), ("sn", amps.SINTERING)):
+    cfg = amps.Config.default(model)
+    cfg.nx = cfg.ny = 64
+    cfg.mode = amps.ADAPTIVE
+    with amps.Context(cfg) as c:
+        c.init()
+        stub.clear(); c.init()
+        init = [k for k in stub.log() if k in ("copy", "memset")]
+        c.step(1); c.info()
+        stub.clear(); c.info()
+        out[name] = [len(init), stub.log()]
+""")
+    for name, (init, info) in out.items():
+        assert init <= (8 if name == "gg" else 6), (name, init)  # gg: two zero masks
+        assert len(info) == 1 and "counters" in info[0], (name, info)

@@ -61,7 +61,13 @@ void set_error_text(const char* msg) { g_last_error = msg ? msg : ""; }
 constexpr size_t FULL_CNT_INTS = 2 * (size_t)NSK_SEGS * NSK_CNT_STRIDE;
 // words of the spread counters: the classification's (all passes, the last
 // pass) and the one-launch step's three
-constexpr size_t CLS_WORDS = 5 * (size_t)CLASSIFY_SLOTS * STATS_STRIDE;
+constexpr size_t STATS_WORDS = 32, CLS_WORDS = 5 * (size_t)CLASSIFY_SLOTS * STATS_STRIDE;
+
+// Words of a context in host memory that kernels write.
+struct HostWords {
+    unsigned long long counted[5];  // amps_get_info: launch_counters
+    int bad;                        // amps_get_field: a value is not finite
+};
 
 struct amps_ctx {
     int model = 0, mode = 0, monitor = 0, tile = 16, every = 10, mfield = 0;
@@ -93,8 +99,8 @@ struct amps_ctx {
     long long* d_step = nullptr;
     double* d_aux[2] = {nullptr, nullptr};
     double* d_scratch = nullptr;           // max instance cells (decoded field of amps_get_field)
-    int* bad = nullptr;                    // host word the read-back kernels set on a non-finite value
-    int* d_bad = nullptr;                  // its device address
+    HostWords* host = nullptr;             // what kernels write to host memory (allocated at first use)
+    HostWords* d_host = nullptr;           // its device address
     int* d_wl = nullptr;                   // [2][total_tiles]: FP64 and low tile work-lists
     int* d_wl_count = nullptr;             // [2]
     int* d_same_flags = nullptr;           // snowflake [total_tiles], grain growth [q][total_tiles]:
@@ -380,6 +386,13 @@ StepArgs step_args(amps_ctx* c, int from) {
 int sync_stream(amps_ctx* c) {
     HIPCHK(hipStreamSynchronize(c->stream));
     c->idle = true;
+    return AMPS_OK;
+}
+
+int host_words(amps_ctx* c) {
+    if (c->host) return AMPS_OK;
+    HIPCHK(hipHostMalloc((void**)&c->host, sizeof(HostWords), hipHostMallocMapped));
+    HIPCHK(hipHostGetDevicePointer((void**)&c->d_host, c->host, 0));
     return AMPS_OK;
 }
 
@@ -877,8 +890,7 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     mem.ask(&c->d_type_old, gt * sizeof(int));
     mem.ask(&c->d_md, gt * sizeof(double));
     if (c->mode == AMPS_ADAPTIVE && c->monitor == AMPS_MON_TEMPORAL) mem.ask(&c->d_last, gt * 16 * sizeof(double));
-    mem.ask(&c->d_stats, 8 * sizeof(unsigned long long));
-    mem.ask(&c->d_cls, CLS_WORDS * sizeof(unsigned long long));
+    mem.ask(&c->d_stats, (STATS_WORDS + CLS_WORDS) * sizeof(unsigned long long));
     mem.ask(&c->d_step, sizeof(long long));
     if (has_low(c)) mem.ask(&c->d_scratch, (size_t)c->max_inst_cells * sizeof(double));
     mem.ask(&c->d_wl, 2 * (size_t)tiles * sizeof(int));
@@ -895,6 +907,7 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     }
     rc = mem.get(c);
     if (rc != AMPS_OK) { std::string m = g_last_error; amps_destroy(c); return fail(rc, m); }
+    c->d_cls = c->d_stats + STATS_WORDS;
     e = hipMemcpy(c->d_desc, c->desc.data(), sizeof(InstDesc) * n, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->d_tile_inst, c->tile_inst.data(), sizeof(int) * tiles, hipMemcpyHostToDevice);
     if (e == hipSuccess && !blk_inst.empty()) {
@@ -935,7 +948,7 @@ void amps_destroy(amps_ctx* c) {
     for (hipGraphExec_t g : {c->many.exec[0], c->many.exec[1], c->few.exec[0], c->few.exec[1]})
         if (g) (void)hipGraphExecDestroy(g);
     if (c->memory) (void)hipFree(c->memory);
-    if (c->bad) (void)hipHostFree(c->bad);
+    if (c->host) (void)hipHostFree(c->host);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -955,9 +968,7 @@ int amps_init(amps_ctx* c) {
     HIPCHK(hipMemcpyAsync(c->d_type_old, types.data(), types.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
     long long zero = 0;
     HIPCHK(hipMemcpyAsync(c->d_step, &zero, sizeof(zero), hipMemcpyHostToDevice, c->stream));
-    static const unsigned long long z8[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    HIPCHK(hipMemcpyAsync(c->d_stats, z8, sizeof(z8), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemsetAsync(c->d_cls, 0, CLS_WORDS * sizeof(unsigned long long), c->stream));
+    HIPCHK(hipMemsetAsync(c->d_stats, 0, (STATS_WORDS + CLS_WORDS) * sizeof(unsigned long long), c->stream));
     // step 0 appends to parity 0
     if (c->d_full_cnt) HIPCHK(hipMemsetAsync(c->d_full_cnt, 0, FULL_CNT_INTS * sizeof(int), c->stream));
     HIPCHK(hipMemsetAsync(c->d_same_flags, 0, c->same_flags_n * sizeof(int), c->stream));
@@ -1049,23 +1060,20 @@ int amps_get_field(amps_ctx* c, int inst, int field, double* dst, size_t n) {
     if (inst < 0 || inst >= c->ninst || field < 0 || field >= c->nfields) return fail(AMPS_E_ARG, "instance or field out of range");
     const InstDesc& d = c->desc[inst];
     if (n != (size_t)d.nx * d.ny) return fail(AMPS_E_ARG, "n must equal nx*ny of the instance");
-    if (!c->bad) {
-        HIPCHK(hipHostMalloc((void**)&c->bad, sizeof(int), hipHostMallocMapped));
-        HIPCHK(hipHostGetDevicePointer((void**)&c->d_bad, c->bad, 0));
-    }
-    *c->bad = 0;  // set by the device if a value is not finite
+    RCCHK(host_words(c));
+    c->host->bad = 0;  // set by the device if a value is not finite
     const int group = has_low(c) ? c->gm.fg[field] : -1;
     const double* src = c->d_scratch;
     if (group >= 0) {
         RCCHK(launch_gather(c->d_desc, c->buf[c->cur], c->total_cells, c->total_tiles, c->d_type, group, inst,
-                            d.tx * d.ty, field, c->d_scratch, c->d_bad, c->tile, c->stream));
+                            d.tx * d.ty, field, c->d_scratch, &c->d_host->bad, c->tile, c->stream));
     } else {
         src = c->buf[c->cur].f64 + (size_t)field * c->total_cells + d.cell_base;
-        RCCHK(launch_nonfinite(src, (long long)n, c->d_bad, c->stream));
+        RCCHK(launch_nonfinite(src, (long long)n, &c->d_host->bad, c->stream));
     }
     HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     RCCHK(sync_stream(c));
-    if (*(volatile int*)c->bad) return fail(AMPS_E_NONFINITE, "field " + std::to_string(field) + " holds non-finite values");
+    if (*(volatile int*)&c->host->bad) return fail(AMPS_E_NONFINITE, "field " + std::to_string(field) + " holds non-finite values");
     return AMPS_OK;
 }
 
@@ -1158,21 +1166,15 @@ int amps_get_raw_field(amps_ctx* c, int inst, int field, uint16_t* words, size_t
 
 int amps_get_info(amps_ctx* c, amps_info* info) {
     if (!c || !info) return fail(AMPS_E_ARG, "NULL argument");
+    RCCHK(host_words(c));
+    RCCHK(launch_counters(c->d_cls, c->d_stats, c->d_host->counted, c->stream));
     RCCHK(sync_stream(c));
-    unsigned long long st[8];
-    HIPCHK(hipMemcpy(st, c->d_stats, sizeof(st), hipMemcpyDeviceToHost));
+    const auto counted = [&](int kind) { return (unsigned long long)((volatile unsigned long long*)c->host->counted)[kind]; };
     std::memset(info, 0, sizeof(*info));
     info->steps_done = c->steps_done;
-    std::vector<unsigned long long> cls(CLS_WORDS);
-    HIPCHK(hipMemcpy(cls.data(), c->d_cls, CLS_WORDS * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-    const auto counted = [&](int kind) {
-        unsigned long long n = 0;
-        for (int k = 0; k < CLASSIFY_SLOTS; ++k) n += cls[(size_t)(kind * CLASSIFY_SLOTS + k) * STATS_STRIDE];
-        return n;
-    };
-    info->fp64_tile_updates = (int64_t)(st[2] + counted(2));
-    info->low_full_tile_updates = (int64_t)(st[3] + counted(3));
-    info->low_listed_tile_updates = (int64_t)(st[4] + counted(4));
+    info->fp64_tile_updates = (int64_t)counted(2);
+    info->low_full_tile_updates = (int64_t)counted(3);
+    info->low_listed_tile_updates = (int64_t)counted(4);
     info->monitor_passes = c->monitor_passes;
     int maxt = 0;
     for (auto& d : c->desc) maxt = std::max(maxt, d.tx * d.ty);

@@ -788,6 +788,24 @@ __global__ __launch_bounds__(256) void nonfinite_kernel(const double* v, long lo
     if (!ok) *bad = 1;
 }
 
+// Sums of the spread counters: one wave, a lane per slot, the five kinds' loads
+// in flight together.  Bound by the launch; amps_get_info takes 25 us with
+// it, 46 where it copied the slots (20 KB) to the host.
+__global__ __launch_bounds__(64) void counters_kernel(const unsigned long long* __restrict__ cls,
+                                                      const unsigned long long* __restrict__ stats,
+                                                      unsigned long long* __restrict__ out) {
+    static_assert(CLASSIFY_SLOTS == 64, "one lane per slot");
+    unsigned long long v[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) v[k] = cls[(size_t)(k * CLASSIFY_SLOTS + (int)threadIdx.x) * STATS_STRIDE];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o);
+        if (threadIdx.x == 0) out[k] = v[k] + (k >= 2 ? stats[k] : 0ull);
+    }
+}
+
 __global__ void fill_u64_kernel(unsigned long long* p, int n, unsigned long long v) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
@@ -1074,6 +1092,12 @@ int launch_nonfinite(const double* v, long long n, int* bad, hipStream_t s) {
     long long g = (n + 255) / 256;
     if (g > 4096) g = 4096;
     hipLaunchKernelGGL(nonfinite_kernel, dim3((int)g), dim3(256), 0, s, v, n, bad);
+    return hip_ok();
+}
+
+int launch_counters(const unsigned long long* cls, const unsigned long long* stats, unsigned long long* out,
+                    hipStream_t s) {
+    hipLaunchKernelGGL(counters_kernel, dim3(1), dim3(64), 0, s, cls, stats, out);
     return hip_ok();
 }
 

@@ -41,6 +41,11 @@ int launch_classify_convert(const InstDesc* inst, const int* tile_inst, const Bu
 int launch_gather(const InstDesc* inst, const Buf& b, long long total_cells, int total_tiles, const int* type,
                   int group, int instid, int ntiles_inst, int field, double* dst, int* bad, int tile, hipStream_t s);
 int launch_nonfinite(const double* v, long long n, int* bad, hipStream_t s);
+// out (host memory): the classification's and the sweeps' counters, kind by
+// kind (see StepArgs::spread; cls: all of them), each summed over its slots
+// and, from kind 2 on, added to stats[kind].
+int launch_counters(const unsigned long long* cls, const unsigned long long* stats, unsigned long long* out,
+                    hipStream_t s);
 int launch_fill_u64(unsigned long long* p, int n, unsigned long long v, hipStream_t s);
 int launch_advance_step(long long* step_ctr, int n, hipStream_t s);
 
