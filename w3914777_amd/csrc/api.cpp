@@ -62,6 +62,8 @@ constexpr size_t FULL_CNT_INTS = 2 * (size_t)NSK_SEGS * NSK_CNT_STRIDE;
 // words of the spread counters: the classification's (all passes, the last
 // pass) and the one-launch step's three
 constexpr size_t STATS_WORDS = 32, CLS_WORDS = 5 * (size_t)CLASSIFY_SLOTS * STATS_STRIDE;
+// all counters of a context, one behind the other
+constexpr size_t COUNTER_BYTES = (STATS_WORDS + CLS_WORDS) * 8 + FULL_CNT_INTS * sizeof(int);
 
 // Words of a context in host memory that kernels write.
 struct HostWords {
@@ -890,7 +892,7 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     mem.ask(&c->d_type_old, gt * sizeof(int));
     mem.ask(&c->d_md, gt * sizeof(double));
     if (c->mode == AMPS_ADAPTIVE && c->monitor == AMPS_MON_TEMPORAL) mem.ask(&c->d_last, gt * 16 * sizeof(double));
-    mem.ask(&c->d_stats, (STATS_WORDS + CLS_WORDS) * sizeof(unsigned long long));
+    mem.ask(&c->d_stats, COUNTER_BYTES);
     mem.ask(&c->d_step, sizeof(long long));
     if (has_low(c)) mem.ask(&c->d_scratch, (size_t)c->max_inst_cells * sizeof(double));
     mem.ask(&c->d_wl, 2 * (size_t)tiles * sizeof(int));
@@ -898,7 +900,6 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     c->same_flags_n = (size_t)(c->model == AMPS_GRAINGROWTH ? c->q : 1) * tiles;
     mem.ask(&c->d_same_flags, c->same_flags_n * sizeof(int));
     mem.ask(&c->d_full_seg, (size_t)NSK_SEGS * nsk_cap(tiles) * sizeof(int));
-    mem.ask(&c->d_full_cnt, FULL_CNT_INTS * sizeof(int));
     std::vector<int> blk_inst, blk_base;
     plan_multi(c, blk_inst, blk_base);
     if (!blk_inst.empty()) {
@@ -908,6 +909,7 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
     rc = mem.get(c);
     if (rc != AMPS_OK) { std::string m = g_last_error; amps_destroy(c); return fail(rc, m); }
     c->d_cls = c->d_stats + STATS_WORDS;
+    c->d_full_cnt = reinterpret_cast<int*>(c->d_cls + CLS_WORDS);
     e = hipMemcpy(c->d_desc, c->desc.data(), sizeof(InstDesc) * n, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->d_tile_inst, c->tile_inst.data(), sizeof(int) * tiles, hipMemcpyHostToDevice);
     if (e == hipSuccess && !blk_inst.empty()) {
@@ -968,9 +970,7 @@ int amps_init(amps_ctx* c) {
     HIPCHK(hipMemcpyAsync(c->d_type_old, types.data(), types.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
     long long zero = 0;
     HIPCHK(hipMemcpyAsync(c->d_step, &zero, sizeof(zero), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemsetAsync(c->d_stats, 0, (STATS_WORDS + CLS_WORDS) * sizeof(unsigned long long), c->stream));
-    // step 0 appends to parity 0
-    if (c->d_full_cnt) HIPCHK(hipMemsetAsync(c->d_full_cnt, 0, FULL_CNT_INTS * sizeof(int), c->stream));
+    HIPCHK(hipMemsetAsync(c->d_stats, 0, COUNTER_BYTES, c->stream));  // the lists' too: step 0 appends to parity 0
     HIPCHK(hipMemsetAsync(c->d_same_flags, 0, c->same_flags_n * sizeof(int), c->stream));
     RCCHK(clear_zmasks(c));
     if (c->mode == AMPS_PURE_HALF2)
@@ -1166,10 +1166,14 @@ int amps_get_raw_field(amps_ctx* c, int inst, int field, uint16_t* words, size_t
 
 int amps_get_info(amps_ctx* c, amps_info* info) {
     if (!c || !info) return fail(AMPS_E_ARG, "NULL argument");
-    RCCHK(host_words(c));
-    RCCHK(launch_counters(c->d_cls, c->d_stats, c->d_host->counted, c->stream));
+    if (has_low(c)) {  // PURE_FP64 steps count nothing
+        RCCHK(host_words(c));
+        RCCHK(launch_counters(c->d_cls, c->d_stats, c->d_host->counted, c->stream));
+    }
     RCCHK(sync_stream(c));
-    const auto counted = [&](int kind) { return (unsigned long long)((volatile unsigned long long*)c->host->counted)[kind]; };
+    const auto counted = [&](int kind) -> unsigned long long {
+        return has_low(c) ? ((volatile unsigned long long*)c->host->counted)[kind] : 0;
+    };
     std::memset(info, 0, sizeof(*info));
     info->steps_done = c->steps_done;
     info->fp64_tile_updates = (int64_t)counted(2);
