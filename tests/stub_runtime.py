@@ -1,8 +1,8 @@
 """Runs a script in a process whose libamps.so is bound to tests/hip_stub.c in
 place of the HIP runtime: kernels are logged, not run.  The script finds
 `amps` (the package), `stub` (live(), peak(), limit(bytes), clear() and
-log(): the kernels launched, "graph" for a replayed graph, "copy", "memset" and
-"free", a leading + while a graph is captured) and `out`, a dict that comes back."""
+log(): the kernels launched, "graph" for a replayed graph, "copy", "memset",
+"free" and "host" (a host function), a leading + while a graph is captured) and `out`, a dict that comes back."""
 import json
 import os
 import re
@@ -38,7 +38,8 @@ out = {{}}
 def build(tmp):
     lib, ver = os.path.join(tmp, "libhipstub.so"), os.path.join(tmp, "hip.map")
     with open(ver, "w") as f:
-        f.write("hip_4.2 { global: *; };\nhip_4.3 { global: " + " ".join(g + ";" for g in GRAPH) + " } hip_4.2;\n")
+        f.write("hip_4.2 { global: *; };\nhip_4.3 { global: " + " ".join(g + ";" for g in GRAPH) + " } hip_4.2;\n"
+                "hip_5.3 { global: hipLaunchHostFunc; } hip_4.3;\n")
     subprocess.run(["gcc", "-O1", "-Wall", "-shared", "-fPIC", os.path.join(HERE, "hip_stub.c"), "-o", lib,
                     "-Wl,-soname,libamdhip64.so.7", "-Wl,--version-script," + ver], check=True)
     return lib

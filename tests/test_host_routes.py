@@ -158,3 +158,42 @@ for name, model in (("sf", amps.SNOWFLAKE), ("gg", amps.GRAINGROWTH), ("sn", amp
     for name, (init, info) in out.items():
         assert init <= (8 if name == "gg" else 6), (name, init)  # gg: two zero masks
         assert len(info) == 1 and "counters" in info[0], (name, info)
+
+
+@pytest.mark.parametrize("n", [64, 512])
+def test_memory_is_freed_after_the_commands_are_retired(run, n):
+    """Between the last command of a stream and the first free of 2 MiB or more
+    after it stands a host function: what is freed before the runtime has retired
+    the commands is released later, on a thread that slows the next calls.
+    Smaller memory needs none."""
+    out = run(f"""
+import numpy as np
+n = {n}
+cfg = amps.Config.default(amps.SNOWFLAKE)
+cfg.nx = cfg.ny = n
+def log(name, f):
+    stub.clear(); f(); out[name] = stub.log()
+c = amps.Context(cfg)
+c.init()
+log("close untaped", lambda: (c.step(5), c.close()))
+c = amps.Context(cfg)
+c.init(); c.tape_begin(2); c.step(5)
+log("adjoint", lambda: c.adjoint([np.zeros((2, n, n))], [1], want_du0=True))
+log("set_field", lambda: c.set_field(0, np.zeros((n, n))))
+c.tape_begin(2); c.step(5)
+log("tape_begin", lambda: (c.step(1), c.tape_begin(1)))
+log("init", lambda: (c.step(1), c.init()))
+c.tape_begin(2)
+log("close", lambda: (c.step(5), c.close()))
+""")
+    assert set(out) == {"close untaped", "adjoint", "set_field", "tape_begin", "init", "close"}
+    for name, log in out.items():
+        assert "free" in log, name
+        if n == 64:
+            assert "host" not in log, name
+            continue
+        retired = False
+        for what in log:
+            assert what != "free" or retired, (name, log)
+            if what != "free":
+                retired = what == "host"
