@@ -91,13 +91,16 @@ __device__ inline int ring_src(int r, int o, int n, int bc) {
 
 // Phase 1 on a box of R-typed values: P = eps eps' gx, Q = eps eps' gy, E2 = eps^2
 // over the (TS+2)^2 ring box (stored as described at SfGeo::PW).
-template <int TS, typename Rt, int NT = WG>
+//
+// FOUR: with the branch-free path for n == 4.  The 32^2 mixed sweep (NT = WG)
+// is at its register limit: there the path costs 3% whether it is taken or not.
+template <int TS, int NT>
+constexpr bool sf_four = TS == 16 || NT != WG;
+
+template <int TS, typename Rt, int NT = WG, bool FOUR = sf_four<TS, NT>>
 __device__ inline void sf_phase1(const Rt* phi, Rt* P, Rt* Q, Rt* E2, const InstDesc& d, int ox, int oy,
                                  Rt inv2dx, Rt inv2dy, Rt cth0, Rt sth0, Rt epsb, Rt epsbd, Rt mend) {
     using G = SfGeo<TS>;
-    // the 32^2 mixed sweep (NT = WG) is at its register limit: the path for
-    // n == 4 costs it 3% whether it is taken or not
-    constexpr bool FOUR = TS == 16 || NT != WG;
     const int n = (int)d.k[SFK_ANISO_N];
     const bool edge = d.bc != AMPS_BC_PERIODIC &&
                       (ox == 0 || oy == 0 || ox + TS == d.nx || oy + TS == d.ny);
@@ -423,7 +426,7 @@ __device__ inline void sf_halo_load(uint2* hp, uint2* ht, const StepArgs& a, con
     }
 }
 
-template <int TS, bool ADAPT, int NT = WG>
+template <int TS, bool ADAPT, int NT = WG, bool FOUR = sf_four<TS, NT>>
 __device__ void sf_tile_f64(SfLds<TS, double>& L, const StepArgs& a, const InstDesc& d, int tile_x, int tile_y,
                             unsigned hmask, long long step) {
     using G = SfGeo<TS, NT>;
@@ -481,7 +484,7 @@ __device__ void sf_tile_f64(SfLds<TS, double>& L, const StepArgs& a, const InstD
     }
     __syncthreads();
 
-    sf_phase1<TS, double, NT>(L.phi, L.P, L.Q, L.E2, d, ox, oy, d.k[SFK_INV_2DX], d.k[SFK_INV_2DY],
+    sf_phase1<TS, double, NT, FOUR>(L.phi, L.P, L.Q, L.E2, d, ox, oy, d.k[SFK_INV_2DX], d.k[SFK_INV_2DY],
                           d.k[SFK_COS_N_THETA0], d.k[SFK_SIN_N_THETA0], d.k[SFK_EPSB], d.k[SFK_EPSB_DELTA],
                           d.k[SFK_MEPSB_ANISO_DELTA]);
     __syncthreads();
@@ -1244,7 +1247,7 @@ __device__ inline unsigned hmask_of(int t) {
 // LDS boxes (50.5 KB) allow 3 workgroups per CU; 32^2 tiles run with NT =
 // 512 threads, 2 cells each (78 VGPRs against 114 at 256 threads and 4
 // cells), so 24 waves per CU share the tile chains' latency instead of 12.
-template <int TS, bool MULTI, int NT = WG>
+template <int TS, bool MULTI, int NT, bool FOUR>
 __global__ __launch_bounds__(NT) void sf_f64_tile_kernel(StepArgs a, const InstDesc* __restrict__ inst,
                                                          const int* __restrict__ tinst) {
     __shared__ __align__(16) SfLds<TS, double> L;
@@ -1255,17 +1258,17 @@ __global__ __launch_bounds__(NT) void sf_f64_tile_kernel(StepArgs a, const InstD
     const InstDesc& d = inst[MULTI ? tinst[w] : 0];
     const int lt = w - d.tile_base;
     const int tile_y = lt / d.tx, tile_x = lt - tile_y * d.tx;
-    sf_tile_f64<TS, false, NT>(L, a, d, tile_x, tile_y, 0x1FFu, step);
+    sf_tile_f64<TS, false, NT, FOUR>(L, a, d, tile_x, tile_y, 0x1FFu, step);
 }
 
 // The same sweep of one grid whose descriptor and step index are kernel
 // arguments (the no-allocation step: no device copy of them to write first).
-template <int TS, int NT>
+template <int TS, int NT, bool FOUR>
 __global__ __launch_bounds__(NT) void sf_f64_arg_kernel(StepArgs a, InstDesc d, long long step) {
     __shared__ __align__(16) SfLds<TS, double> L;
     const int w = xcd_remap(blockIdx.x, a.nwork);
     const int tile_y = w / d.tx, tile_x = w - tile_y * d.tx;
-    sf_tile_f64<TS, false, NT>(L, a, d, tile_x, tile_y, 0x1FFu, step);
+    sf_tile_f64<TS, false, NT, FOUR>(L, a, d, tile_x, tile_y, 0x1FFu, step);
 }
 
 // Inclusive prefix sum over the wave's lanes, by lane moves within the vector
@@ -1823,6 +1826,21 @@ static int resident_grid(int nwork, int cap) {
     return (int)(g < nwork ? g : nwork);
 }
 
+// The single FP64 step has the branch-free four-fold path (sf_unit_power4) up
+// to this many cells: it shortens a tile's chain, which small grids wait on,
+// and costs issue slots, which large ones are bound by.  us a step with :
+// without, four-fold, reference physics and Laplacian:
+//   tile 16:  800^2 10.4 : 10.6; 1024^2 13.2 : 13.6; 1152^2 17.3 : 16.7; 2048^2 38.4 : 35.7; 4096^2 156 : 145
+//   tile 32: 1024^2 12.2 : 12.5; 1152^2 16.2 : 15.4; 2048^2 33.9 : 32.4; 4096^2 136 : 131
+// With the 5-point Laplacian it costs at every size (tile 16, 800^2 9.5 : 9.2,
+// 1024^2 12.6 : 12.2).  The no-allocation step, whose descriptor arrives with
+// the launch, gains further up, to FOUR_CELLS with the 5-point Laplacian:
+//   tile 16:  512^2 5.5 : 6.1; 1024^2 14.2 : 15.8; 2048^2 40.8 : 42.9; 2560^2 59 : 60; 3072^2 91 : 90; 4096^2 160 : 145
+//             5-point 1024^2 13.2 : 14.2; 1280^2 19.0 : 19.0; 1408^2 21.9 : 21.7; 2560^2 56 : 53
+//   tile 32:  512^2 5.5 : 5.9; 1024^2 12.3 : 13.4; 2048^2 36.3 : 37.5; 2560^2 50 : 51; 3072^2 76 : 76; 4096^2 130 : 127
+//             5-point 1024^2 11.3 : 12.0; 1152^2 15.2 : 15.0; 2048^2 33.1 : 32.2
+constexpr int FOUR_CELLS = 1 << 20, FOUR_ARG_CELLS = 1 << 23;
+
 template <int TS, bool MULTI>
 static void sf_launch(const StepArgs& a, bool adaptive, hipStream_t s, const hipEvent_t* ev) {
     dim3 blk(WG);
@@ -1864,7 +1882,11 @@ static void sf_launch(const StepArgs& a, bool adaptive, hipStream_t s, const hip
     } else {
         // 32^2 tiles: 512 threads, 2 cells each (see sf_f64_tile_kernel)
         constexpr int NT = TS == 32 ? 512 : WG;
-        launch_sweep(sf_f64_tile_kernel<TS, MULTI, NT>, dim3(a.nwork), dim3(NT), s, ev, a, a.inst, a.tile_inst);
+        const dim3 g(a.nwork), b(NT);
+        if (a.t_halo == 2 && a.nwork <= FOUR_CELLS / (TS * TS))
+            launch_sweep(sf_f64_tile_kernel<TS, MULTI, NT, true>, g, b, s, ev, a, a.inst, a.tile_inst);
+        else
+            launch_sweep(sf_f64_tile_kernel<TS, MULTI, NT, false>, g, b, s, ev, a, a.inst, a.tile_inst);
     }
 }
 
@@ -1891,8 +1913,12 @@ int launch_sf_one(const StepArgs& a, int tile, hipStream_t s) {
 
 int launch_sf_step_arg(const StepArgs& a, const InstDesc& d, long long step, int tile, hipStream_t s) {
     // thread counts as in sf_launch
-    if (tile == 16) hipLaunchKernelGGL((sf_f64_arg_kernel<16, WG>), dim3(a.nwork), dim3(WG), 0, s, a, d, step);
-    else if (tile == 32) hipLaunchKernelGGL((sf_f64_arg_kernel<32, 512>), dim3(a.nwork), dim3(512), 0, s, a, d, step);
+    const bool four = a.nwork <= (d.stencil == AMPS_STENCIL_REF ? FOUR_ARG_CELLS : FOUR_CELLS) / (tile * tile);
+    const dim3 g(a.nwork);
+    if (tile == 16 && four) hipLaunchKernelGGL((sf_f64_arg_kernel<16, WG, true>), g, dim3(WG), 0, s, a, d, step);
+    else if (tile == 16) hipLaunchKernelGGL((sf_f64_arg_kernel<16, WG, false>), g, dim3(WG), 0, s, a, d, step);
+    else if (tile == 32 && four) hipLaunchKernelGGL((sf_f64_arg_kernel<32, 512, true>), g, dim3(512), 0, s, a, d, step);
+    else if (tile == 32) hipLaunchKernelGGL((sf_f64_arg_kernel<32, 512, false>), g, dim3(512), 0, s, a, d, step);
     else return AMPS_E_UNSUPPORTED;
     return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;
 }
