@@ -170,12 +170,19 @@ namespace {
 //
 // Grids of power-of-two sides would put the same cell of every buffer, and of
 // every field of a buffer, on the same memory channels: the buffers are
-// STAGGER bytes further apart than they need to be, the fields FIELD_PAD
+// STAGGER bytes further apart than they need to be, the fields field_pad
 // cells (a multiple of 32: the vector loads' alignment).  Measured on Q = 36
 // grain growth: adaptive 1024^2 137 us a step with neither (the buffers'
-// stagger alone gives 134), 129 with both; FP64 2048^2 567 -> 530.
+// stagger alone gives 134), 129 with both; FP64 2048^2 567 -> 530.  Fields of
+// two or three beyond the cache lose by it, us a step without : with:
+//   snowflake FP64 4096^2 tile 16 143.6 : 145.6, 5-point 140.6 : 143.5; tile 32 130.1 : 131.3, 5-point 125.4 : 126.8
+//                  2048^2 tile 32 32.8 : 32.5, 5-point 31.0 : 29.8; 3072^2 77.2 : 76.6
+//   sintering FP64 4096^2 123.5 : 124.2; 2048^2 30.4 : 29.8
 constexpr size_t STAGGER = 4352;
-constexpr long long FIELD_PAD = 1056;
+
+long long field_pad(int model, long long cells) {
+    return model == AMPS_GRAINGROWTH || cells < 12ll << 20 ? 1056 : 0;
+}
 
 struct DeviceArena {
     struct Ask {
@@ -185,7 +192,7 @@ struct DeviceArena {
     std::vector<Ask> asks;
     template <typename T>
     void ask(T** p, size_t bytes) {
-asks.push_back({reinterpret_cast<void**>(p), ((std::max<size_t>(bytes, 8) + 255) & ~(size_t)255) + STAGGER});
+        asks.push_back({reinterpret_cast<void**>(p), ((std::max<size_t>(bytes, 8) + 255) & ~(size_t)255) + STAGGER});
     }
     int get(amps_ctx* c) {
         size_t total = 0;
@@ -884,7 +891,7 @@ int amps_create_batch(const amps_config* cfgs, int n, amps_ctx** out) {
         for (int t = 0; t < d.tx * d.ty; ++t) c->tile_inst.push_back(i);
     }
     c->cells = cells;
-    c->total_cells = cells + FIELD_PAD;
+    c->total_cells = cells + field_pad(c->model, cells);
     c->total_tiles = tiles;
 
     int rc = AMPS_OK;
