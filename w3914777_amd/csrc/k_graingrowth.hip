@@ -666,88 +666,127 @@ __global__ __launch_bounds__(NT, 4) void gg_block_kernel(StepArgs a, const InstD
 // field changed precision are refreshed (a conversion re-rounds the stored
 // values; elsewhere S already matches them).
 //
-// Workgroup b takes tiles b, b + grid, ...: one round of loads brings the
-// types (and type_old, codes) of all fields of a tile into LDS, one thread a
-// field; a tile to refresh then has the values of AUX_NF fields in flight at
-// once, added in field order.  One workgroup per tile up to AUX_GRID
-// workgroups, where a workgroup took WG / q tiles in a row, field by field:
-// 512^2 with q = 2 (1024 tiles) 133 -> 6 us, the changed tiles of 1024^2
-// with q = 36 41 -> 13 us.
-constexpr int AUX_NF = 6, AUX_GRID = 4096;
+// Up to AUX_GRID tiles a workgroup takes one: one round of loads brings the
+// types (and type_old, codes) of all its fields into LDS, one thread a field; a
+// tile to refresh then has the values of AUX_NF fields in flight at once, added
+// in field order.  512^2 with q = 2 (1024 tiles) 6 us, the changed tiles of
+// 1024^2 with q = 36 13 us (133 and 41 with WG / q tiles a workgroup, field by
+// field).  Of more tiles few change type in a pass: a workgroup then looks for
+// them among AUX_ROUND at once, 16 threads a tile (MANY).  A pass that changes
+// nothing, q = 2: 65,536 tiles of 16^2 2.7 us against 25.5 tile by tile, of 32^2
+// 4.0 against 44.7.
+constexpr int AUX_NF = 6, AUX_GRID = 4096, AUX_ROUND = 16;
+
+struct GgAuxLds {
+    int ty[AMPS_MAX_FIELDS];
+    double off[AMPS_MAX_FIELDS], scl[AMPS_MAX_FIELDS];
+};
+
+// The tables of tile w, thread f loading field f's; true where f changed type.
+__device__ inline bool gg_aux_tables(GgAuxLds& L, const StepArgs& a, int w, const int* __restrict__ type_old,
+                                     const int* __restrict__ types) {
+    const int f = threadIdx.x;
+    if (f >= a.q || !types) return false;
+    const size_t i = (size_t)f * a.total_tiles + w;
+    const int ty = types[i];
+    L.ty[f] = ty;
+    L.off[f] = a.in.off[i];
+    L.scl[f] = a.in.scl[i];
+    return type_old && type_old[i] != ty;
+}
 
 template <int TS>
-__global__ __launch_bounds__(256) void gg_aux_kernel(StepArgs a, const int* __restrict__ type_old,
-                                                     const int* __restrict__ types) {
+__device__ inline void gg_aux_tile(const GgAuxLds& L, const StepArgs& a, int w, const int* __restrict__ types) {
     constexpr int PER = TS * TS / WG;
-    __shared__ int lty[AMPS_MAX_FIELDS];
-    __shared__ double loff[AMPS_MAX_FIELDS], lscl[AMPS_MAX_FIELDS];
-    __shared__ int changed;
-    const size_t T = (size_t)a.total_tiles;
-    for (int w = blockIdx.x; w < a.total_tiles; w += gridDim.x) {
-        if (threadIdx.x < 64) {
-            const int f = threadIdx.x;
-            bool chg = type_old == nullptr;
-            if (f < a.q && types) {
-                const size_t i = (size_t)f * T + w;
-                const int ty = types[i];
-                lty[f] = ty;
-                loff[f] = a.in.off[i];
-                lscl[f] = a.in.scl[i];
-                if (type_old) chg = type_old[i] != ty;
-            }
-            const unsigned long long m = __ballot(chg);
-            if (threadIdx.x == 0) changed = m != 0ull;
+    const InstDesc& d = a.inst[a.tile_inst[w]];
+    const int lt = w - d.tile_base;
+    const int tile_y = lt / d.tx, tile_x = lt - tile_y * d.tx;
+    double S[PER];
+    size_t gc[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int e = threadIdx.x + i * WG, ly = e / TS, lx = e - ly * TS;
+        gc[i] = d.cell_base + (size_t)(tile_y * TS + ly) * d.nx + tile_x * TS + lx;
+        S[i] = 0.0;
+    }
+    for (int f0 = 0; f0 < a.q; f0 += AUX_NF) {
+        // FP64 bits, or the aligned 4-word fp16 group holding the word
+        // (one load sequence for both storages); fields past the last
+        // repeat it and are not added
+        uint2 raw[AUX_NF][PER];
+#pragma unroll
+        for (int k = 0; k < AUX_NF; ++k) {
+            const int f = min(f0 + k, a.q - 1);
+            const bool wide = !types || L.ty[f] == 2;
+            const size_t fb = (size_t)f * a.total_cells;
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+                raw[k][i] = *(wide ? reinterpret_cast<const uint2*>(a.in.f64 + fb + gc[i])
+                                   : reinterpret_cast<const uint2*>(
+                                         reinterpret_cast<const unsigned short*>(a.in.f16) +
+                                         ((fb + gc[i]) & ~(size_t)3)));
         }
-        __syncthreads();
-        if (changed) {
-            const InstDesc& d = a.inst[a.tile_inst[w]];
-            const int lt = w - d.tile_base;
-            const int tile_y = lt / d.tx, tile_x = lt - tile_y * d.tx;
-            double S[PER];
-            size_t gc[PER];
+#pragma unroll
+        for (int k = 0; k < AUX_NF; ++k) {
+            const int f = f0 + k;
+            if (f >= a.q) break;
+            const bool wide = !types || L.ty[f] == 2;
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
-                const int e = threadIdx.x + i * WG, ly = e / TS, lx = e - ly * TS;
-                gc[i] = d.cell_base + (size_t)(tile_y * TS + ly) * d.nx + tile_x * TS + lx;
-                S[i] = 0.0;
-            }
-            for (int f0 = 0; f0 < a.q; f0 += AUX_NF) {
-                // FP64 bits, or the aligned 4-word fp16 group holding the word
-                // (one load sequence for both storages); fields past the last
-                // repeat it and are not added
-                uint2 raw[AUX_NF][PER];
-#pragma unroll
-                for (int k = 0; k < AUX_NF; ++k) {
-                    const int f = min(f0 + k, a.q - 1);
-                    const bool wide = !types || lty[f] == 2;
-                    const size_t fb = (size_t)f * a.total_cells;
-#pragma unroll
-                    for (int i = 0; i < PER; ++i)
-                        raw[k][i] = *(wide ? reinterpret_cast<const uint2*>(a.in.f64 + fb + gc[i])
-                                           : reinterpret_cast<const uint2*>(
-                                                 reinterpret_cast<const unsigned short*>(a.in.f16) +
-                                                 ((fb + gc[i]) & ~(size_t)3)));
-                }
-#pragma unroll
-                for (int k = 0; k < AUX_NF; ++k) {
-                    const int f = f0 + k;
-                    if (f >= a.q) break;
-                    const bool wide = !types || lty[f] == 2;
-#pragma unroll
-                    for (int i = 0; i < PER; ++i) {
-                        // the square and the sum are two roundings
+                // the square and the sum are two roundings
 #pragma clang fp contract(off)
-                        const double v =
-                            wide ? raw_f64(raw[k][i].x, raw[k][i].y)
-                                 : loff[f] + (double)half_word(raw_word4(raw[k][i], (int)(gc[i] & 3))) * lscl[f];
-                        S[i] += v * v;
-                    }
-                }
+                const double v =
+                    wide ? raw_f64(raw[k][i].x, raw[k][i].y)
+                         : L.off[f] + (double)half_word(raw_word4(raw[k][i], (int)(gc[i] & 3))) * L.scl[f];
+                S[i] += v * v;
             }
-#pragma unroll
-            for (int i = 0; i < PER; ++i) a.aux_in[gc[i]] = S[i];
         }
-        __syncthreads();  // the tables are rewritten for the next tile
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) a.aux_in[gc[i]] = S[i];
+}
+
+template <int TS, bool MANY>
+__global__ __launch_bounds__(256) void gg_aux_kernel(StepArgs a, const int* __restrict__ type_old,
+                                                     const int* __restrict__ types) {
+    __shared__ GgAuxLds L;
+    __shared__ unsigned changed[WG / 64];
+    if constexpr (MANY) {
+        const int j = threadIdx.x & (AUX_ROUND - 1);
+        for (long long c0 = (long long)blockIdx.x * AUX_ROUND; c0 < a.total_tiles; c0 += (long long)gridDim.x * AUX_ROUND) {
+            bool chg = false;
+            if (c0 + j < a.total_tiles)
+                for (int f = threadIdx.x / AUX_ROUND; f < a.q; f += WG / AUX_ROUND) {
+                    const size_t i = (size_t)f * a.total_tiles + c0 + j;
+                    chg |= type_old[i] != types[i];
+                }
+            const unsigned long long m = __ballot(chg);
+            if ((threadIdx.x & 63) == 0)
+                changed[threadIdx.x >> 6] = (unsigned)(m | m >> 16 | m >> 32 | m >> 48) & 0xFFFFu;
+            static_assert(AUX_ROUND == 16, "four tiles' threads a wave, folded to 16 bits");
+            __syncthreads();
+            unsigned todo = changed[0] | changed[1] | changed[2] | changed[3];
+            while (todo) {
+                const int w = (int)c0 + __ffs((int)todo) - 1;
+                todo &= todo - 1;
+                (void)gg_aux_tables(L, a, w, nullptr, types);
+                __syncthreads();
+                gg_aux_tile<TS>(L, a, w, types);
+                __syncthreads();  // the tables are rewritten for the next tile
+            }
+            __syncthreads();  // changed is rewritten by the next round
+        }
+    } else {
+        for (int w = blockIdx.x; w < a.total_tiles; w += gridDim.x) {
+            if (threadIdx.x < 64) {
+                const bool chg = gg_aux_tables(L, a, w, type_old, types) || type_old == nullptr;
+                const unsigned long long m = __ballot(chg);
+                if (threadIdx.x == 0) changed[0] = m != 0ull;
+            }
+            __syncthreads();
+            if (changed[0]) gg_aux_tile<TS>(L, a, w, types);
+            __syncthreads();  // the tables are rewritten for the next tile
+        }
     }
 }
 
@@ -912,9 +951,14 @@ int launch_gg_step(const StepArgs& a, int tile, bool adaptive, int grid, hipStre
 }
 
 int launch_gg_aux(const StepArgs& a, int tile, const int* type_old, hipStream_t s) {
-    const int grid = a.total_tiles < 1 ? 1 : (a.total_tiles < AUX_GRID ? a.total_tiles : AUX_GRID);
-    if (tile == 16) hipLaunchKernelGGL((gg_aux_kernel<16>), dim3(grid), dim3(WG), 0, s, a, type_old, a.type);
-    else if (tile == 32) hipLaunchKernelGGL((gg_aux_kernel<32>), dim3(grid), dim3(WG), 0, s, a, type_old, a.type);
+    const bool many = type_old && a.total_tiles > AUX_GRID;
+    const int items = many ? (a.total_tiles + AUX_ROUND - 1) / AUX_ROUND : a.total_tiles;
+    const int cap = many ? 4 * AUX_GRID : AUX_GRID;
+    const dim3 g(items < 1 ? 1 : (items < cap ? items : cap)), b(WG);
+    if (tile == 16 && many) hipLaunchKernelGGL((gg_aux_kernel<16, true>), g, b, 0, s, a, type_old, a.type);
+    else if (tile == 16) hipLaunchKernelGGL((gg_aux_kernel<16, false>), g, b, 0, s, a, type_old, a.type);
+    else if (tile == 32 && many) hipLaunchKernelGGL((gg_aux_kernel<32, true>), g, b, 0, s, a, type_old, a.type);
+    else if (tile == 32) hipLaunchKernelGGL((gg_aux_kernel<32, false>), g, b, 0, s, a, type_old, a.type);
     else return AMPS_E_UNSUPPORTED;
     return hipGetLastError() == hipSuccess ? AMPS_OK : AMPS_E_HIP;
 }
