@@ -131,7 +131,7 @@ typedef struct {
     int32_t monitor;        /* amps_monitor (ADAPTIVE only)                        */
     int32_t nx, ny;         /* grid; multiples of tile                             */
     int32_t q;              /* grain growth: order parameters (>=2); others ignore */
-    int32_t tile;           /* square tile edge: 16, 32 or 64                      */
+    int32_t tile;           /* square tile edge: 16 or 32                          */
     int32_t monitor_every;  /* steps between monitor passes (reference: 10)        */
     int32_t monitor_field;  /* field the monitor reads; -1 (grain growth only):
                                each field gets its own per-tile type             */
@@ -275,7 +275,8 @@ int amps_get_info(amps_ctx* ctx, amps_info* info);
 /* When enabled, every sweep kernel launched by amps_step carries a pair of
  * HIP events bound to its own dispatch (hipExtLaunchKernel), so the summed
  * durations are the kernels' execution times without dispatch gaps; graph
- * replay and launches of several steps are suspended meanwhile, and the
+ * replay, launches of several steps and the one-launch low-precision step of
+ * small snowflake grids (two sweeps instead) are suspended meanwhile, and the
  * counters below restart from zero.  Replaces the per-kernel cudaEvent
  * pairs of the reference's timing-decomposition drivers
  * (snowflake/monitor_independent_withoutmonitor.cu:85-127). */

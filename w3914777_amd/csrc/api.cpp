@@ -329,10 +329,10 @@ void fill_desc(InstDesc& d, const amps_config& c) {
 
 bool has_low(const amps_ctx* c) { return c->mode != AMPS_PURE_FP64; }
 
-// The snowflake's low-precision step runs two sweep kernels: the bulk-hold
-// sweep over the low tiles, then the mixed sweep (FP64 tiles and the low
-// tiles it did not hold); with NO_SKIP the FP64 sweep, then the full low
-// sweep.
+// The snowflake's low-precision step runs two sweep kernels where it is not
+// one launch: the bulk-hold sweep (NO_SKIP: the flat sweep) over the low tiles,
+// then the mixed sweep over the FP64 tiles and the low tiles the first one
+// listed.
 bool two_sweeps(const amps_ctx* c) { return c->model == AMPS_SNOWFLAKE && has_low(c); }
 bool low_sweep_first(const amps_ctx* c) { return two_sweeps(c); }
 

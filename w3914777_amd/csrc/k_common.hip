@@ -152,8 +152,8 @@ __device__ void decode_tile(const Buf& b, long long total_cells, int total_tiles
 }
 
 // Convert tiles whose type changed (old -> new) for every field of the group:
-// 2 -> 1 encodes FP64 into fp16, 1 -> 2 decodes into FP64.  force_encode /
-// force_decode convert every tile whose new type is 1 / every type-1 tile.
+// 2 -> 1 encodes FP64 into fp16, 1 -> 2 decodes into FP64.  CONVERT_ENCODE_LOW
+// encodes every tile whose type is 1.
 //
 // A pass after a monitor converts few items, the first one nearly all of
 // them: workgroup b decides items b, b + grid, b + 2 grid, ... (at most
@@ -182,7 +182,6 @@ __global__ __launch_bounds__(256) void convert_kernel(const InstDesc* __restrict
             const int to = type_old ? type_old[w] : tn;
             if (mode == CONVERT_CHANGED) op = (to == 2 && tn == 1) ? 1 : ((to == 1 && tn == 2) ? 2 : 0);
             else if (mode == CONVERT_ENCODE_LOW) op = tn == 1 ? 1 : 0;
-            else if (mode == CONVERT_DECODE_LOW) op = tn == 1 ? 2 : 0;
         }
         // one wave decides: the items that convert, in order
         static_assert(CONVERT_ITEMS <= 64, "one deciding wave");
@@ -832,7 +831,6 @@ int launch_convert(const InstDesc* inst, const int* tile_inst, const Buf& b, lon
     const int grid = items < 1 ? 1 : (items < CONVERT_GRID ? items : CONVERT_GRID);
     if (tile == 16) hipLaunchKernelGGL((convert_kernel<16>), dim3(grid), dim3(256), 0, s, inst, tile_inst, b, total_cells, total_tiles, type_old, type, gm, mode);
     else if (tile == 32) hipLaunchKernelGGL((convert_kernel<32>), dim3(grid), dim3(256), 0, s, inst, tile_inst, b, total_cells, total_tiles, type_old, type, gm, mode);
-    else if (tile == 64) hipLaunchKernelGGL((convert_kernel<64>), dim3(grid), dim3(256), 0, s, inst, tile_inst, b, total_cells, total_tiles, type_old, type, gm, mode);
     else return AMPS_E_UNSUPPORTED;
     return hip_ok();
 }
@@ -1037,7 +1035,6 @@ int launch_monitor(const StepArgs& a, int kind, int tile, int ngroups_eval, int 
                                a.type, field0, md, reset);
         }
         else if (tile == 32) hipLaunchKernelGGL((monitor_grad_kernel<32>), dim3(grid), dim3(256), 0, s, a, ngroups_eval, field0, field_stride, type_groups, md, reset);
-        else if (tile == 64) hipLaunchKernelGGL((monitor_grad_kernel<64>), dim3(grid), dim3(256), 0, s, a, ngroups_eval, field0, field_stride, type_groups, md, reset);
         else return AMPS_E_UNSUPPORTED;
     } else {
         hipLaunchKernelGGL(monitor_samples_kernel, dim3((n + 15) / 16), dim3(256), 0, s, a.inst, a.tile_inst, a.in,

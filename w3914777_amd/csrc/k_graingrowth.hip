@@ -72,8 +72,9 @@ __device__ inline T gg_lap(const T* B, int c, int LW, const T* cv, int i, bool m
 }
 
 // FP64 update of one cell of value eta (graingrowth/function.h:20-23) with
-// S = sum_j eta_j^2, its multiply-adds written out so that every FP64 sweep
-// rounds alike.
+// S = sum_j eta_j^2, its multiply-adds written out so that the PURE_FP64 sweeps
+// (wave, block, several steps a launch) round alike.  The FP64 tiles of the
+// adaptive sweeps keep the compiler's contraction of the same expression.
 __device__ inline double gg_f64_update(double eta, double lap, double S, double g2, double be, double al, double kap,
                                        double dtl) {
     const double others = fma(-eta, eta, S);

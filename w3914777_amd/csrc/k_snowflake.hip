@@ -1298,8 +1298,6 @@ union SfMixLds {
     SfLowLds<TS, NT> l;
 };
 
-
-//
 // NOSKIP: the low items are the tiles the flat sweep (sf_flat_kernel)
 // appended to this step parity's NSK_SEGS segments, levels 0 and 1 of
 // low_flat_level, each updated by the full low path (H2: its half2 form).

@@ -12,7 +12,7 @@ struct GroupMap {
     signed char fg[AMPS_MAX_FIELDS];
 };
 
-enum { CONVERT_CHANGED = 0, CONVERT_ENCODE_LOW = 1, CONVERT_DECODE_LOW = 2 };
+enum { CONVERT_CHANGED = 0, CONVERT_ENCODE_LOW = 1 };
 
 // Config validation, the descriptor of one instance (tile base and cell
 // base 0) and error recording, shared with host code outside api.cpp.
