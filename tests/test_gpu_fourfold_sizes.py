@@ -11,11 +11,12 @@ from tests.test_zz_no_alloc import Hip
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("ny,nx", [(1024, 1024), (1024, 1056), (2880, 2880), (2912, 2912)])
-@pytest.mark.parametrize("tile,stencil,bc", [(16, 0, 0), (32, 0, 1), (16, 1, 1), (32, 1, 0)])
-def test_same_bits_on_both_sides(amps, O, ny, nx, tile, stencil, bc):
-    if ny > 1024 and (tile, stencil) not in ((32, 0), (16, 1)):
-        pytest.skip("one tile size a Laplacian at the large sizes")
+SMALL = [(t, s, b, 1024, nx) for t, s, b in ((16, 0, 0), (32, 0, 1), (16, 1, 1), (32, 1, 0)) for nx in (1024, 1056)]
+LARGE = [(t, s, 1, n, n) for t, s in ((32, 0), (16, 1)) for n in (2880, 2912)]
+
+
+@pytest.mark.parametrize("tile,stencil,bc,ny,nx", SMALL + LARGE)
+def test_same_bits_on_both_sides(amps, O, tile, stencil, bc, ny, nx):
     c = amps.Config.default(amps.SNOWFLAKE)
     c.nx, c.ny, c.tile, c.stencil, c.bc, c.seed = nx, ny, tile, stencil, bc, 3
     c.params[amps.SF["NOISE"]] = 0.01
